@@ -282,6 +282,8 @@ struct NodesT {
   unsigned char* d_dense = nullptr;  // gather: per-tile LDS-path flag
   int* d_items = nullptr;            // gather: (tile, chunk) pairs
   int n_items = 0;
+  int4* d_ranges = nullptr;          // FP64, m <= 6: position ranges of the gather's items
+  bool ranges = false;
   unsigned char* d_dense_s = nullptr;  // scatter: every nonempty tile takes the LDS path
   int* d_items_s = nullptr;
   int n_items_s = 0;
@@ -616,6 +618,8 @@ static void nodes_release_device(NodesT<R>* D) {
   dfree(D->d_tpartial);
   dfree(D->d_dense);
   dfree(D->d_items);
+  dfree(D->d_ranges);
+  D->ranges = false;
   dfree(D->d_dense_s);
   dfree(D->d_items_s);
   D->items_cap = 0;
@@ -758,9 +762,11 @@ static bool ensure_sort_capacity(NodesT<R>* D, const TileLayout& T) {
   if (D->items_cap < icap) {
     dfree(D->d_items);
     dfree(D->d_items_s);
+    dfree(D->d_ranges);
     D->d_items = dalloc<int>(2 * icap);
     D->d_items_s = dalloc<int>(2 * icap);
-    if (!D->d_items || !D->d_items_s) return false;
+    D->d_ranges = sizeof(R) == 8 ? dalloc<int4>(icap) : nullptr;
+    if (!D->d_items || !D->d_items_s || (sizeof(R) == 8 && !D->d_ranges)) return false;
     D->items_cap = icap;
   }
   return true;
@@ -806,16 +812,17 @@ static void set_tiles(BArgs<R>& A, const NodesT<R>* D, bool for_scatter = false)
   A.tile_dense = for_scatter ? D->d_dense_s : D->d_dense;
   A.items = for_scatter ? D->d_items_s : D->d_items;
   A.n_items = for_scatter ? D->n_items_s : D->n_items;
+  A.ranges = (!for_scatter && D->ranges) ? D->d_ranges : nullptr;
   // the scatter's list holds every nonempty tile; the gather's when dense_min is 1
   A.all_dense = (for_scatter || dense_min() == 1) ? 1 : 0;
   A.no_mfma = mfma_disabled() ? 1 : 0;
+  A.stale_count = D->d_stale_count;
+  A.stale_list = D->d_stale;
   if (D->n_torder > 0) {
     A.torder = D->d_torder;
     A.n_torder = D->n_torder;
     A.n_heavy = D->n_heavy;
     A.n_single = D->n_single;
-    A.stale_count = D->d_stale_count;
-    A.stale_list = D->d_stale;
   }
   if (for_scatter && D->n_torder > 0) {
     A.slots = D->d_slots;
@@ -861,6 +868,9 @@ static int bin(PlanT<R>* P, NodesT<R>* D, const R* dx, const GridGeom& g) {
     D->n_items = ni;
     D->n_items_s = ns;
   }
+  D->ranges = sizeof(R) == 8 && P->m <= 6 && D->n_items > 0 && P->tiles.ts[2] == 8 &&
+              build_ranges(D->d_items, D->n_items, D->d_tile_start, D->d_keys, (unsigned)P->tiles.tile_vol(),
+                           D->d_ranges, P->stream) == kOk;
   D->n_torder = 0;
   const int pad = cols_enabled() ? cols_pad(P->m, sizeof(R) == 8, P->tiles.ts) : 0;
   if (pad > 0 && D->M > 0) {
@@ -941,6 +951,29 @@ static T* grow(T*& p, size_t& cap, size_t need) {
   return p;
 }
 
+// Window tables for the FP64 matrix-core kernels, which take every window from
+// tables (their own evaluation would hold them to half the waves): where
+// precompute_psi made none for this call (or none of the derivatives), the
+// tables are computed into the node set's buffers now.  Without memory for them
+// the arguments stay without tables and the vector kernels evaluate the windows.
+template <class R>
+static void call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s) {
+  if (sizeof(R) != 8 || A.no_mfma || A.g.m > 6 || D->M == 0 || (A.pre_psi && (A.pre_dpsi || !need_grad))) return;
+  const bool kept = A.pre_psi != nullptr;  // psi tables of precompute_psi: written again with equal values
+  const size_t M = (size_t)D->M, cm = 2 * (size_t)A.g.m + 1;
+  R* psi = grow(D->d_pre_psi, D->pre_psi_cap, 3 * cm * M);
+  R* dpsi = need_grad ? grow(D->d_pre_dpsi, D->pre_dpsi_cap, 3 * cm * M) : nullptr;
+  R* xo = grow(D->d_pre_x, D->pre_x_cap, 3 * M);
+  if (!kept) D->pre_valid = false;
+  if (!psi || !xo || (need_grad && !dpsi)) return;
+  A.pre_psi = nullptr;
+  A.pre_dpsi = nullptr;
+  if (precompute_tables<R>(A, psi, dpsi, xo, s) != kOk) return;
+  A.pre_psi = psi;
+  A.pre_dpsi = dpsi;
+  A.pre_x = xo;
+}
+
 // B stage arguments for geometry g: bins the nodes unless the bins of
 // pnfft_precompute_psi are valid for g (device-resident x), then the tile lists
 // and, with valid bins, the window tables.  false on a binning failure.
@@ -965,6 +998,7 @@ static bool b_args(PlanT<R>* P, NodesT<R>* D, R* dx, const GridGeom& g, bool hos
   A.c2r = P->c2r;
   set_tiles(A, D, for_scatter);
   if (reuse) set_tables(A, P, D);
+  if (!P->tab_only) call_tables(A, D, need_grad, P->stream);
   if (P->tab_only && D->M > 0) {
     const size_t M = (size_t)D->M, cm = 2 * (size_t)P->m + 1;
     R* psi = grow(D->d_pre_psi, D->pre_psi_cap, 3 * cm * M);
@@ -1390,6 +1424,7 @@ static void vjp_impl(PlanT<R>* P, NodesT<R>* D, const Cplx<R>* w, R* gx) {
   A.c2r = P->c2r;
   set_tiles(A, D);
   if (reuse) set_tables(A, P, D);
+  call_tables(A, D, true, s);
   if (gather<R>(A, B_VJP, s) != kOk) set_error("gather launch failed");
   if (host_gx) (void)hipMemcpyAsync(gx, dgx, sizeof(R) * 3 * M, hipMemcpyDeviceToHost, s);
   if (hipStreamSynchronize(s) != hipSuccess) set_error("vjp: HIP error %s", hipGetErrorString(hipGetLastError()));

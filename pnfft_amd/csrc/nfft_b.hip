@@ -509,6 +509,33 @@ int build_items(const int* tile_start, long ntiles, int dense_min, unsigned* chu
   return (int)total;
 }
 
+// one thread per item: bisection of its sorted keys, whose in-tile cell index
+// counts the runs of four cells along axis 2 outermost (bin_keys_k)
+__global__ __launch_bounds__(kB) void item_ranges_k(const int* __restrict__ items, int n_items,
+                                                    const int* __restrict__ tile_start,
+                                                    const unsigned* __restrict__ keys, unsigned vol, int4* ranges) {
+  const int i = blockIdx.x * kB + threadIdx.x;
+  if (i >= n_items) return;
+  const int tile = items[2 * i];
+  const int beg = tile_start[tile] + items[2 * i + 1] * kTileNodes;
+  const int end = min(tile_start[tile + 1], beg + kTileNodes);
+  int lo = beg, hi = end;
+  while (lo < hi) {
+    const int c = (lo + hi) >> 1;
+    if (keys[c] % vol < vol / 2) lo = c + 1;
+    else hi = c;
+  }
+  ranges[i] = make_int4(tile, beg, lo, end);
+}
+
+int build_ranges(const int* items, int n_items, const int* tile_start, const unsigned* keys, unsigned tile_vol,
+                 int4* ranges, hipStream_t s) {
+  if (n_items <= 0) return kOk;
+  hipLaunchKernelGGL(item_ranges_k, dim3(grid1d(n_items, kB)), dim3(kB), 0, s, items, n_items, tile_start, keys,
+                     tile_vol, ranges);
+  return hipGetLastError() == hipSuccess ? kOk : kHipError;
+}
+
 int cols_pad(int m, bool is_double, const int* ts) {
   if (m < 2 || m > 8 || (is_double && m > 6)) return 0;
   const int TS = std_tile(m, is_double);
@@ -591,6 +618,17 @@ template <class R>
 int gather(const BArgs<R>& A, int mode, hipStream_t s) {
   if (A.M == 0) return kOk;
   if (A.g.m < kMinPlanM || A.g.m > kMaxPlanM) return kUnsupported;
+  if constexpr (sizeof(R) == 8) {
+    int st = kUnsupported;
+    switch (mode) {
+      case B_F: st = gather_mm64<B_F>(A, s); break;
+      case B_GRAD: st = gather_mm64<B_GRAD>(A, s); break;
+      case B_FGRAD: st = gather_mm64<B_FGRAD>(A, s); break;
+      case B_VJP: st = gather_mm64<B_VJP>(A, s); break;
+      default: break;
+    }
+    if (st != kUnsupported) return st;  // kUnsupported: nothing was launched
+  }
   switch (mode) {
     case B_F: return b_launch<R, 0, B_F>(A, s);
     case B_GRAD: return b_launch<R, 0, B_GRAD>(A, s);

@@ -31,6 +31,7 @@ struct BArgs {
   const unsigned char* tile_dense;  // [ntiles] 1 if the tile's nodes go through the LDS path
   const int* items;        // work items: pairs (tile id, chunk index)
   int n_items;
+  const int4* ranges;      // per work item (tile, first position, first position past the lower half of axis 2, end)
   int ts[3];               // tile size per axis
   int ntile[3];            // tiles per axis
   int all_dense;           // every nonempty tile is a work item: the direct kernel has no nodes to take
@@ -89,11 +90,24 @@ int build_tile_order(const int* tile_start, long ntiles, unsigned* work, unsigne
 template <class R, int MODE>
 int cols_launch(const BArgs<R>& A, hipStream_t s);
 
+// FP64 gather on the matrix cores (gather_mm64.hip) for MODE (B_F, B_GRAD,
+// B_FGRAD, B_VJP): m = 2..6 on tiles of 8^3 cells with the work items of every
+// nonempty tile; kUnsupported (nothing launched) otherwise.
+template <int MODE>
+int gather_mm64(const BArgs<double>& A, hipStream_t s);
+
 // Work items of the tiled kernels: every tile with at least dense_min nodes is
 // cut into chunks of kTileNodes sorted nodes.  Writes tile_dense[ntiles],
 // items[2 * n_items] and returns n_items (host value; synchronizes s), or -1.
 int build_items(const int* tile_start, long ntiles, int dense_min, unsigned* chunks, unsigned* partial,
                 unsigned char* tile_dense, int* items, long items_cap, hipStream_t s);
+
+// The items' position ranges for the FP64 matrix-core kernels: ranges[i] =
+// (tile, beg, mid, end), where the nodes [beg, mid) of the item start in the
+// lower half of the tile's cells along axis 2 and [mid, end) in the upper half
+// (the bin order puts them in this order).
+int build_ranges(const int* items, int n_items, const int* tile_start, const unsigned* keys, unsigned tile_vol,
+                 int4* ranges, hipStream_t s);
 
 // Tile layout used by the binning: a node belongs to the tile that holds its
 // stencil start (floor(n x) - m) mod n on every axis.

@@ -1,0 +1,93 @@
+"""FP64 matrix-core gather against the oracle at the sizes where its tiling can go wrong (GPU).
+
+A tile holds 8^3 cells and its padded subgrid 8 + 2m per axis (12 to 20: below, at and past the sixteen
+rows of a product, with 2 or 4 rows left over); nodes are taken in groups of 16, work items in chunks of
+512 nodes, and items of at most three nodes take the per-node path.  Both sides sum the same
+O((2m+1)^3) products in FP64 in different orders on coefficients of size 1, so the rel-l2 of f, grad_f
+stays below 1e-12 (about 1e-15 times the growth of the window factors).
+"""
+import numpy as np
+import pytest
+
+import pnfft_amd as PA
+from pnfft_amd.device import DevicePlan
+from pnfft_amd.workloads import SplitMix64
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+
+def rel(a, b):
+    a, b = np.asarray(a).reshape(-1), np.asarray(b).reshape(-1)
+    return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
+
+
+def node_set(kind, rng, n):
+    h = 1.0 / np.array(n)
+    if kind == "few":  # tiles of one to four nodes, some alone
+        x = rng.uniform(3 * 70).reshape(70, 3) - 0.5
+    elif kind == "tile":  # one tile's worth of cells, 513 + 40 nodes: two items, ragged groups
+        x = (np.array([8, 8, 8]) + 8 * rng.uniform(3 * 553).reshape(553, 3)) * h - 0.5
+    elif kind == "corner":  # around the wrap of every axis, and exactly on cell borders
+        x = (rng.uniform(3 * 300).reshape(300, 3) - 0.5) * 6 * h + 0.5
+        x[:40] = np.round(x[:40] / h) * h
+    else:  # one cell run along each axis: groups whose offsets reach a single row, plane or K-block
+        x = np.concatenate([np.stack([np.where(t == k, 8 * u, 3.5) for k in range(3)], 1)
+                            for t, u in ((t, rng.uniform(37)) for t in range(3))]) * h
+    x = x - np.floor(x + 0.5)
+    x[x >= 0.5] = -0.5
+    return np.ascontiguousarray(x)
+
+
+@pytest.mark.parametrize("kind", ["few", "tile", "corner", "lines"])
+@pytest.mark.parametrize("m", [2, 3, 4, 5, 6])
+@pytest.mark.parametrize("tables", [False, True])
+def test_gather_matches_oracle(gpu, oracle, kind, m, tables):
+    print("case mm64 gather", kind, m, tables, flush=True)
+    rng = SplitMix64(1000 + 10 * m + len(kind))
+    N, n = (8, 16, 12), (16, 32, 32)
+    x = node_set(kind, rng, n)
+    M = len(x)
+    fh = rng.complex_normal(int(np.prod(N)))
+    w = rng.complex_normal(M)
+    dp = DevicePlan(N, n, m, 0, M)
+    dp.set_x(x)
+    dp.set_f_hat(fh)
+    if tables:
+        dp.precompute(PA.PNFFT_PRE_PSI | PA.PNFFT_PRE_GRAD_PSI)
+    dp.trafo(PA.PNFFT_COMPUTE_F | PA.PNFFT_COMPUTE_GRAD_F)
+    both = dp.f.cpu().numpy().copy(), dp.grad.cpu().numpy().copy()
+    dp.trafo(PA.PNFFT_COMPUTE_F)
+    f = dp.f.cpu().numpy().copy()
+    dp.trafo(PA.PNFFT_COMPUTE_GRAD_F)
+    g = dp.grad.cpu().numpy().copy()
+    import torch
+    gx = dp.grad_x_vjp(torch.as_tensor(w, device="cuda:0")).cpu().numpy()
+    assert dp.api.last_error() is None
+    dp.close()
+    f_o, g_o = oracle.Plan(N, n, m, 0).trafo(x, fh, compute_grad=True)
+    assert rel(f, f_o) < TOL and rel(both[0], f_o) < TOL
+    assert rel(g, g_o) < TOL and rel(both[1], g_o) < TOL
+    assert rel(gx, (np.conj(w)[:, None] * np.asarray(g_o).reshape(M, 3)).real) < TOL
+
+
+@pytest.mark.parametrize("kind", ["few", "tile", "corner"])
+@pytest.mark.parametrize("m", [2, 3, 4, 5, 6])
+def test_gather_real_grid_matches_oracle(gpu, oracle, kind, m):
+    print("case mm64 gather c2r", kind, m, flush=True)
+    rng = SplitMix64(2000 + 10 * m + len(kind))
+    N, n = (8, 16, 12), (16, 32, 32)
+    x = node_set(kind, rng, n)
+    M = len(x)
+    fh = rng.complex_normal(8 * 16 * 7).reshape(8, 16, 7)
+    fh[0], fh[:, 0], fh[:, :, 0] = 0, 0, 0  # Nyquist planes
+    dp = DevicePlan(N, n, m, 0, M, c2r=True)
+    dp.set_x(x)
+    dp.set_f_hat(fh)
+    dp.trafo(PA.PNFFT_COMPUTE_F | PA.PNFFT_COMPUTE_GRAD_F)
+    assert dp.api.last_error() is None
+    f, g = dp.f.cpu().numpy().copy(), dp.grad.cpu().numpy().copy()
+    dp.close()
+    f_o, g_o = oracle.Plan(N, n, m, 0, c2r=True).trafo_c2r(x, fh, compute_grad=True)
+    assert rel(f, f_o) < TOL and rel(g, g_o) < TOL
