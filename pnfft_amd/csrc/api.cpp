@@ -282,8 +282,10 @@ struct NodesT {
   unsigned char* d_dense = nullptr;  // gather: per-tile LDS-path flag
   int* d_items = nullptr;            // gather: (tile, chunk) pairs
   int n_items = 0;
-  int4* d_ranges = nullptr;          // FP64, m <= 6: position ranges of the gather's items
-  bool ranges = false;
+  // FP64, m <= 6: position ranges of the gather's items and of the nonempty tiles in torder
+  int4* d_ranges = nullptr;
+  int4* d_oranges = nullptr;
+  bool ranges = false, oranges = false;
   unsigned char* d_dense_s = nullptr;  // scatter: every nonempty tile takes the LDS path
   int* d_items_s = nullptr;
   int n_items_s = 0;
@@ -619,7 +621,8 @@ static void nodes_release_device(NodesT<R>* D) {
   dfree(D->d_dense);
   dfree(D->d_items);
   dfree(D->d_ranges);
-  D->ranges = false;
+  dfree(D->d_oranges);
+  D->ranges = D->oranges = false;
   dfree(D->d_dense_s);
   dfree(D->d_items_s);
   D->items_cap = 0;
@@ -743,6 +746,11 @@ static bool ensure_sort_capacity(NodesT<R>* D, const TileLayout& T) {
     dfree(D->d_twork);
     dfree(D->d_box_tile);
     dfree(D->d_box_ord);
+    dfree(D->d_oranges);
+    if (sizeof(R) == 8) {
+      D->d_oranges = dalloc<int4>(T.ntiles());
+      if (!D->d_oranges) return false;
+    }
     D->d_tile_start = dalloc<int>(T.ntiles() + 1);
     D->d_chunks = dalloc<unsigned>(2 * T.ntiles());
     D->d_tpartial = dalloc<unsigned>((T.ntiles() + 4095) / 4096 + 1);
@@ -812,7 +820,7 @@ static void set_tiles(BArgs<R>& A, const NodesT<R>* D, bool for_scatter = false)
   A.tile_dense = for_scatter ? D->d_dense_s : D->d_dense;
   A.items = for_scatter ? D->d_items_s : D->d_items;
   A.n_items = for_scatter ? D->n_items_s : D->n_items;
-  A.ranges = (!for_scatter && D->ranges) ? D->d_ranges : nullptr;
+  A.ranges = for_scatter ? (D->oranges ? D->d_oranges : nullptr) : (D->ranges ? D->d_ranges : nullptr);
   // the scatter's list holds every nonempty tile; the gather's when dense_min is 1
   A.all_dense = (for_scatter || dense_min() == 1) ? 1 : 0;
   A.no_mfma = mfma_disabled() ? 1 : 0;
@@ -869,7 +877,7 @@ static int bin(PlanT<R>* P, NodesT<R>* D, const R* dx, const GridGeom& g) {
     D->n_items_s = ns;
   }
   D->ranges = sizeof(R) == 8 && P->m <= 6 && D->n_items > 0 && P->tiles.ts[2] == 8 &&
-              build_ranges(D->d_items, D->n_items, D->d_tile_start, D->d_keys, (unsigned)P->tiles.tile_vol(),
+              build_ranges(D->d_items, D->n_items, true, D->d_tile_start, D->d_keys, (unsigned)P->tiles.tile_vol(),
                            D->d_ranges, P->stream) == kOk;
   D->n_torder = 0;
   const int pad = cols_enabled() ? cols_pad(P->m, sizeof(R) == 8, P->tiles.ts) : 0;
@@ -892,6 +900,9 @@ static int bin(PlanT<R>* P, NodesT<R>* D, const R* dx, const GridGeom& g) {
     // without slot memory the scatter takes the LDS-atomic path
     D->n_torder = D->d_slots ? nt : 0;
   }
+  D->oranges = sizeof(R) == 8 && P->m <= 6 && D->n_torder > 0 &&
+               build_ranges(D->d_torder, D->n_torder, false, D->d_tile_start, D->d_keys,
+                            (unsigned)P->tiles.tile_vol(), D->d_oranges, P->stream) == kOk;
   // the boxes serve only the FP32 matrix-core scatter and its fold on 8^3 tiles
   // whose padded subgrids are a multiple of four cells wide (m = 2, 4)
   const int pb = 8 + 2 * P->m;

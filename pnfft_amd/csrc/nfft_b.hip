@@ -511,14 +511,14 @@ int build_items(const int* tile_start, long ntiles, int dense_min, unsigned* chu
 
 // one thread per item: bisection of its sorted keys, whose in-tile cell index
 // counts the runs of four cells along axis 2 outermost (bin_keys_k)
-__global__ __launch_bounds__(kB) void item_ranges_k(const int* __restrict__ items, int n_items,
+__global__ __launch_bounds__(kB) void item_ranges_k(const int* __restrict__ items, int n_items, int chunked,
                                                     const int* __restrict__ tile_start,
                                                     const unsigned* __restrict__ keys, unsigned vol, int4* ranges) {
   const int i = blockIdx.x * kB + threadIdx.x;
   if (i >= n_items) return;
-  const int tile = items[2 * i];
-  const int beg = tile_start[tile] + items[2 * i + 1] * kTileNodes;
-  const int end = min(tile_start[tile + 1], beg + kTileNodes);
+  const int tile = chunked ? items[2 * i] : items[i];
+  const int beg = tile_start[tile] + (chunked ? items[2 * i + 1] * kTileNodes : 0);
+  const int end = chunked ? min(tile_start[tile + 1], beg + kTileNodes) : tile_start[tile + 1];
   int lo = beg, hi = end;
   while (lo < hi) {
     const int c = (lo + hi) >> 1;
@@ -528,11 +528,11 @@ __global__ __launch_bounds__(kB) void item_ranges_k(const int* __restrict__ item
   ranges[i] = make_int4(tile, beg, lo, end);
 }
 
-int build_ranges(const int* items, int n_items, const int* tile_start, const unsigned* keys, unsigned tile_vol,
+int build_ranges(const int* items, int n_items, bool chunked, const int* tile_start, const unsigned* keys, unsigned tile_vol,
                  int4* ranges, hipStream_t s) {
   if (n_items <= 0) return kOk;
-  hipLaunchKernelGGL(item_ranges_k, dim3(grid1d(n_items, kB)), dim3(kB), 0, s, items, n_items, tile_start, keys,
-                     tile_vol, ranges);
+  hipLaunchKernelGGL(item_ranges_k, dim3(grid1d(n_items, kB)), dim3(kB), 0, s, items, n_items, chunked ? 1 : 0,
+                     tile_start, keys, tile_vol, ranges);
   return hipGetLastError() == hipSuccess ? kOk : kHipError;
 }
 
@@ -642,6 +642,16 @@ template <class R>
 int scatter(const BArgs<R>& A, int mode, hipStream_t s) {
   if (A.M == 0) return kOk;
   if (A.g.m < kMinPlanM || A.g.m > kMaxPlanM) return kUnsupported;
+  if constexpr (sizeof(R) == 8) {
+    int st = kUnsupported;
+    switch (mode) {
+      case B_F: st = scatter_mm64<B_F>(A, s); break;
+      case B_GRAD: st = scatter_mm64<B_GRAD>(A, s); break;
+      case B_FGRAD: st = scatter_mm64<B_FGRAD>(A, s); break;
+      default: break;
+    }
+    if (st != kUnsupported) return st;  // kUnsupported: nothing was launched
+  }
   if (A.slots) {  // column path: writes every grid cell through the fold
     int st = kUnsupported;
     switch (mode) {

@@ -31,7 +31,9 @@ struct BArgs {
   const unsigned char* tile_dense;  // [ntiles] 1 if the tile's nodes go through the LDS path
   const int* items;        // work items: pairs (tile id, chunk index)
   int n_items;
-  const int4* ranges;      // per work item (tile, first position, first position past the lower half of axis 2, end)
+  // per work item (gather) or nonempty tile in the tile order (scatter): (tile,
+  // first position, first position past the lower half of axis 2, end)
+  const int4* ranges;
   int ts[3];               // tile size per axis
   int ntile[3];            // tiles per axis
   int all_dense;           // every nonempty tile is a work item: the direct kernel has no nodes to take
@@ -96,17 +98,26 @@ int cols_launch(const BArgs<R>& A, hipStream_t s);
 template <int MODE>
 int gather_mm64(const BArgs<double>& A, hipStream_t s);
 
+// FP64 scatter on the matrix cores (scatter_mm64.hip) for MODE (B_F, B_GRAD,
+// B_FGRAD): m = 2..6 on tiles of 8^3 cells, every window from tables; slots,
+// fold and stale nodes as cols_launch.  kUnsupported (nothing launched) otherwise.
+template <int MODE>
+int scatter_mm64(const BArgs<double>& A, hipStream_t s);
+
+// Fold of the FP64 slots (tiles of 8^3 cells, m = 2..6) into the grid, which it overwrites.
+int fold_slots64(const BArgs<double>& A, hipStream_t s);
+
 // Work items of the tiled kernels: every tile with at least dense_min nodes is
 // cut into chunks of kTileNodes sorted nodes.  Writes tile_dense[ntiles],
 // items[2 * n_items] and returns n_items (host value; synchronizes s), or -1.
 int build_items(const int* tile_start, long ntiles, int dense_min, unsigned* chunks, unsigned* partial,
                 unsigned char* tile_dense, int* items, long items_cap, hipStream_t s);
 
-// The items' position ranges for the FP64 matrix-core kernels: ranges[i] =
-// (tile, beg, mid, end), where the nodes [beg, mid) of the item start in the
-// lower half of the tile's cells along axis 2 and [mid, end) in the upper half
-// (the bin order puts them in this order).
-int build_ranges(const int* items, int n_items, const int* tile_start, const unsigned* keys, unsigned tile_vol,
+// Position ranges for the FP64 matrix-core kernels: ranges[i] = (tile, beg, mid,
+// end), where the nodes [beg, mid) start in the lower half of the tile's cells
+// along axis 2 and [mid, end) in the upper half (the bin order puts them in this
+// order), of item i (chunked: pairs (tile, chunk) of items) or of tile items[i].
+int build_ranges(const int* items, int n_items, bool chunked, const int* tile_start, const unsigned* keys, unsigned tile_vol,
                  int4* ranges, hipStream_t s);
 
 // Tile layout used by the binning: a node belongs to the tile that holds its

@@ -1,7 +1,8 @@
 // scatter_cols.hip -- adjoint window scatter B^T with register accumulators.
 //
 // This file is compiled once per (precision, mode); the build passes
-// PNFFT_B_REAL (float|double) and PNFFT_B_MODE (B_F, B_GRAD or B_FGRAD).
+// PNFFT_B_REAL (float|double), PNFFT_B_IS_DOUBLE (0|1) and PNFFT_B_MODE (B_F,
+// B_GRAD or B_FGRAD).
 //
 // Reference: the scatter node loop of kernel/ndft-parallel.c:2890-3009 with
 // the stencil kernels spread_f_c2c / spread_grad_f_c2c of
@@ -811,6 +812,29 @@ __global__ void zero_count_k(unsigned* c) {
 
 inline unsigned grid1d(long n, int t) { return (unsigned)((n + t - 1) / t); }
 
+// the fold kernel of the layout (tiles of TS cells, padded subgrids of P)
+template <class R, int TS, int P>
+void fold_launch(const BArgs<R>& A, hipStream_t s) {
+  const long ntiles = (long)A.ntile[0] * A.ntile[1] * A.ntile[2];
+  if constexpr (TS == 8) {
+    bool brick = false;
+    if constexpr (P <= 16 && P % 4 == 0) {
+      if (A.ts[2] == 8 && A.ntile[2] % 2 == 0) {
+        hipLaunchKernelGGL((fold8b_k<R, P>), dim3((unsigned)(ntiles / 2)), dim3(256), 0, s, A);
+        brick = true;
+      }
+    }
+    if (!brick) hipLaunchKernelGGL((fold8_k<R, P>), dim3((unsigned)ntiles), dim3(128), 0, s, A);
+  } else if constexpr (P <= 16) {
+    if (A.ts[2] == 4 && A.ntile[2] % 4 == 0)
+      hipLaunchKernelGGL((fold4_k<R, P>), dim3((unsigned)(ntiles / 4)), dim3(128), 0, s, A);
+    else
+      hipLaunchKernelGGL((fold_k<R, TS, P>), dim3((unsigned)ntiles), dim3(TS * TS * TS), 0, s, A);
+  } else {
+    hipLaunchKernelGGL((fold_k<R, TS, P>), dim3((unsigned)ntiles), dim3(TS * TS * TS), 0, s, A);
+  }
+}
+
 template <class R, int MT, int MODE>
 void launch_m(const BArgs<R>& A0, hipStream_t s) {
   using S = ColsShape<R, MT, MODE>;
@@ -832,24 +856,7 @@ void launch_m(const BArgs<R>& A0, hipStream_t s) {
   }
   if (!done) hipLaunchKernelGGL((scatter_cols_k<R, MT, MODE>), dim3((unsigned)A.n_torder), dim3(S::NT), 0, s, A);
   if (A.mid) (void)hipEventRecord(A.mid, s);
-  const long ntiles = (long)A.ntile[0] * A.ntile[1] * A.ntile[2];
-  if constexpr (S::TS == 8) {
-    bool brick = false;
-    if constexpr (S::P <= 16 && S::P % 4 == 0) {
-      if (A.ts[2] == 8 && A.ntile[2] % 2 == 0) {
-        hipLaunchKernelGGL((fold8b_k<R, S::P>), dim3((unsigned)(ntiles / 2)), dim3(256), 0, s, A);
-        brick = true;
-      }
-    }
-    if (!brick) hipLaunchKernelGGL((fold8_k<R, S::P>), dim3((unsigned)ntiles), dim3(128), 0, s, A);
-  } else if constexpr (S::P <= 16) {
-    if (A.ts[2] == 4 && A.ntile[2] % 4 == 0)
-      hipLaunchKernelGGL((fold4_k<R, S::P>), dim3((unsigned)(ntiles / 4)), dim3(128), 0, s, A);
-    else
-      hipLaunchKernelGGL((fold_k<R, S::TS, S::P>), dim3((unsigned)ntiles), dim3(S::TS * S::TS * S::TS), 0, s, A);
-  } else {
-    hipLaunchKernelGGL((fold_k<R, S::TS, S::P>), dim3((unsigned)ntiles), dim3(S::TS * S::TS * S::TS), 0, s, A);
-  }
+  fold_launch<R, S::TS, S::P>(A, s);
   if (A.mid2) (void)hipEventRecord(A.mid2, s);
   hipLaunchKernelGGL((scatter_stale_k<R, MT, MODE>), dim3(256), dim3(256), 0, s, A);
 }
@@ -882,6 +889,21 @@ int cols_launch(const BArgs<R>& A, hipStream_t s) {
     return hipGetLastError() == hipSuccess ? kOk : kHipError;
   }
 }
+
+#if PNFFT_B_MODE == 1 && PNFFT_B_IS_DOUBLE
+int fold_slots64(const BArgs<double>& A, hipStream_t s) {
+  using R = double;
+  switch (A.g.m) {
+    case 2: fold_launch<R, 8, 12>(A, s); break;
+    case 3: fold_launch<R, 8, 14>(A, s); break;
+    case 4: fold_launch<R, 8, 16>(A, s); break;
+    case 5: fold_launch<R, 8, 18>(A, s); break;
+    case 6: fold_launch<R, 8, 20>(A, s); break;
+    default: return kUnsupported;
+  }
+  return hipGetLastError() == hipSuccess ? kOk : kHipError;
+}
+#endif
 
 template int cols_launch<PNFFT_B_REAL, PNFFT_B_MODE>(const BArgs<PNFFT_B_REAL>&, hipStream_t);
 

@@ -1,4 +1,4 @@
-"""FP64 matrix-core gather against the oracle at the sizes where its tiling can go wrong (GPU).
+"""FP64 matrix-core gather and scatter against the oracle at the sizes where its tiling can go wrong (GPU).
 
 A tile holds 8^3 cells and its padded subgrid 8 + 2m per axis (12 to 20: below, at and past the sixteen
 rows of a product, with 2 or 4 rows left over); nodes are taken in groups of 16, work items in chunks of
@@ -91,3 +91,37 @@ def test_gather_real_grid_matches_oracle(gpu, oracle, kind, m):
     dp.close()
     f_o, g_o = oracle.Plan(N, n, m, 0, c2r=True).trafo_c2r(x, fh, compute_grad=True)
     assert rel(f, f_o) < TOL and rel(g, g_o) < TOL
+
+
+@pytest.mark.parametrize("c2r", [False, True])
+@pytest.mark.parametrize("kind", ["few", "tile", "corner", "lines"])
+@pytest.mark.parametrize("m", [2, 3, 4, 5, 6])
+def test_scatter_matches_oracle(gpu, oracle, kind, m, c2r):
+    """adj of f, of grad_f and of both, without tables and with them (the two phases of m = 5, 6 with
+    one of them empty: "lines" along axes 0 and 1)."""
+    print("case mm64 scatter", kind, m, c2r, flush=True)
+    rng = SplitMix64(3000 + 10 * m + len(kind))
+    N, n = (8, 16, 12), (16, 32, 32)
+    x = node_set(kind, rng, n)
+    if kind == "lines":
+        x = x[:74]
+    M = len(x)
+    fv = rng.normal(M) if c2r else rng.complex_normal(M)
+    gv = rng.normal(3 * M) if c2r else rng.complex_normal(3 * M)
+    P = oracle.Plan(N, n, m, 0, c2r=c2r)
+    adj = P.adj_c2r if c2r else P.adj
+    refs = [np.asarray(adj(x, f=fv)).reshape(-1), np.asarray(adj(x, grad=gv)).reshape(-1)]
+    refs.append(refs[0] + refs[1])
+    dp = DevicePlan(N, n, m, 0, M, c2r=c2r)
+    dp.set_x(x)
+    dp.set_f(fv)
+    dp.set_grad(gv)
+    for tables in (False, True):
+        if tables:
+            dp.precompute(PA.PNFFT_PRE_PSI | PA.PNFFT_PRE_GRAD_PSI)
+        for flags, ref in zip((PA.PNFFT_COMPUTE_F, PA.PNFFT_COMPUTE_GRAD_F,
+                               PA.PNFFT_COMPUTE_F | PA.PNFFT_COMPUTE_GRAD_F), refs):
+            dp.adj(flags)
+            assert dp.api.last_error() is None
+            assert rel(dp.f_hat.cpu().numpy(), ref) < TOL, (flags, tables)
+    dp.close()
