@@ -272,37 +272,19 @@ struct NodesT {
   int* d_hess_st = nullptr;
   size_t tmp_cap = 0, hess_tab_cap = 0, hess_st_cap = 0;
 
-  // binning
+  // binning: one allocation (bin_mem) that holds the sorted node ids and keys, the
+  // sort's scratch and the per-tile lists (TileLists), sized for bin_M nodes and
+  // bin_ntiles tiles
+  char* bin_mem = nullptr;
+  size_t bin_cap = 0;
   int* d_perm = nullptr;
   unsigned* d_keys = nullptr;
-  int* d_tile_start = nullptr;
-  long tile_cap = 0;
-  unsigned* d_chunks = nullptr;      // 2 * ntiles: per-tile chunk counts and their offsets
-  unsigned* d_tpartial = nullptr;    // scan partials of the tile counts
-  unsigned char* d_dense = nullptr;  // gather: per-tile LDS-path flag
-  int* d_items = nullptr;            // gather: (tile, chunk) pairs
-  int n_items = 0;
-  // FP64, m <= 6: position ranges of the gather's items and of the nonempty tiles in torder
-  int4* d_ranges = nullptr;
-  int4* d_oranges = nullptr;
-  bool ranges = false, oranges = false;
-  unsigned char* d_dense_s = nullptr;  // scatter: every nonempty tile takes the LDS path
-  int* d_items_s = nullptr;
-  int n_items_s = 0;
-  long items_cap = 0;
-  // column scatter: nonempty tiles by decreasing node count, tile -> slot map, slots
-  int* d_torder = nullptr;
-  int* d_tile_slot = nullptr;
-  unsigned* d_twork = nullptr;
+  TileLists tl{};
+  TileCounts tc{};
+  bool has_ranges = false, boxes = false;
+  int n_torder = 0;        // order entries (0: the layout has no column scatter)
   Cplx<R>* d_slots = nullptr;
-  size_t slots_cap = 0;  // complex elements
-  int n_torder = 0;
-  int n_heavy = 0;       // torder[0, n_heavy): tiles with 32 nodes or more
-  int n_single = 0;      // the last n_single tiles of torder: one node each
-  // offsets of each tile's nodes per axis (build_tile_boxes), by tile id and by position in torder
-  unsigned* d_box_tile = nullptr;
-  unsigned* d_box_ord = nullptr;
-  bool boxes = false;
+  size_t slots_cap = 0;    // complex elements
   int* d_stale = nullptr;            // [M] sorted positions of nodes outside their tile
   unsigned* d_stale_count = nullptr;
   // window tables of precompute_psi (sorted order, see precompute_tables)
@@ -613,44 +595,16 @@ static void nodes_release_device(NodesT<R>* D) {
   dfree(D->d_hess_tab);
   dfree(D->d_hess_st);
   D->tmp_cap = D->hess_tab_cap = D->hess_st_cap = 0;
-  dfree(D->d_perm);
-  dfree(D->d_keys);
-  dfree(D->d_tile_start);
-  dfree(D->d_chunks);
-  dfree(D->d_tpartial);
-  dfree(D->d_dense);
-  dfree(D->d_items);
-  dfree(D->d_ranges);
-  dfree(D->d_oranges);
-  D->ranges = D->oranges = false;
-  dfree(D->d_dense_s);
-  dfree(D->d_items_s);
-  D->items_cap = 0;
-  D->n_items = D->n_items_s = 0;
-  dfree(D->d_torder);
-  dfree(D->d_tile_slot);
-  dfree(D->d_twork);
-  dfree(D->d_box_tile);
-  dfree(D->d_box_ord);
-  D->boxes = false;
+  dfree(D->bin_mem);
+  D->bin_cap = 0;
   dfree(D->d_slots);
   D->slots_cap = 0;
   D->n_torder = 0;
-  dfree(D->d_stale);
-  dfree(D->d_stale_count);
   dfree(D->d_pre_psi);
   dfree(D->d_pre_dpsi);
   dfree(D->d_pre_x);
   D->pre_psi_cap = D->pre_dpsi_cap = D->pre_x_cap = 0;
   D->pre_valid = false;
-  dfree(D->sw.keys[0]);
-  dfree(D->sw.keys[1]);
-  dfree(D->sw.vals[0]);
-  dfree(D->sw.vals[1]);
-  dfree(D->sw.hist);
-  dfree(D->sw.partial);
-  D->sw.cap = D->sw.hist_cap = D->sw.partial_cap = 0;
-  D->tile_cap = 0;
   D->bins_valid = false;
 }
 
@@ -695,87 +649,56 @@ static T* stage_in(void* user, T*& mirror, size_t count, bool upload, hipStream_
   return mirror;
 }
 
+// Nodes per order entry (slot) of a tile.
+static int part_nodes(long M) {
+  (void)M;
+  return 1 << 30;
+}
+
+// Lays the binning arrays for M nodes in tiles T out in bin_mem, (re)allocated when too small.
 template <class R>
-static bool ensure_sort_capacity(NodesT<R>* D, const TileLayout& T) {
-  const long M = D->M;
-  if (D->sw.cap < M) {
-    dfree(D->sw.keys[0]);
-    dfree(D->sw.keys[1]);
-    dfree(D->sw.vals[0]);
-    dfree(D->sw.vals[1]);
-    dfree(D->d_perm);
-    dfree(D->d_keys);
-    dfree(D->d_stale);
-    dfree(D->d_stale_count);
-    D->sw.keys[0] = dalloc<unsigned>(M);
-    D->sw.keys[1] = dalloc<unsigned>(M);
-    D->sw.vals[0] = dalloc<int>(M);
-    D->sw.vals[1] = dalloc<int>(M);
-    D->d_perm = dalloc<int>(M);
-    D->d_keys = dalloc<unsigned>(M);
-    D->d_stale = dalloc<int>(M);
-    D->d_stale_count = dalloc<unsigned>(1);
-    if (!D->sw.keys[0] || !D->sw.keys[1] || !D->sw.vals[0] || !D->sw.vals[1] || !D->d_perm || !D->d_keys ||
-        !D->d_stale || !D->d_stale_count)
-      return false;
-    D->sw.cap = M;
-  }
-  const long nblk = (M + 4095) / 4096;
-  const long hist = 256 * nblk;
-  if (D->sw.hist_cap < hist) {
-    dfree(D->sw.hist);
-    D->sw.hist = dalloc<unsigned>(hist);
-    if (!D->sw.hist) return false;
-    D->sw.hist_cap = hist;
-  }
-  const long parts = (hist + 4095) / 4096;
-  if (D->sw.partial_cap < parts) {
-    dfree(D->sw.partial);
-    D->sw.partial = dalloc<unsigned>(parts);
-    if (!D->sw.partial) return false;
-    D->sw.partial_cap = parts;
-  }
-  if (D->tile_cap < T.ntiles() + 1) {
-    dfree(D->d_tile_start);
-    dfree(D->d_chunks);
-    dfree(D->d_tpartial);
-    dfree(D->d_dense);
-    dfree(D->d_dense_s);
-    dfree(D->d_torder);
-    dfree(D->d_tile_slot);
-    dfree(D->d_twork);
-    dfree(D->d_box_tile);
-    dfree(D->d_box_ord);
-    dfree(D->d_oranges);
-    if (sizeof(R) == 8) {
-      D->d_oranges = dalloc<int4>(T.ntiles());
-      if (!D->d_oranges) return false;
+static bool ensure_bin_memory(NodesT<R>* D, const TileLayout& T) {
+  const size_t M = (size_t)D->M, nt = (size_t)T.ntiles();
+  const size_t items = nt + M / kTileNodes + 2, order = nt + M / (size_t)part_nodes(D->M) + 2;
+  for (int pass = 0; pass < 2; pass++) {
+    size_t at = 0;
+    auto take = [&](auto*& p, size_t count) {
+      using E = std::remove_reference_t<decltype(*p)>;
+      if (pass == 1) p = reinterpret_cast<E*>(D->bin_mem + at);
+      at += (sizeof(E) * count + 255) / 256 * 256;
+    };
+    take(D->d_perm, M);
+    take(D->d_keys, M);
+    take(D->sw.keys[0], M);
+    take(D->sw.keys[1], M);
+    take(D->sw.vals[0], M);
+    take(D->sw.vals[1], M);
+    take(D->sw.hist, (size_t)sort_hist_words(D->M));
+    take(D->sw.total, 256);
+    take(D->d_stale, M);
+    take(D->d_stale_count, 1);
+    take(D->tl.tile_start, nt + 1);
+    take(D->tl.scan, 4 * nt);
+    take(D->tl.partial, 4 * (nt / 4096 + 1));
+    take(D->tl.work, kTileWork);
+    take(D->tl.dense, nt);
+    take(D->tl.dense_s, nt);
+    take(D->tl.items, 2 * items);
+    take(D->tl.items_s, 2 * items);
+    take(D->tl.order, order);
+    take(D->tl.tile_slot, nt);
+    take(D->tl.ranges, items);
+    take(D->tl.oranges, order);
+    take(D->tl.box_tile, nt);
+    take(D->tl.box_ord, order);
+    D->tl.order_cap = (long)order;
+    if (pass == 0 && D->bin_cap < at) {
+      dfree(D->bin_mem);
+      D->bin_cap = 0;
+      D->bin_mem = dalloc<char>(at);
+      if (!D->bin_mem) return false;
+      D->bin_cap = at;
     }
-    D->d_tile_start = dalloc<int>(T.ntiles() + 1);
-    D->d_chunks = dalloc<unsigned>(2 * T.ntiles());
-    D->d_tpartial = dalloc<unsigned>((T.ntiles() + 4095) / 4096 + 1);
-    D->d_dense = dalloc<unsigned char>(T.ntiles());
-    D->d_dense_s = dalloc<unsigned char>(T.ntiles());
-    D->d_torder = dalloc<int>(T.ntiles());
-    D->d_tile_slot = dalloc<int>(T.ntiles());
-    D->d_twork = dalloc<unsigned>(65);
-    D->d_box_tile = dalloc<unsigned>(T.ntiles());
-    D->d_box_ord = dalloc<unsigned>(T.ntiles());
-    if (!D->d_tile_start || !D->d_chunks || !D->d_tpartial || !D->d_dense || !D->d_dense_s || !D->d_torder ||
-        !D->d_tile_slot || !D->d_twork || !D->d_box_tile || !D->d_box_ord)
-      return false;
-    D->tile_cap = T.ntiles() + 1;
-  }
-  const long icap = T.ntiles() + (M + kTileNodes - 1) / kTileNodes + 1;
-  if (D->items_cap < icap) {
-    dfree(D->d_items);
-    dfree(D->d_items_s);
-    dfree(D->d_ranges);
-    D->d_items = dalloc<int>(2 * icap);
-    D->d_items_s = dalloc<int>(2 * icap);
-    D->d_ranges = sizeof(R) == 8 ? dalloc<int4>(icap) : nullptr;
-    if (!D->d_items || !D->d_items_s || (sizeof(R) == 8 && !D->d_ranges)) return false;
-    D->items_cap = icap;
   }
   return true;
 }
@@ -815,30 +738,32 @@ static int dense_min() {
 
 template <class R>
 static void set_tiles(BArgs<R>& A, const NodesT<R>* D, bool for_scatter = false) {
-  A.tile_start = D->d_tile_start;
+  const bool two = for_scatter && dense_min() > 1;  // the scatter's own list: every nonempty tile
+  A.tile_start = D->tl.tile_start;
   A.keys = D->d_keys;
-  A.tile_dense = for_scatter ? D->d_dense_s : D->d_dense;
-  A.items = for_scatter ? D->d_items_s : D->d_items;
-  A.n_items = for_scatter ? D->n_items_s : D->n_items;
-  A.ranges = for_scatter ? (D->oranges ? D->d_oranges : nullptr) : (D->ranges ? D->d_ranges : nullptr);
+  A.tile_dense = two ? D->tl.dense_s : D->tl.dense;
+  A.items = two ? D->tl.items_s : D->tl.items;
+  A.n_items = two ? D->tc.n_items_s : D->tc.n_items;
+  A.ranges = D->has_ranges ? D->tl.ranges : nullptr;
   // the scatter's list holds every nonempty tile; the gather's when dense_min is 1
   A.all_dense = (for_scatter || dense_min() == 1) ? 1 : 0;
   A.no_mfma = mfma_disabled() ? 1 : 0;
   A.stale_count = D->d_stale_count;
   A.stale_list = D->d_stale;
   if (D->n_torder > 0) {
-    A.torder = D->d_torder;
+    A.torder = D->tl.order;
+    A.oranges = D->tl.oranges;
     A.n_torder = D->n_torder;
-    A.n_heavy = D->n_heavy;
-    A.n_single = D->n_single;
-  }
-  if (for_scatter && D->n_torder > 0) {
-    A.slots = D->d_slots;
-    A.tile_slot = D->d_tile_slot;
-  }
-  if (D->n_torder > 0 && D->boxes) {
-    A.box_tile = D->d_box_tile;
-    A.box_ord = D->d_box_ord;
+    A.n_heavy = D->tc.n_heavy;
+    A.n_single = D->tc.n_single;
+    if (for_scatter && D->d_slots) {
+      A.slots = D->d_slots;
+      A.tile_slot = D->tl.tile_slot;
+    }
+    if (D->boxes) {
+      A.box_tile = D->tl.box_tile;
+      A.box_ord = D->tl.box_ord;
+    }
   }
   for (int t = 0; t < 3; t++) {
     A.ts[t] = D->bin_tiles.ts[t];
@@ -850,67 +775,50 @@ static bool same_geom(const GridGeom& a, const GridGeom& b) {
   return a.n[0] == b.n[0] && a.n[1] == b.n[1] && a.n[2] == b.n[2] && a.m == b.m && a.shift == b.shift;
 }
 
+// Slots of the column scatter for the current bins.  Without memory for them the
+// scatter takes the LDS-atomic path.
+template <class R>
+static void ensure_slots(PlanT<R>* P, NodesT<R>* D) {
+  if (D->n_torder <= 0) return;
+  const size_t pad = (size_t)cols_pad(P->m, sizeof(R) == 8, D->bin_tiles.ts);
+  const size_t need = (size_t)D->n_torder * pad * pad * pad;
+  if (D->slots_cap < need) {
+    dfree(D->d_slots);
+    D->slots_cap = 0;
+    D->d_slots = dalloc<Cplx<R>>(need);
+    if (D->d_slots) D->slots_cap = need;
+    (void)hipGetLastError();
+  }
+}
+
 // Bin the nodes of D for plan P (on P's stream) in geometry g (the plan's, or
 // the half-cell shifted one of an interlaced pass).
 template <class R>
 static int bin(PlanT<R>* P, NodesT<R>* D, const R* dx, const GridGeom& g) {
-  if (!ensure_sort_capacity(D, P->tiles)) {
+  D->bins_valid = false;
+  if (!ensure_bin_memory(D, P->tiles)) {
     set_error("device allocation for node binning failed");
     return kHipError;
   }
-  int st = bin_nodes<R>(dx, D->M, g, P->tiles, D->sw, D->d_perm, D->d_keys, D->d_tile_start, P->stream);
+  int st = bin_nodes<R>(dx, D->M, g, P->tiles, D->sw, D->d_perm, D->d_keys, P->stream);
   if (st != kOk) {
     set_error("node binning failed (%d)", st);
     return st;
   }
-  D->n_items = D->n_items_s = 0;
-  if (P->m >= 2 && P->m <= 8) {
-    const int ni = build_items(D->d_tile_start, P->tiles.ntiles(), dense_min(), D->d_chunks, D->d_tpartial,
-                               D->d_dense, D->d_items, D->items_cap, P->stream);
-    const int ns = build_items(D->d_tile_start, P->tiles.ntiles(), 1, D->d_chunks, D->d_tpartial, D->d_dense_s,
-                               D->d_items_s, D->items_cap, P->stream);
-    if (ni < 0 || ns < 0) {
-      set_error("building the tile work list failed");
-      return kHipError;
-    }
-    D->n_items = ni;
-    D->n_items_s = ns;
-  }
-  D->ranges = sizeof(R) == 8 && P->m <= 6 && D->n_items > 0 && P->tiles.ts[2] == 8 &&
-              build_ranges(D->d_items, D->n_items, true, D->d_tile_start, D->d_keys, (unsigned)P->tiles.tile_vol(),
-                           D->d_ranges, P->stream) == kOk;
-  D->n_torder = 0;
-  const int pad = cols_enabled() ? cols_pad(P->m, sizeof(R) == 8, P->tiles.ts) : 0;
-  if (pad > 0 && D->M > 0) {
-    const int nt = build_tile_order(D->d_tile_start, P->tiles.ntiles(), D->d_twork, D->d_chunks, D->d_tpartial,
-                                    D->d_torder, D->d_tile_slot, &D->n_heavy, &D->n_single,
-                                    P->stream);
-    if (nt < 0) {
-      set_error("building the tile order failed");
-      return kHipError;
-    }
-    const size_t need = (size_t)nt * (size_t)pad * pad * pad;
-    if (D->slots_cap < need) {
-      dfree(D->d_slots);
-      D->slots_cap = 0;
-      D->d_slots = dalloc<Cplx<R>>(need);
-      if (D->d_slots) D->slots_cap = need;
-      (void)hipGetLastError();
-    }
-    // without slot memory the scatter takes the LDS-atomic path
-    D->n_torder = D->d_slots ? nt : 0;
-  }
-  D->oranges = sizeof(R) == 8 && P->m <= 6 && D->n_torder > 0 &&
-               build_ranges(D->d_torder, D->n_torder, false, D->d_tile_start, D->d_keys,
-                            (unsigned)P->tiles.tile_vol(), D->d_oranges, P->stream) == kOk;
   // the boxes serve only the FP32 matrix-core scatter and its fold on 8^3 tiles
   // whose padded subgrids are a multiple of four cells wide (m = 2, 4)
-  const int pb = 8 + 2 * P->m;
-  const bool want_boxes = sizeof(R) == 4 && P->tiles.ts[0] == 8 && P->tiles.ts[1] == 8 && P->tiles.ts[2] == 8 &&
-                          pb <= 16 && pb % 4 == 0;
-  D->boxes = want_boxes && D->n_torder > 0 &&
-             build_tile_boxes(D->d_keys, D->M, P->tiles, D->d_torder, D->n_torder, D->d_box_tile, D->d_box_ord,
-                              P->stream) == kOk;
+  const int pad = cols_enabled() ? cols_pad(P->m, sizeof(R) == 8, P->tiles.ts) : 0;
+  D->boxes = sizeof(R) == 4 && pad > 0 && P->tiles.ts[0] == 8 && pad <= 16 && pad % 4 == 0;
+  // ranges: FP64 matrix-core gather on tiles of 8 cells; its tile lists hold no fewer-node cut
+  D->has_ranges = sizeof(R) == 8 && P->m <= 6 && P->tiles.ts[2] == 8;
+  TileLists tl = D->tl;
+  if (!D->has_ranges) tl.ranges = nullptr;
+  if (build_tile_lists(D->d_keys, D->M, P->tiles, dense_min(), part_nodes(D->M), D->boxes, tl, &D->tc, P->stream) !=
+      kOk) {
+    set_error("building the tile lists failed");
+    return kHipError;
+  }
+  D->n_torder = pad > 0 && D->M > 0 ? D->tc.n_order : 0;
   D->bin_geom = g;
   D->bin_tiles = P->tiles;
   D->bins_valid = true;
@@ -1007,6 +915,7 @@ static bool b_args(PlanT<R>* P, NodesT<R>* D, R* dx, const GridGeom& g, bool hos
   A.perm = D->d_perm;
   A.grid = P->d_grid;
   A.c2r = P->c2r;
+  if (for_scatter) ensure_slots(P, D);
   set_tiles(A, D, for_scatter);
   if (reuse) set_tables(A, P, D);
   if (!P->tab_only) call_tables(A, D, need_grad, P->stream);
@@ -1463,6 +1372,7 @@ static void precompute_impl(PlanT<R>* P, NodesT<R>* D, unsigned flags) {
   R* dx = stage_in<R>(D->x, D->d_x, 3 * D->M, true, P->stream, &host_x);
   if (!dx) return;
   if (bin(P, D, dx, P->geom) != kOk) return;
+  ensure_slots(P, D);
   // plans whose windows come from tables tabulate on every call (b_args)
   if (!host_x && P->m >= 2 && P->m <= 8 && tables_enabled() && !P->tab_only) {
     const size_t M = (size_t)D->M, cm = 2 * (size_t)P->m + 1;

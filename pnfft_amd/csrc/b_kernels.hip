@@ -408,7 +408,7 @@ struct AxisLoad {
   float dpsi[WG ? CM : 1];
 };
 
-// blocks take the tiles torder[first + blockIdx.x]
+// blocks take the order entries first + blockIdx.x
 // RG: the real grid of a c2r plan (imaginary parts zero: staged as zeros, and
 // the products that would multiply them are left out)
 template <int MT, int MODE, int NW, bool RG>
@@ -425,13 +425,14 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
   const int li = lane & 15, lk = lane >> 4;
   float* rows = s_gi + P * 256 + wave * S::ROWSZ;  // this wave's window rows
 
-  const int tile = A.torder[first + blockIdx.x];
+  const int4 range = A.oranges[first + blockIdx.x];
+  const int tile = range.x;
   const int t2 = tile % A.ntile[2];
   const int t1 = (tile / A.ntile[2]) % A.ntile[1];
   const int t0 = tile / (A.ntile[2] * A.ntile[1]);
   const int o0 = t0 * TS, o1 = t1 * TS, o2 = t2 * TS;
   const unsigned n0 = A.g.n[0], n1 = A.g.n[1], n2 = A.g.n[2];
-  const int beg = A.tile_start[tile], end = A.tile_start[tile + 1];
+  const int beg = range.y, end = range.w;
 
   // stage the subgrid, split into real and imaginary parts; pairs of cells along c
   if constexpr (P < 16) {
@@ -865,7 +866,7 @@ bool mfma_gather(const BArgs<R>& A) {
     return false;
   } else {
     constexpr int TS = GatherMfmaShape<MT, MODE, 4>::TS;
-    return !A.no_mfma && A.torder && A.n_torder > 0 && A.stale_count && A.stale_list && A.ts[0] == TS &&
+    return !A.no_mfma && A.torder && A.oranges && A.n_torder > 0 && A.stale_count && A.stale_list && A.ts[0] == TS &&
            A.ts[1] == TS && A.ts[2] == TS;
   }
 }

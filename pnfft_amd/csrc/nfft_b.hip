@@ -12,6 +12,7 @@
 // s = 0..2m (cutoff 2m+1, :910, :2165-2174).  floor(n x) is taken in FP64 for
 // both precisions; the window is evaluated in the compute precision from the
 // FP64 fractional part.
+#include <algorithm>
 #include <cstdio>
 #include <mutex>
 
@@ -28,43 +29,71 @@ constexpr int kB = 256;  // threads per block of the B kernels
 
 // ---------------------------------------------------------------------------
 // binning: keys, stable LSD radix sort, tile bounds
+//
+// Up to about 2^21 nodes it is bound by the number of dependent launches and
+// host waits, not by bytes: three launches per digit pass (the first pass takes
+// its counts from the key kernel), four for the tile lists, one host wait.  With
+// five launches per pass, separate kernels for the items, classes and bounds and
+// five waits a binning took 357 us at M = 2^19 (now 135) and 365 at 2^20 (now 148).
 // ---------------------------------------------------------------------------
 constexpr int kSortT = 256;
-constexpr int kSortIPB = 4096;  // items per block
 constexpr int kScanChunk = 4096;
 
-template <class R>
-__global__ __launch_bounds__(kB) void bin_keys_k(const R* __restrict__ x, long M, GridGeom g, TileLayout T,
-                                                 unsigned* keys, int* vals) {
-  const long j = (long)blockIdx.x * kB + threadIdx.x;
-  if (j >= M) return;
-  unsigned long long tile = 0;
-  unsigned l[3];
-  for (int t = 0; t < 3; t++) {
-    const NodeAxis<R> a = node_axis<R>(x[3 * j + t], g.n[t], g.m, g.shift);
-    tile = tile * T.ntile[t] + (unsigned)(a.start / T.ts[t]);
-    l[t] = (unsigned)(a.start % T.ts[t]);
-  }
+// Items per block of the sort passes.  A block ranks its items 256 at a time, a
+// chain of barriers, so small node sets take small blocks (M = 20001: 20 us per
+// pass with 4096 items, 8 us with 1024); from 2^20 nodes on 4096 items fill the
+// chip and keep the digit counts few.
+inline int sort_ipb(long M) { return M <= (1L << 18) ? 1024 : (M <= (1L << 20) ? 2048 : 4096); }
+inline long sort_blocks(long M) { return (M + sort_ipb(M) - 1) / sort_ipb(M); }
+
+// Bin key of every node, and the counts of the keys' lowest digit per block of
+// IPB items (digit-major: hist[d nblk + block]).
+template <class R, int IPB>
+__global__ __launch_bounds__(kSortT) void bin_keys_k(const R* __restrict__ x, long M, GridGeom g, TileLayout T,
+                                                     unsigned* keys, unsigned* hist, int nblk) {
+  __shared__ unsigned h[256];
+  const int tid = threadIdx.x;
+  h[tid] = 0;
+  __syncthreads();
   // cell order inside a tile: runs of q = min(TS2, 4) cells along axis 2
   // outermost, then axis 0, axis 1 and the cell within the run, so that
   // consecutive nodes of a tile share the quarter of axis 2 their stencils start
   // in (the matrix-core gather then skips one of its four K-blocks for most
   // 16-node groups)
   const unsigned q = T.ts[2] < 4 ? (unsigned)T.ts[2] : 4u;
-  const unsigned long long in =
-      ((unsigned long long)(l[2] / q) * (T.ts[0] * T.ts[1]) + l[0] * T.ts[1] + l[1]) * q + l[2] % q;
-  keys[j] = (unsigned)(tile * (unsigned long long)(T.ts[0] * T.ts[1] * T.ts[2]) + in);
-  vals[j] = (int)j;
+  const long base = (long)blockIdx.x * IPB;
+#pragma unroll 4
+  for (int i = 0; i < IPB / kSortT; i++) {
+    const long j = base + (long)i * kSortT + tid;
+    if (j < M) {
+      unsigned long long tile = 0;
+      unsigned l[3];
+      for (int t = 0; t < 3; t++) {
+        const NodeAxis<R> a = node_axis<R>(x[3 * j + t], g.n[t], g.m, g.shift);
+        tile = tile * T.ntile[t] + (unsigned)(a.start / T.ts[t]);
+        l[t] = (unsigned)(a.start % T.ts[t]);
+      }
+      const unsigned long long in =
+          ((unsigned long long)(l[2] / q) * (T.ts[0] * T.ts[1]) + l[0] * T.ts[1] + l[1]) * q + l[2] % q;
+      const unsigned key = (unsigned)(tile * (unsigned long long)(T.ts[0] * T.ts[1] * T.ts[2]) + in);
+      keys[j] = key;
+      atomicAdd(&h[key & 255u], 1u);
+    }
+  }
+  __syncthreads();
+  hist[(long)tid * nblk + blockIdx.x] = h[tid];
 }
 
+template <int IPB>
 __global__ __launch_bounds__(kSortT) void sort_hist_k(const unsigned* __restrict__ keys, long M, int shift,
                                                       unsigned* hist, int nblk) {
   __shared__ unsigned h[256];
   const int tid = threadIdx.x;
   h[tid] = 0;
   __syncthreads();
-  const long base = (long)blockIdx.x * kSortIPB;
-  for (int i = 0; i < kSortIPB / kSortT; i++) {
+  const long base = (long)blockIdx.x * IPB;
+#pragma unroll 4
+  for (int i = 0; i < IPB / kSortT; i++) {
     const long idx = base + (long)i * kSortT + tid;
     if (idx < M) atomicAdd(&h[(keys[idx] >> shift) & 255u], 1u);
   }
@@ -89,53 +118,78 @@ __device__ inline unsigned block_exscan256(unsigned v, unsigned* tmp, unsigned* 
   return incl - v;
 }
 
-// chunk sums
-__global__ __launch_bounds__(kSortT) void scan_reduce_k(const unsigned* __restrict__ d, long n, unsigned* partial) {
-  __shared__ unsigned tmp[256];
-  const long base = (long)blockIdx.x * kScanChunk;
-  unsigned s = 0;
-  for (int i = 0; i < kScanChunk / kSortT; i++) {
-    const long idx = base + (long)threadIdx.x * (kScanChunk / kSortT) + i;
-    if (idx < n) s += d[idx];
-  }
-  unsigned total;
-  __shared__ unsigned tot;
-  (void)block_exscan256(s, tmp, &tot);
-  total = tot;
-  if (threadIdx.x == 0) partial[blockIdx.x] = total;
-}
-
-// exclusive scan of the chunk sums, one block, sequential over 256-wide pieces
-__global__ __launch_bounds__(kSortT) void scan_partials_k(unsigned* partial, long np) {
-  __shared__ unsigned tmp[256];
+// exclusive scan in place of d[0, n) by one block, 16 values per thread and round
+__device__ inline void block_scan(unsigned* d, long n, unsigned* tmp, unsigned* total) {
+  constexpr int PER = 16;
   __shared__ unsigned tot;
   unsigned carry = 0;
-  for (long base = 0; base < np; base += 256) {
-    const long idx = base + threadIdx.x;
-    const unsigned v = idx < np ? partial[idx] : 0u;
-    const unsigned ex = block_exscan256(v, tmp, &tot);
-    if (idx < np) partial[idx] = ex + carry;
+  for (long base = 0; base < n; base += 256 * PER) {
+    const long at = base + (long)threadIdx.x * PER;
+    unsigned loc[PER], s = 0;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      loc[i] = at + i < n ? d[at + i] : 0u;
+      s += loc[i];
+    }
+    unsigned ex = block_exscan256(s, tmp, &tot) + carry;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      if (at + i < n) d[at + i] = ex;
+      ex += loc[i];
+    }
     carry += tot;
     __syncthreads();
   }
+  if (total && threadIdx.x == 0) *total = carry;
+}
+
+// block d: exclusive scan of digit d's per-block counts in place; total[d] = their sum
+__global__ __launch_bounds__(kSortT) void digit_scan_k(unsigned* hist, int nblk, unsigned* total) {
+  __shared__ unsigned tmp[256];
+  block_scan(hist + (long)blockIdx.x * nblk, nblk, tmp, total + blockIdx.x);
+}
+
+// Exclusive scans of several arrays of n values (array blockIdx.y at d +
+// blockIdx.y n): one block per array, or chunk sums, their scan and its addition.
+__global__ __launch_bounds__(kSortT) void scan_whole_k(unsigned* d, long n) {
+  __shared__ unsigned tmp[256];
+  block_scan(d + (long)blockIdx.y * n, n, tmp, nullptr);
+}
+
+__global__ __launch_bounds__(kSortT) void scan_reduce_k(const unsigned* __restrict__ d, long n, unsigned* partial) {
+  __shared__ unsigned tmp[256];
+  __shared__ unsigned tot;
+  constexpr int PER = kScanChunk / kSortT;
+  const long base = (long)blockIdx.x * kScanChunk + (long)threadIdx.x * PER;
+  unsigned s = 0;
+  for (int i = 0; i < PER; i++)
+    if (base + i < n) s += d[(long)blockIdx.y * n + base + i];
+  (void)block_exscan256(s, tmp, &tot);
+  if (threadIdx.x == 0) partial[(long)blockIdx.y * gridDim.x + blockIdx.x] = tot;
+}
+
+__global__ __launch_bounds__(kSortT) void scan_partials_k(unsigned* partial, long np) {
+  __shared__ unsigned tmp[256];
+  block_scan(partial + (long)blockIdx.y * np, np, tmp, nullptr);
 }
 
 __global__ __launch_bounds__(kSortT) void scan_apply_k(unsigned* d, long n, const unsigned* __restrict__ partial) {
   __shared__ unsigned tmp[256];
   __shared__ unsigned tot;
   constexpr int PER = kScanChunk / kSortT;
+  unsigned* const dd = d + (long)blockIdx.y * n;
   const long base = (long)blockIdx.x * kScanChunk + (long)threadIdx.x * PER;
   unsigned loc[PER];
   unsigned s = 0;
   for (int i = 0; i < PER; i++) {
     const long idx = base + i;
-    loc[i] = idx < n ? d[idx] : 0u;
+    loc[i] = idx < n ? dd[idx] : 0u;
     s += loc[i];
   }
-  unsigned ex = block_exscan256(s, tmp, &tot) + partial[blockIdx.x];
+  unsigned ex = block_exscan256(s, tmp, &tot) + partial[(long)blockIdx.y * gridDim.x + blockIdx.x];
   for (int i = 0; i < PER; i++) {
     const long idx = base + i;
-    if (idx < n) d[idx] = ex;
+    if (idx < n) dd[idx] = ex;
     ex += loc[i];
   }
 }
@@ -143,12 +197,15 @@ __global__ __launch_bounds__(kSortT) void scan_apply_k(unsigned* d, long n, cons
 // Stable scatter of one digit pass: items of a block are ranked in index order
 // and placed by digit in LDS first, so that the stores to the output are runs
 // of consecutive positions (one per digit present in the block) rather than
-// one scattered 4-byte store per item.  offs: the exclusive scan of the
-// per-(digit, block) counts in digit-major order, so that a count is the
-// difference of neighbouring entries.
+// one scattered 4-byte store per item.  offs: per digit, the exclusive scan of
+// its per-block counts (digit_scan_k), total: the digits' counts, whose scan
+// every block forms itself.  vin null: the first pass, item ids in order.
+template <int IPB>
 __global__ __launch_bounds__(kSortT) void sort_scatter_k(const unsigned* __restrict__ kin, const int* __restrict__ vin,
                                                          unsigned* kout, int* vout, long M, int shift,
-                                                         const unsigned* __restrict__ offs, int nblk) {
+                                                         const unsigned* __restrict__ offs,
+                                                         const unsigned* __restrict__ total, int nblk) {
+  constexpr int kSortIPB = IPB;
   __shared__ unsigned run[256];
   __shared__ unsigned wcnt[4][256];
   __shared__ unsigned loc[256];   // first LDS position of digit d
@@ -161,8 +218,9 @@ __global__ __launch_bounds__(kSortT) void sort_scatter_k(const unsigned* __restr
   const long base = (long)blockIdx.x * kSortIPB;
   {
     const long e = (long)tid * nblk + blockIdx.x;  // entry (digit tid, this block)
-    const unsigned o = offs[e];
-    const unsigned c = (e + 1 < 256L * nblk ? offs[e + 1] : (unsigned)M) - o;
+    const unsigned in = offs[e], all = total[tid];
+    const unsigned c = ((int)blockIdx.x + 1 < nblk ? offs[e + 1] : all) - in;
+    const unsigned o = block_exscan256(all, tmp, nullptr) + in;
     const unsigned l = block_exscan256(c, tmp, nullptr);
     loc[tid] = l;
     gdst[tid] = o - l;
@@ -177,7 +235,7 @@ __global__ __launch_bounds__(kSortT) void sort_scatter_k(const unsigned* __restr
     unsigned d = 0;
     if (valid) {
       key = kin[idx];
-      val = vin[idx];
+      val = vin ? vin[idx] : (int)idx;
       d = (key >> shift) & 255u;
     }
 #pragma unroll
@@ -213,39 +271,22 @@ __global__ __launch_bounds__(kSortT) void sort_scatter_k(const unsigned* __restr
   }
 }
 
-__global__ void fill_int_k(int* p, long n, int v) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
-}
-
+// First sorted position of every tile by bisection (a walk over the keys would
+// leave the gap before a tile to one thread: clustered nodes), and cleared
+// counters and offset masks.
 __global__ __launch_bounds__(kB) void tile_bounds_k(const unsigned* __restrict__ skeys, long M, unsigned vol,
-                                                    int* tile_start) {
-  const long i = (long)blockIdx.x * kB + threadIdx.x;
-  if (i >= M) return;
-  const long t = skeys[i] / vol;
-  const long tprev = (i == 0) ? -1 : (long)(skeys[i - 1] / vol);
-  for (long tt = tprev + 1; tt <= t; tt++) tile_start[tt] = (int)i;
-}
-
-__global__ __launch_bounds__(kB) void tile_chunks_k(const int* __restrict__ tile_start, long ntiles, int dense_min,
-                                                    unsigned* chunks, unsigned char* dense) {
+                                                    long ntiles, int* tile_start, unsigned* work, unsigned* box) {
   const long t = (long)blockIdx.x * kB + threadIdx.x;
-  if (t >= ntiles) return;
-  const int cnt = tile_start[t + 1] - tile_start[t];
-  const bool d = cnt >= dense_min && cnt > 0;
-  dense[t] = d ? 1 : 0;
-  chunks[t] = d ? (unsigned)((cnt + kTileNodes - 1) / kTileNodes) : 0u;
-}
-
-__global__ __launch_bounds__(kB) void tile_items_k(const unsigned* __restrict__ chunks,
-                                                   const unsigned* __restrict__ offs, long ntiles, int* items) {
-  const long t = (long)blockIdx.x * kB + threadIdx.x;
-  if (t >= ntiles) return;
-  const unsigned c = chunks[t], o = offs[t];
-  for (unsigned k = 0; k < c; k++) {
-    items[2 * (o + k)] = (int)t;
-    items[2 * (o + k) + 1] = (int)k;
+  if (t < kTileWork) work[t] = 0u;
+  if (t > ntiles) return;
+  long lo = 0, hi = M;
+  while (lo < hi) {
+    const long c = (lo + hi) >> 1;
+    if ((long)(skeys[c] / vol) < t) lo = c + 1;
+    else hi = c;
   }
+  tile_start[t] = (int)lo;
+  if (t < ntiles) box[t] = 0u;
 }
 
 // For each class of the wave's active lanes, one lane adds the class's lane
@@ -274,87 +315,135 @@ __device__ inline unsigned wave_class_add(bool act, int cls, unsigned* ctr) {
 // gathered in LDS over this many tiles, so that a block adds each class to the
 // global counters once (per-wave global atomics on the 32 counters serialize).
 constexpr int kClassTiles = 8 * kB;
+// (one tile per thread for small grids, where eight in a row would be a chain)
+inline int class_rounds(long ntiles) { return ntiles > 65536 ? kClassTiles / kB : 1; }
 
-// nonempty tiles by node-count class (leading zeros of the count: more nodes,
-// smaller class), then placed class by class: most nodes first
-__global__ __launch_bounds__(kB) void tile_class_k(const int* __restrict__ tile_start, long ntiles, unsigned* work,
-                                                   int* tile_slot) {
+// Slots (order entries) of a tile: one, or one per part_nodes nodes.
+__device__ inline unsigned tile_parts(int cnt, int part_nodes) {
+  return cnt > part_nodes ? (unsigned)((cnt + part_nodes - 1) / part_nodes) : (cnt > 0 ? 1u : 0u);
+}
+
+// Per tile: order entries by node-count class (leading zeros of the count: more
+// nodes, smaller class) added to work[class], and the values whose scans place
+// the tile: flag of 2..31 nodes, flag of one node, work items of the gather (and
+// of the scatter, where they differ).
+__global__ __launch_bounds__(kB) void tile_class_k(const int* __restrict__ tile_start, long ntiles, int dense_min,
+                                                   int part_nodes, bool two_lists, int rounds, unsigned* work,
+                                                   unsigned* scan, unsigned char* dense, unsigned char* dense_s) {
   __shared__ unsigned lc[32];
   if (threadIdx.x < 32) lc[threadIdx.x] = 0;
   __syncthreads();
-  for (int i = 0; i < kClassTiles / kB; i++) {
-    const long t = (long)blockIdx.x * kClassTiles + (long)i * kB + threadIdx.x;
+  for (int i = 0; i < rounds; i++) {
+    const long t = ((long)blockIdx.x * rounds + i) * kB + threadIdx.x;
     const int cnt = t < ntiles ? tile_start[t + 1] - tile_start[t] : 0;
-    if (t < ntiles) tile_slot[t] = -1;
+    if (t < ntiles) {
+      const bool d = cnt >= dense_min && cnt > 0;
+      const unsigned ch = (unsigned)((cnt + kTileNodes - 1) / kTileNodes);
+      dense[t] = d ? 1 : 0;
+      dense_s[t] = cnt > 0 ? 1 : 0;
+      scan[t] = (cnt > 1 && cnt < 32) ? 1u : 0u;
+      scan[ntiles + t] = cnt == 1 ? 1u : 0u;
+      scan[2 * ntiles + t] = d ? ch : 0u;
+      if (two_lists) scan[3 * ntiles + t] = ch;
+    }
+    const unsigned parts = tile_parts(cnt, part_nodes);
     (void)wave_class_add(cnt > 0, cnt > 0 ? __clz(cnt) : 0, lc);
+    if (parts > 1) atomicAdd(&lc[__clz(cnt)], parts - 1);
   }
   __syncthreads();
   if (threadIdx.x < 32 && lc[threadIdx.x]) atomicAdd(&work[threadIdx.x], lc[threadIdx.x]);
 }
 
-// work[0..31] class sizes -> work[32..63] class offsets, work[64] total
-__global__ void tile_class_scan_k(unsigned* work) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  unsigned acc = 0;
-  for (int k = 0; k < 32; k++) {
-    work[32 + k] = acc;
-    acc += work[k];
-  }
-  work[64] = acc;
-}
-
-// tiles of 2..31 nodes (classes 27..30): flag[t] = 1; tiles of one node (class
-// 31): flag[ntiles + t] = 1
-__global__ __launch_bounds__(kB) void tile_light_k(const int* __restrict__ tile_start, long ntiles, unsigned* flag) {
-  const long t = (long)blockIdx.x * kB + threadIdx.x;
-  if (t >= ntiles) return;
-  const int cnt = tile_start[t + 1] - tile_start[t];
-  flag[t] = (cnt > 1 && cnt < 32) ? 1u : 0u;
-  flag[ntiles + t] = cnt == 1 ? 1u : 0u;
-}
-
-// Tiles of 32 nodes or more are placed class by class (most nodes first; in a
-// class, block by block, a block's tiles in the order of their LDS ranks); the
-// tiles of 2..31 nodes follow in tile order (light_off = exclusive scan of
-// their flags), so that neighbouring light tiles, whose padded subgrids
-// overlap, are taken by neighbouring blocks, and the tiles of one node come
-// last, in tile order as well (single_off).
-__global__ __launch_bounds__(kB) void tile_place_k(const int* __restrict__ tile_start, long ntiles, unsigned* work,
-                                                   const unsigned* __restrict__ light_off,
-                                                   const unsigned* __restrict__ single_off, int* order,
-                                                   int* tile_slot) {
+// Order entries of tiles of 32 nodes or more are placed class by class (most
+// nodes first; in a class, block by block), a tile's entries together; the tiles
+// of 2..31 nodes follow in tile order (scanned flags), so that neighbouring light
+// tiles, whose padded subgrids overlap, are taken by neighbouring blocks, and the
+// tiles of one node come last, in tile order as well.  tile_slot[t] = (first
+// entry of tile t, -1: none; entries).  ranges, oranges (or null): the position
+// ranges of the gather's work items and of the order entries; the nodes of a
+// range from mid on start in the upper half of axis 2, by bisection of the keys,
+// whose in-tile index counts the runs of four cells along axis 2 outermost.
+__global__ __launch_bounds__(kB) void tile_place_k(const int* __restrict__ tile_start, long ntiles, int dense_min,
+                                                   int part_nodes, bool two_lists, int rounds,
+                                                   const unsigned* __restrict__ keys, unsigned vol, unsigned* work,
+                                                   const unsigned* __restrict__ scan, int* items, int* items_s,
+                                                   int* order, int2* tile_slot, int4* ranges, int4* oranges) {
   constexpr int NI = kClassTiles / kB;
   __shared__ unsigned lc[32], gb[32];
+  __shared__ unsigned light0, single0;
   if (threadIdx.x < 32) lc[threadIdx.x] = 0;
   __syncthreads();
   unsigned lpos[NI];
 #pragma unroll
   for (int i = 0; i < NI; i++) {
-    const long t = (long)blockIdx.x * kClassTiles + (long)i * kB + threadIdx.x;
+    if (i >= rounds) break;
+    const long t = ((long)blockIdx.x * rounds + i) * kB + threadIdx.x;
     const int cnt = t < ntiles ? tile_start[t + 1] - tile_start[t] : 0;
-    lpos[i] = wave_class_add(cnt >= 32, cnt > 0 ? __clz(cnt) : 0, lc);
+    const unsigned parts = tile_parts(cnt, part_nodes);
+    lpos[i] = wave_class_add(cnt >= 32 && parts == 1, cnt > 0 ? __clz(cnt) : 0, lc);
+    if (cnt >= 32 && parts > 1) lpos[i] = atomicAdd(&lc[__clz(cnt)], parts);
   }
   __syncthreads();
-  if (threadIdx.x < 32 && lc[threadIdx.x]) gb[threadIdx.x] = atomicAdd(&work[32 + threadIdx.x], lc[threadIdx.x]);
+  // classes before class k: work[0 .. k); work[32 + k] counts the entries placed
+  if (threadIdx.x < 32) {
+    unsigned before = 0;
+    for (int k = 0; k < 32; k++) {
+      if (k < (int)threadIdx.x) before += work[k];
+    }
+    if (lc[threadIdx.x]) gb[threadIdx.x] = before + atomicAdd(&work[32 + threadIdx.x], lc[threadIdx.x]);
+    if (threadIdx.x == 27) light0 = before;
+    if (threadIdx.x == 31) single0 = before;
+  }
   __syncthreads();
-  // class 27 starts after the heavy tiles; work[27..30] are the sizes of classes 27..30
-  const unsigned light0 = work[32 + 27];
-  const unsigned single0 = light0 + work[27] + work[28] + work[29] + work[30];
+  auto mid_of = [&](int lo, int hi) {
+    while (lo < hi) {
+      const int c = (lo + hi) >> 1;
+      if (keys[c] % vol < vol / 2) lo = c + 1;
+      else hi = c;
+    }
+    return lo;
+  };
 #pragma unroll
   for (int i = 0; i < NI; i++) {
-    const long t = (long)blockIdx.x * kClassTiles + (long)i * kB + threadIdx.x;
-    const int cnt = t < ntiles ? tile_start[t + 1] - tile_start[t] : 0;
+    const long t = ((long)blockIdx.x * rounds + i) * kB + threadIdx.x;
+    if (i >= rounds || t >= ntiles) continue;
+    const int beg = tile_start[t], end = tile_start[t + 1], cnt = end - beg;
+    const unsigned parts = tile_parts(cnt, part_nodes);
+    unsigned p = 0;
     if (cnt > 0) {
-      const unsigned p = cnt >= 32 ? gb[__clz(cnt)] + lpos[i] : cnt > 1 ? light0 + light_off[t] : single0 + single_off[t];
-      order[p] = (int)t;
-      tile_slot[t] = (int)p;
+      p = cnt >= 32 ? gb[__clz(cnt)] + lpos[i] : cnt > 1 ? light0 + scan[t] : single0 + scan[ntiles + t];
+      const int mid = oranges ? mid_of(beg, end) : end;
+      for (unsigned k = 0; k < parts; k++) {
+        order[p + k] = (int)t;
+        if (oranges) {
+          const int b = beg + (int)k * part_nodes, e = parts > 1 ? min(end, b + part_nodes) : end;
+          oranges[p + k] = make_int4((int)t, b, min(max(mid, b), e), e);
+        }
+      }
+      const unsigned o = scan[2 * ntiles + t], ch = (unsigned)((cnt + kTileNodes - 1) / kTileNodes);
+      for (unsigned k = 0; k < ch; k++) {
+        if (cnt >= dense_min) {
+          items[2 * (o + k)] = (int)t;
+          items[2 * (o + k) + 1] = (int)k;
+          if (ranges) {
+            const int b = beg + (int)k * kTileNodes, e = min(end, b + kTileNodes);
+            ranges[o + k] = make_int4((int)t, b, min(max(mid, b), e), e);
+          }
+        }
+        if (two_lists) {
+          const unsigned os = scan[3 * ntiles + t];
+          items_s[2 * (os + k)] = (int)t;
+          items_s[2 * (os + k) + 1] = (int)k;
+        }
+      }
+    }
+    tile_slot[t] = cnt > 0 ? make_int2((int)p, (int)parts) : make_int2(-1, 0);
+    if (t == ntiles - 1) {
+      const unsigned ch = (unsigned)((cnt + kTileNodes - 1) / kTileNodes);
+      work[64] = scan[2 * ntiles + t] + (cnt >= dense_min ? ch : 0u);
+      work[65] = two_lists ? scan[3 * ntiles + t] + ch : work[64];
     }
   }
-}
-
-__global__ void fill_uint_k(unsigned* p, long n, unsigned v) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
 }
 
 template <class R>
@@ -373,12 +462,39 @@ int sort_passes(unsigned long long key_limit) {
   return (bits + 7) / 8;
 }
 
-static int scan_exclusive(unsigned* d, long n, unsigned* partial, hipStream_t s) {
+// exclusive scans in place of `arrays` arrays of n values each, one after the other at d
+static void scan_exclusive(unsigned* d, long n, int arrays, unsigned* partial, hipStream_t s) {
   const long nch = (n + kScanChunk - 1) / kScanChunk;
-  hipLaunchKernelGGL(scan_reduce_k, dim3(grid1d(nch * 1, 1)), dim3(kSortT), 0, s, d, n, partial);
-  hipLaunchKernelGGL(scan_partials_k, dim3(1), dim3(kSortT), 0, s, partial, nch);
-  hipLaunchKernelGGL(scan_apply_k, dim3(grid1d(nch, 1)), dim3(kSortT), 0, s, d, n, partial);
-  return kOk;
+  if (nch <= 4) {  // one block per array in one launch
+    hipLaunchKernelGGL(scan_whole_k, dim3(1, arrays), dim3(kSortT), 0, s, d, n);
+    return;
+  }
+  const dim3 grid((unsigned)nch, arrays);
+  hipLaunchKernelGGL(scan_reduce_k, grid, dim3(kSortT), 0, s, d, n, partial);
+  hipLaunchKernelGGL(scan_partials_k, dim3(1, arrays), dim3(kSortT), 0, s, partial, nch);
+  hipLaunchKernelGGL(scan_apply_k, grid, dim3(kSortT), 0, s, d, n, partial);
+}
+
+long sort_hist_words(long M) { return 256 * std::max(sort_blocks(M), 1L); }
+
+template <class R, int IPB>
+static void sort_passes_launch(const R* x, long M, const GridGeom& g, const TileLayout& T, SortWork& W, int passes,
+                               int* perm_out, unsigned* keys_out, hipStream_t s) {
+  const int nblk = (int)((M + IPB - 1) / IPB);
+  hipLaunchKernelGGL((bin_keys_k<R, IPB>), dim3(nblk), dim3(kSortT), 0, s, x, M, g, T, W.keys[0], W.hist, nblk);
+  // the last pass stores straight into the outputs (separate from the scratch)
+  int cur = 0;
+  for (int ps = 0; ps < passes; ps++) {
+    const int shift = 8 * ps;
+    const bool last = ps == passes - 1;
+    if (ps > 0)
+      hipLaunchKernelGGL((sort_hist_k<IPB>), dim3(nblk), dim3(kSortT), 0, s, W.keys[cur], M, shift, W.hist, nblk);
+    hipLaunchKernelGGL(digit_scan_k, dim3(256), dim3(kSortT), 0, s, W.hist, nblk, W.total);
+    hipLaunchKernelGGL((sort_scatter_k<IPB>), dim3(nblk), dim3(kSortT), 0, s, W.keys[cur],
+                       ps > 0 ? W.vals[cur] : nullptr, last ? keys_out : W.keys[1 - cur],
+                       last ? perm_out : W.vals[1 - cur], M, shift, W.hist, W.total, nblk);
+    cur = 1 - cur;
+  }
 }
 
 // Bin keys of the M nodes sorted stably (LSD radix, 8-bit digits) with the
@@ -388,57 +504,36 @@ static int sort_bins(const R* x, long M, const GridGeom& g, const TileLayout& T,
                      unsigned* keys_out, hipStream_t s) {
   const unsigned long long key_limit = (unsigned long long)T.ntiles() * (unsigned long long)T.tile_vol();
   if (key_limit > (1ull << 32)) return kUnsupported;
-  const int passes = sort_passes(key_limit);
-  const int nblk = (int)((M + kSortIPB - 1) / kSortIPB);
-  hipLaunchKernelGGL((bin_keys_k<R>), dim3(grid1d(M, kB)), dim3(kB), 0, s, x, M, g, T, W.keys[0], W.vals[0]);
-  // the last pass stores straight into the outputs (separate from the scratch)
-  int cur = 0;
-  for (int ps = 0; ps < passes; ps++) {
-    const int shift = 8 * ps;
-    const bool last = ps == passes - 1;
-    hipLaunchKernelGGL(sort_hist_k, dim3(nblk), dim3(kSortT), 0, s, W.keys[cur], M, shift, W.hist, nblk);
-    scan_exclusive(W.hist, 256L * nblk, W.partial, s);
-    hipLaunchKernelGGL(sort_scatter_k, dim3(nblk), dim3(kSortT), 0, s, W.keys[cur], W.vals[cur],
-                       last ? keys_out : W.keys[1 - cur], last ? perm_out : W.vals[1 - cur], M, shift, W.hist,
-                       nblk);
-    cur = 1 - cur;
-  }
-  if (passes == 0) {  // keys below 2: already in order
-    if (hipMemcpyAsync(perm_out, W.vals[0], sizeof(int) * M, hipMemcpyDeviceToDevice, s) != hipSuccess)
-      return kHipError;
-    if (hipMemcpyAsync(keys_out, W.keys[0], sizeof(unsigned) * M, hipMemcpyDeviceToDevice, s) != hipSuccess)
-      return kHipError;
+  const int passes = std::max(1, sort_passes(key_limit));  // keys below 2 take one pass as well
+  switch (sort_ipb(M)) {
+    case 1024: sort_passes_launch<R, 1024>(x, M, g, T, W, passes, perm_out, keys_out, s); break;
+    case 2048: sort_passes_launch<R, 2048>(x, M, g, T, W, passes, perm_out, keys_out, s); break;
+    default: sort_passes_launch<R, 4096>(x, M, g, T, W, passes, perm_out, keys_out, s); break;
   }
   return hipGetLastError() == hipSuccess ? kOk : kHipError;
 }
 
 template <class R>
 int bin_nodes(const R* x, long M, const GridGeom& g, const TileLayout& T, SortWork& W, int* perm_out,
-              unsigned* keys_out, int* tile_start, hipStream_t s) {
-  const long ntiles = T.ntiles();
-  hipLaunchKernelGGL(fill_int_k, dim3(grid1d(ntiles + 1, 256)), dim3(256), 0, s, tile_start, ntiles + 1, (int)M);
-  if (M == 0) return hipGetLastError() == hipSuccess ? kOk : kHipError;
-  const int st = sort_bins<R>(x, M, g, T, W, perm_out, keys_out, s);
-  if (st != kOk) return st;
-  hipLaunchKernelGGL(tile_bounds_k, dim3(grid1d(M, kB)), dim3(kB), 0, s, keys_out, M, (unsigned)T.tile_vol(),
-                     tile_start);
-  return hipGetLastError() == hipSuccess ? kOk : kHipError;
+              unsigned* keys_out, hipStream_t s) {
+  if (M == 0) return kOk;
+  return sort_bins<R>(x, M, g, T, W, perm_out, keys_out, s);
 }
 
 // ---------------------------------------------------------------------------
 // binning without allocation: the sort's scratch (two key and two id buffers,
-// the digit histograms and their scan partials) lives in one file-scope device
+// the digits' per-block counts and totals) lives in one file-scope device
 // array per GPU, of kNoAllocMaxNodes nodes at most.  Its address is taken once
 // per device with hipGetSymbolAddress (the host-side name is not a device
 // address); every call on a GPU shares that GPU's array, so calls that overlap
 // on one GPU race.  Every scratch word a call reads was written earlier by the
-// same call (the histograms are rebuilt per pass), so nothing needs clearing.
+// same call (the digit counts are rebuilt per pass), so nothing needs clearing.
 // ---------------------------------------------------------------------------
 namespace {
-constexpr long kNaBlocks = (kNoAllocMaxNodes + kSortIPB - 1) / kSortIPB;
+constexpr long kNaBlocks = 512;  // sort_blocks() of up to kNoAllocMaxNodes nodes
+static_assert(kNoAllocMaxNodes <= 2048 * kNaBlocks && (1L << 18) <= 1024 * kNaBlocks, "digit counts of every M fit");
 constexpr long kNaHist = 256L * kNaBlocks;
-constexpr long kNaPartial = (kNaHist + kScanChunk - 1) / kScanChunk + 1;
-constexpr long kNaWords = 4 * kNoAllocMaxNodes + kNaHist + kNaPartial;
+constexpr long kNaWords = 4 * kNoAllocMaxNodes + kNaHist + 256;
 }  // namespace
 
 static __device__ __align__(256) unsigned scratch[kNaWords];
@@ -478,62 +573,8 @@ int bin_nodes_noalloc(const R* x, long M, const GridGeom& g, const TileLayout& T
   W.vals[0] = reinterpret_cast<int*>(base + 2 * kNoAllocMaxNodes);
   W.vals[1] = reinterpret_cast<int*>(base + 3 * kNoAllocMaxNodes);
   W.hist = base + 4 * kNoAllocMaxNodes;
-  W.partial = W.hist + kNaHist;
-  W.cap = kNoAllocMaxNodes;
-  W.hist_cap = kNaHist;
-  W.partial_cap = kNaPartial;
+  W.total = W.hist + kNaHist;
   return sort_bins<R>(x, M, g, T, W, perm_out, keys_out, s);
-}
-
-int build_items(const int* tile_start, long ntiles, int dense_min, unsigned* chunks, unsigned* partial,
-                unsigned char* tile_dense, int* items, long items_cap, hipStream_t s) {
-  hipLaunchKernelGGL(tile_chunks_k, dim3(grid1d(ntiles, kB)), dim3(kB), 0, s, tile_start, ntiles, dense_min, chunks,
-                     tile_dense);
-  unsigned last_cnt = 0, last_off = 0;
-  if (hipMemcpyAsync(&last_cnt, chunks + ntiles - 1, sizeof(unsigned), hipMemcpyDeviceToHost, s) != hipSuccess)
-    return -1;
-  // chunks -> exclusive offsets in place (a copy of the last count was taken above)
-  if (hipStreamSynchronize(s) != hipSuccess) return -1;
-  unsigned* offs = chunks;
-  // keep counts: scan a copy held in the second half of the chunk buffer
-  if (hipMemcpyAsync(offs + ntiles, chunks, sizeof(unsigned) * ntiles, hipMemcpyDeviceToDevice, s) != hipSuccess)
-    return -1;
-  scan_exclusive(offs + ntiles, ntiles, partial, s);
-  if (hipMemcpyAsync(&last_off, offs + 2 * ntiles - 1, sizeof(unsigned), hipMemcpyDeviceToHost, s) != hipSuccess)
-    return -1;
-  if (hipStreamSynchronize(s) != hipSuccess) return -1;
-  const long total = (long)last_off + (long)last_cnt;
-  if (total > items_cap) return -1;
-  hipLaunchKernelGGL(tile_items_k, dim3(grid1d(ntiles, kB)), dim3(kB), 0, s, chunks, offs + ntiles, ntiles, items);
-  if (hipGetLastError() != hipSuccess) return -1;
-  return (int)total;
-}
-
-// one thread per item: bisection of its sorted keys, whose in-tile cell index
-// counts the runs of four cells along axis 2 outermost (bin_keys_k)
-__global__ __launch_bounds__(kB) void item_ranges_k(const int* __restrict__ items, int n_items, int chunked,
-                                                    const int* __restrict__ tile_start,
-                                                    const unsigned* __restrict__ keys, unsigned vol, int4* ranges) {
-  const int i = blockIdx.x * kB + threadIdx.x;
-  if (i >= n_items) return;
-  const int tile = chunked ? items[2 * i] : items[i];
-  const int beg = tile_start[tile] + (chunked ? items[2 * i + 1] * kTileNodes : 0);
-  const int end = chunked ? min(tile_start[tile + 1], beg + kTileNodes) : tile_start[tile + 1];
-  int lo = beg, hi = end;
-  while (lo < hi) {
-    const int c = (lo + hi) >> 1;
-    if (keys[c] % vol < vol / 2) lo = c + 1;
-    else hi = c;
-  }
-  ranges[i] = make_int4(tile, beg, lo, end);
-}
-
-int build_ranges(const int* items, int n_items, bool chunked, const int* tile_start, const unsigned* keys, unsigned tile_vol,
-                 int4* ranges, hipStream_t s) {
-  if (n_items <= 0) return kOk;
-  hipLaunchKernelGGL(item_ranges_k, dim3(grid1d(n_items, kB)), dim3(kB), 0, s, items, n_items, chunked ? 1 : 0,
-                     tile_start, keys, tile_vol, ranges);
-  return hipGetLastError() == hipSuccess ? kOk : kHipError;
 }
 
 int cols_pad(int m, bool is_double, const int* ts) {
@@ -575,43 +616,47 @@ __global__ __launch_bounds__(kB) void tile_box_k(const unsigned* __restrict__ ke
   if (live && (lane == 63 || tn != tile)) atomicOr(box + tile, m);
 }
 
-// box_ord[p] = box_tile[order[p]]: the masks by position in the tile order
-__global__ __launch_bounds__(kB) void box_order_k(const int* __restrict__ order, int n, const unsigned* __restrict__ box_tile,
-                                                  unsigned* box_ord) {
+// box_ord[p] = box_tile[order[p]] for the n order entries (n: work's class
+// counts, on the device): the masks by position in the tile order
+__global__ __launch_bounds__(kB) void box_order_k(const int* __restrict__ order, const unsigned* __restrict__ work,
+                                                  const unsigned* __restrict__ box_tile, unsigned* box_ord) {
   const int p = blockIdx.x * kB + threadIdx.x;
+  int n = 0;
+  for (int k = 0; k < 32; k++) n += (int)work[k];
   if (p < n) box_ord[p] = box_tile[order[p]];
 }
 
-int build_tile_boxes(const unsigned* keys, long M, const TileLayout& T, const int* order, int n_order,
-                     unsigned* box_tile, unsigned* box_ord, hipStream_t s) {
-  if (T.ts[0] > 8 || T.ts[1] > 8 || T.ts[2] > 8) return kUnsupported;
-  const long ntiles = T.ntiles();
-  hipLaunchKernelGGL(fill_uint_k, dim3(grid1d(ntiles, kB)), dim3(kB), 0, s, box_tile, ntiles, 0u);
-  if (M > 0) hipLaunchKernelGGL(tile_box_k, dim3(grid1d(M, kB)), dim3(kB), 0, s, keys, M, T, box_tile);
-  if (n_order > 0)
-    hipLaunchKernelGGL(box_order_k, dim3(grid1d(n_order, kB)), dim3(kB), 0, s, order, n_order, box_tile, box_ord);
-  return hipGetLastError() == hipSuccess ? kOk : kHipError;
-}
-
-int build_tile_order(const int* tile_start, long ntiles, unsigned* work, unsigned* light, unsigned* partial,
-                     int* order, int* tile_slot, int* n_heavy, int* n_single, hipStream_t s) {
-  hipLaunchKernelGGL(fill_uint_k, dim3(1), dim3(128), 0, s, work, 65L, 0u);
-  hipLaunchKernelGGL(tile_class_k, dim3(grid1d(ntiles, kClassTiles)), dim3(kB), 0, s, tile_start, ntiles, work,
-                     tile_slot);
-  hipLaunchKernelGGL(tile_class_scan_k, dim3(1), dim3(64), 0, s, work);
-  hipLaunchKernelGGL(tile_light_k, dim3(grid1d(ntiles, kB)), dim3(kB), 0, s, tile_start, ntiles, light);
-  scan_exclusive(light, ntiles, partial, s);
-  scan_exclusive(light + ntiles, ntiles, partial, s);
-  hipLaunchKernelGGL(tile_place_k, dim3(grid1d(ntiles, kClassTiles)), dim3(kB), 0, s, tile_start, ntiles, work,
-                     light, light + ntiles, order, tile_slot);
-  // work[k] is the size of class k; after the placement work[32 + k] is the end
-  // of class k for k <= 26 (32 nodes or more) and work[64] the total
-  unsigned w[65] = {0};
-  if (hipMemcpyAsync(w, work, 65 * sizeof(unsigned), hipMemcpyDeviceToHost, s) != hipSuccess) return -1;
-  if (hipStreamSynchronize(s) != hipSuccess) return -1;
-  if (n_heavy) *n_heavy = (int)w[32 + 26];
-  if (n_single) *n_single = (int)w[31];
-  return (int)w[64];
+int build_tile_lists(const unsigned* keys, long M, const TileLayout& T, int dense_min, int part_nodes, bool boxes,
+                     TileLists& L, TileCounts* out, hipStream_t s) {
+  const long nt = T.ntiles();
+  const bool two = dense_min > 1;
+  hipLaunchKernelGGL(tile_bounds_k, dim3(grid1d(std::max(nt + 1, (long)kTileWork), kB)), dim3(kB), 0, s, keys, M,
+                     (unsigned)T.tile_vol(), nt, L.tile_start, L.work, L.box_tile);
+  const int rounds = class_rounds(nt);
+  hipLaunchKernelGGL(tile_class_k, dim3(grid1d(nt, rounds * kB)), dim3(kB), 0, s, L.tile_start, nt, dense_min,
+                     part_nodes, two, rounds, L.work, L.scan, L.dense, L.dense_s);
+  scan_exclusive(L.scan, nt, two ? 4 : 3, L.partial, s);
+  hipLaunchKernelGGL(tile_place_k, dim3(grid1d(nt, rounds * kB)), dim3(kB), 0, s, L.tile_start, nt, dense_min,
+                     part_nodes, two, rounds, keys, (unsigned)T.tile_vol(), L.work, L.scan, L.items, L.items_s, L.order,
+                     L.tile_slot, L.ranges, L.oranges);
+  if (boxes && M > 0) {
+    if (T.ts[0] > 8 || T.ts[1] > 8 || T.ts[2] > 8) return kUnsupported;
+    hipLaunchKernelGGL(tile_box_k, dim3(grid1d(M, kB)), dim3(kB), 0, s, keys, M, T, L.box_tile);
+    hipLaunchKernelGGL(box_order_k, dim3(grid1d(L.order_cap, kB)), dim3(kB), 0, s, L.order, L.work, L.box_tile,
+                       L.box_ord);
+  }
+  unsigned w[kTileWork] = {0};
+  if (hipMemcpyAsync(w, L.work, sizeof(w), hipMemcpyDeviceToHost, s) != hipSuccess) return kHipError;
+  if (hipStreamSynchronize(s) != hipSuccess) return kHipError;
+  out->n_order = out->n_heavy = 0;
+  for (int k = 0; k < 32; k++) {
+    out->n_order += (int)w[k];
+    if (k <= 26) out->n_heavy += (int)w[k];
+  }
+  out->n_single = (int)w[31];
+  out->n_items = (int)w[64];
+  out->n_items_s = (int)w[65];
+  return kOk;
 }
 
 template <class R>
@@ -685,9 +730,9 @@ int fill_zero(Cplx<R>* p, size_t n, hipStream_t s) {
 }
 
 template int bin_nodes<float>(const float*, long, const GridGeom&, const TileLayout&, SortWork&, int*, unsigned*,
-                              int*, hipStream_t);
+                              hipStream_t);
 template int bin_nodes<double>(const double*, long, const GridGeom&, const TileLayout&, SortWork&, int*, unsigned*,
-                               int*, hipStream_t);
+                               hipStream_t);
 template int bin_nodes_noalloc<float>(const float*, long, const GridGeom&, const TileLayout&, int*, unsigned*,
                                       hipStream_t);
 template int bin_nodes_noalloc<double>(const double*, long, const GridGeom&, const TileLayout&, int*, unsigned*,

@@ -31,20 +31,20 @@ struct BArgs {
   const unsigned char* tile_dense;  // [ntiles] 1 if the tile's nodes go through the LDS path
   const int* items;        // work items: pairs (tile id, chunk index)
   int n_items;
-  // per work item (gather) or nonempty tile in the tile order (scatter): (tile,
-  // first position, first position past the lower half of axis 2, end)
+  // position ranges (tile, beg, mid, end) of the work items and of the order entries (TileLists)
   const int4* ranges;
+  const int4* oranges;
   int ts[3];               // tile size per axis
   int ntile[3];            // tiles per axis
   int all_dense;           // every nonempty tile is a work item: the direct kernel has no nodes to take
-  // nonempty tiles, most nodes first (column scatter and matrix-core gather)
+  // nonempty tiles, most nodes first (column scatter and matrix-core gather; see TileLists)
   const int* torder;       // [n_torder]
   int n_torder;
   int n_heavy;             // tiles torder[0, n_heavy) hold 32 nodes or more, the rest at most 31
   int n_single;            // the last n_single tiles of torder hold one node each
   // column scatter (scatter_cols.hip): when slots is set, scatter() runs it instead of the LDS-atomic path
-  Cplx<R>* slots;          // [n_torder][P^3] padded subgrid of every nonempty tile
-  const int* tile_slot;    // [ntiles] slot of each tile, -1 if empty
+  Cplx<R>* slots;          // [n_torder][P^3] padded subgrid of every order entry
+  const int2* tile_slot;   // [ntiles] (first slot of each tile, -1 if empty; slots)
   // offsets of each tile's nodes at binning time, per axis (bits 8 t + l for
   // offset l on axis t), by tile id and by position in torder (or null)
   const unsigned* box_tile;
@@ -75,16 +75,6 @@ constexpr int kTileNodes = 512;    // nodes per work item
 // axis of a tile's padded subgrid.  Returns P, or 0 if the path does not apply.
 int cols_pad(int m, bool is_double, const int* ts);
 
-// Nonempty tiles: those of 32 nodes or more by decreasing node count
-// (power-of-two classes, most nodes first), then those of 2..31 nodes and then
-// those of one node, both in tile order; tile_slot[t] = position of tile t (-1
-// if empty).  work holds 65 unsigned, partial the scan partials of ntiles values.
-// Returns the number of nonempty tiles (host value; synchronizes s), or -1;
-// *n_heavy = the number of them with 32 nodes or more; the tiles of one node
-// come last, *n_single of them.  light holds 2 ntiles unsigned.
-int build_tile_order(const int* tile_start, long ntiles, unsigned* work, unsigned* light, unsigned* partial,
-                     int* order, int* tile_slot, int* n_heavy, int* n_single, hipStream_t s);
-
 // Launch of the column scatter for MODE (B_F, B_GRAD, B_FGRAD): column kernel
 // into the slots, fold of the slots into the grid (which it overwrites), then
 // the nodes the column kernel listed as outside their tile (bins older than
@@ -107,19 +97,6 @@ int scatter_mm64(const BArgs<double>& A, hipStream_t s);
 // Fold of the FP64 slots (tiles of 8^3 cells, m = 2..6) into the grid, which it overwrites.
 int fold_slots64(const BArgs<double>& A, hipStream_t s);
 
-// Work items of the tiled kernels: every tile with at least dense_min nodes is
-// cut into chunks of kTileNodes sorted nodes.  Writes tile_dense[ntiles],
-// items[2 * n_items] and returns n_items (host value; synchronizes s), or -1.
-int build_items(const int* tile_start, long ntiles, int dense_min, unsigned* chunks, unsigned* partial,
-                unsigned char* tile_dense, int* items, long items_cap, hipStream_t s);
-
-// Position ranges for the FP64 matrix-core kernels: ranges[i] = (tile, beg, mid,
-// end), where the nodes [beg, mid) start in the lower half of the tile's cells
-// along axis 2 and [mid, end) in the upper half (the bin order puts them in this
-// order), of item i (chunked: pairs (tile, chunk) of items) or of tile items[i].
-int build_ranges(const int* items, int n_items, bool chunked, const int* tile_start, const unsigned* keys, unsigned tile_vol,
-                 int4* ranges, hipStream_t s);
-
 // Tile layout used by the binning: a node belongs to the tile that holds its
 // stencil start (floor(n x) - m) mod n on every axis.
 struct TileLayout {
@@ -129,33 +106,62 @@ struct TileLayout {
   long tile_vol() const { return (long)ts[0] * ts[1] * ts[2]; }
 };
 
-// Per-tile offset masks of the nodes whose sorted bin keys are keys[0, M)
-// (tile layout T, tile sizes of at most 8): box_tile[ntiles] by tile id and
-// box_ord[n_order] by position in order.  The slots of the matrix-core column
-// scatter (with the brick fold) hold only the box these masks span (from the
-// smallest offset to the largest plus 2m per axis); a node whose stencil
-// leaves that box (moved since binning) takes the stale path.  Returns kOk,
-// kUnsupported for larger tiles, or kHipError.
-int build_tile_boxes(const unsigned* keys, long M, const TileLayout& T, const int* order, int n_order,
-                     unsigned* box_tile, unsigned* box_ord, hipStream_t s);
+// Per-tile lists made from the sorted keys (device arrays of ntiles entries
+// unless said otherwise):
+//  * tile_start [ntiles + 1]: first sorted position of every tile;
+//  * dense, items: tiles of at least dense_min nodes, cut into work items (tile,
+//    chunk) of kTileNodes nodes in tile order; dense_s, items_s: every nonempty
+//    tile (the same list, and items_s unused, for dense_min = 1);
+//  * order: nonempty tiles, those of 32 nodes or more by decreasing node count
+//    (power-of-two classes), then those of 2..31 nodes and those of one node, both
+//    in tile order; a tile of more than part_nodes nodes has an entry per
+//    part_nodes nodes; tile_slot = (first entry, -1: empty tile; entries);
+//  * ranges, oranges (or null): position ranges (tile, beg, mid, end) of the items
+//    and of the order entries; the nodes [beg, mid) start in the lower half of the
+//    tile's cells along axis 2, [mid, end) in the upper half;
+//  * box_tile, box_ord: offset masks of the tile's nodes per axis, by tile and by
+//    order entry (with `boxes`).  The slots of the matrix-core column scatter (with
+//    the brick fold) hold only the box these masks span (from the smallest offset to
+//    the largest plus 2m per axis); a node whose stencil leaves that box (moved
+//    since binning) takes the stale path.
+constexpr int kTileWork = 66;  // counters: entries per class (32), placed (32), items, items_s
+struct TileLists {
+  int* tile_start;
+  unsigned* scan;     // [4 ntiles]
+  unsigned* partial;  // [4 (ntiles / 4096 + 1)]
+  unsigned* work;     // [kTileWork]
+  unsigned char *dense, *dense_s;
+  int *items, *items_s;
+  int* order;
+  int2* tile_slot;
+  int4 *ranges, *oranges;
+  unsigned *box_tile, *box_ord;
+  long order_cap;     // entries order, oranges and box_ord hold
+};
+struct TileCounts {
+  int n_items, n_items_s, n_order;
+  int n_heavy;   // order entries of tiles of 32 nodes or more
+  int n_single;  // the last n_single entries: tiles of one node
+};
+// Returns kOk (synchronizes s), kUnsupported (boxes of tiles of more than 8 cells) or kHipError.
+int build_tile_lists(const unsigned* keys, long M, const TileLayout& T, int dense_min, int part_nodes, bool boxes,
+                     TileLists& L, TileCounts* out, hipStream_t s);
 
-// Sorting scratch (device): keys/values double-buffered, histograms, scan partials.
+// Sorting scratch (device): keys/values double-buffered, per-block digit counts, digit totals.
 struct SortWork {
   unsigned* keys[2] = {nullptr, nullptr};
   int* vals[2] = {nullptr, nullptr};
-  unsigned* hist = nullptr;      // 256 * nblocks
-  unsigned* partial = nullptr;   // scan partials
-  long cap = 0;                  // capacity in nodes
-  long hist_cap = 0;
-  long partial_cap = 0;
+  unsigned* hist = nullptr;      // [sort_hist_words(M)]
+  unsigned* total = nullptr;     // [256]
 };
+long sort_hist_words(long M);
 
 // Compute bin keys of every node and sort the node ids by key (stable LSD
-// radix sort, 8-bit digits).  Result: perm (sorted node ids, == vals[res]),
-// sorted keys, and tile_start[ntiles+1].  Returns kOk or an error code.
+// radix sort, 8-bit digits): perm_out (sorted node ids) and keys_out (sorted
+// keys).  Returns kOk or an error code.
 template <class R>
 int bin_nodes(const R* x, long M, const GridGeom& g, const TileLayout& T, SortWork& W, int* perm_out,
-              unsigned* keys_out, int* tile_start, hipStream_t s);
+              unsigned* keys_out, hipStream_t s);
 
 // Kernel launchers, one object file per (R, KIND, MODE); KIND 0 = gather, 1 = scatter.
 template <class R, int KIND, int MODE>

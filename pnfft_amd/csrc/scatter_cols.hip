@@ -21,7 +21,7 @@
 // window does not reach are skipped by a uniform branch).
 // Each thread then writes its column to the tile's slot, and the fold kernel
 // sums, for every grid cell, the slots of the tiles whose subgrids cover it in
-// a fixed order and writes the cell.  Accumulation and fold use no atomics, so
+// a fixed order (a tile of very many nodes has several) and writes the cell.  Accumulation and fold use no atomics, so
 // the adjoint is deterministic; only nodes whose bins are older than their
 // coordinates (listed by the column kernel) go through the direct path
 // (global atomics) afterwards.
@@ -134,13 +134,14 @@ __global__ __launch_bounds__((ColsShape<R, MT, MODE>::NT)) void scatter_cols_k(B
   __shared__ R s_py[NB][CM], s_pz[NB][CM];
   __shared__ R s_dy[WG ? NB : 1][CM], s_dz[WG ? NB : 1][CM];
 
-  const int tile = A.torder[blockIdx.x];
+  const int4 range = A.oranges[blockIdx.x];
+  const int tile = range.x;
   const int t2 = tile % A.ntile[2];
   const int t1 = (tile / A.ntile[2]) % A.ntile[1];
   const int t0 = tile / (A.ntile[2] * A.ntile[1]);
   const int o0 = t0 * TS, o1 = t1 * TS, o2 = t2 * TS;
   const int n0 = A.g.n[0], n1 = A.g.n[1], n2 = A.g.n[2];
-  const int beg = A.tile_start[tile], end = A.tile_start[tile + 1];
+  const int beg = range.y, end = range.w;
   const int tid = threadIdx.x;
   const int b = tid / P, c = tid % P;  // rows b (and b + H when NC = 2) of column c
   const bool own = tid < S::NCOL;
@@ -293,13 +294,14 @@ __global__ __launch_bounds__(256, (MfmaShape<MODE>::WAVES + (MODE == B_F && MT <
   __shared__ unsigned s_pm[NBUF];                  // planes the batch's stencils reach (bit a)
   static_assert(RS % 4 == 0, "row buffers of whole 16-byte chunks");
 
-  const int tile = A.torder[blockIdx.x];
+  const int4 range = A.oranges[blockIdx.x];
+  const int tile = range.x;
   const int t2 = tile % A.ntile[2];
   const int t1 = (tile / A.ntile[2]) % A.ntile[1];
   const int t0 = tile / (A.ntile[2] * A.ntile[1]);
   const int o0 = t0 * TS, o1 = t1 * TS, o2 = t2 * TS;
   const int n0 = A.g.n[0], n1 = A.g.n[1], n2 = A.g.n[2];
-  const int beg = A.tile_start[tile], end = A.tile_start[tile + 1];
+  const int beg = range.y, end = range.w;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, lk = lane >> 4;
   // rows phase: thread (role, q) handles node q of the batch; roles 0..2 the
@@ -523,14 +525,14 @@ __global__ __launch_bounds__(TS* TS* TS) void fold_k(BArgs<R> A) {
 #pragma unroll
       for (int d2 = 0; d2 < D; d2++) {
         const int s2 = (T2 - d2 % nt2 + nt2) % nt2;
-        const int slot = A.tile_slot[((long)s0 * nt1 + s1) * nt2 + s2];
-        if (slot < 0) continue;
+        const int2 ts = A.tile_slot[((long)s0 * nt1 + s1) * nt2 + s2];
         const int p0 = q0 + d0 * TS, p1 = q1 + d1 * TS, p2 = q2 + d2 * TS;
-        if (p0 < P && p1 < P && p2 < P) {
-          const Cplx<R> v = A.slots[(size_t)slot * VOL + ((size_t)p0 * P + p1) * P + p2];
-          sr += (double)v.x;
-          si += (double)v.y;
-        }
+        if (p0 < P && p1 < P && p2 < P)
+          for (int slot = ts.x; slot < ts.x + ts.y; slot++) {
+            const Cplx<R> v = A.slots[(size_t)slot * VOL + ((size_t)p0 * P + p1) * P + p2];
+            sr += (double)v.x;
+            si += (double)v.y;
+          }
       }
     }
   }
@@ -565,35 +567,36 @@ __global__ __launch_bounds__(128) void fold8_k(BArgs<R> A) {
 #pragma unroll
       for (int d2 = 0; d2 < D; d2++) {
         const int s2 = (T2 - d2 % nt2 + nt2) % nt2;
-        const int slot = A.tile_slot[((long)s0 * nt1 + s1) * nt2 + s2];
-        if (slot < 0) continue;
+        const int2 ts = A.tile_slot[((long)s0 * nt1 + s1) * nt2 + s2];
         const int p0 = q0 + d0 * TS, p1 = q1 + d1 * TS, p2 = q2 + d2 * TS;
         if (p0 >= P || p1 >= P) continue;
-        const Cplx<R>* src = A.slots + (size_t)slot * VOL + ((size_t)p0 * P + p1) * P + p2;
-        if (p2 + 3 < P) {
-          Cplx<R> v[4];
-          if constexpr (sizeof(R) == 4) {  // two aligned 16-byte loads (p2 is a multiple of 4)
-            const float4 a = reinterpret_cast<const float4*>(src)[0], b = reinterpret_cast<const float4*>(src)[1];
-            v[0] = cmk<R>(a.x, a.y);
-            v[1] = cmk<R>(a.z, a.w);
-            v[2] = cmk<R>(b.x, b.y);
-            v[3] = cmk<R>(b.z, b.w);
+        for (int slot = ts.x; slot < ts.x + ts.y; slot++) {
+          const Cplx<R>* src = A.slots + (size_t)slot * VOL + ((size_t)p0 * P + p1) * P + p2;
+          if (p2 + 3 < P) {
+            Cplx<R> v[4];
+            if constexpr (sizeof(R) == 4) {  // two aligned 16-byte loads (p2 is a multiple of 4)
+              const float4 a = reinterpret_cast<const float4*>(src)[0], b = reinterpret_cast<const float4*>(src)[1];
+              v[0] = cmk<R>(a.x, a.y);
+              v[1] = cmk<R>(a.z, a.w);
+              v[2] = cmk<R>(b.x, b.y);
+              v[3] = cmk<R>(b.z, b.w);
+            } else {
+#pragma unroll
+              for (int k = 0; k < 4; k++) v[k] = src[k];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+              sr[k] += (double)v[k].x;
+              si[k] += (double)v[k].y;
+            }
           } else {
 #pragma unroll
-            for (int k = 0; k < 4; k++) v[k] = src[k];
-          }
-#pragma unroll
-          for (int k = 0; k < 4; k++) {
-            sr[k] += (double)v[k].x;
-            si[k] += (double)v[k].y;
-          }
-        } else {
-#pragma unroll
-          for (int k = 0; k < 4; k++) {
-            if (p2 + k < P) {
-              const Cplx<R> v = src[k];
-              sr[k] += (double)v.x;
-              si[k] += (double)v.y;
+            for (int k = 0; k < 4; k++) {
+              if (p2 + k < P) {
+                const Cplx<R> v = src[k];
+                sr[k] += (double)v.x;
+                si[k] += (double)v.y;
+              }
             }
           }
         }
@@ -656,10 +659,9 @@ __global__ __launch_bounds__(256) void fold8b_k(BArgs<R> A) {
       for (int j = 0; j < 3; j++) {
         const int s2 = ((T2 - 1 + j) % nt2 + nt2) % nt2;
         const long tix = ((long)s0 * nt1 + s1) * nt2 + s2;
-        const int slot = A.tile_slot[tix];
-        if (slot < 0) continue;
+        const int2 ts = A.tile_slot[tix];
         const int p2 = c + 8 - 8 * j;
-        if (row_ok && p2 >= 0 && p2 < P) {
+        if (ts.y > 0 && row_ok && p2 >= 0 && p2 < P) {
           // box slots: only the cells of the slot's box were written; zq marks
           // which of the four cells lie in it
           unsigned zq = 0xFu;
@@ -669,29 +671,31 @@ __global__ __launch_bounds__(256) void fold8b_k(BArgs<R> A) {
             zq = (cells((bmb >> 16) & 0xFFu) >> p2) & 0xFu;
             if (!zq) continue;
           }
-          const Cplx<R>* src = A.slots + (size_t)slot * VOL + ((size_t)p0 * P + p1) * P + p2;
-          if constexpr (sizeof(R) == 4) {  // two aligned 16-byte loads (P and p2 multiples of 4)
-            float4 a = reinterpret_cast<const float4*>(src)[0], b = reinterpret_cast<const float4*>(src)[1];
-            if (zq != 0xFu) {
-              if (!(zq & 1u)) a.x = a.y = 0.f;
-              if (!(zq & 2u)) a.z = a.w = 0.f;
-              if (!(zq & 4u)) b.x = b.y = 0.f;
-              if (!(zq & 8u)) b.z = b.w = 0.f;
-            }
-            sr[0] += (double)a.x;
-            si[0] += (double)a.y;
-            sr[1] += (double)a.z;
-            si[1] += (double)a.w;
-            sr[2] += (double)b.x;
-            si[2] += (double)b.y;
-            sr[3] += (double)b.z;
-            si[3] += (double)b.w;
-          } else {
+          for (int slot = ts.x; slot < ts.x + ts.y; slot++) {
+            const Cplx<R>* src = A.slots + (size_t)slot * VOL + ((size_t)p0 * P + p1) * P + p2;
+            if constexpr (sizeof(R) == 4) {  // two aligned 16-byte loads (P and p2 multiples of 4)
+              float4 a = reinterpret_cast<const float4*>(src)[0], b = reinterpret_cast<const float4*>(src)[1];
+              if (zq != 0xFu) {
+                if (!(zq & 1u)) a.x = a.y = 0.f;
+                if (!(zq & 2u)) a.z = a.w = 0.f;
+                if (!(zq & 4u)) b.x = b.y = 0.f;
+                if (!(zq & 8u)) b.z = b.w = 0.f;
+              }
+              sr[0] += (double)a.x;
+              si[0] += (double)a.y;
+              sr[1] += (double)a.z;
+              si[1] += (double)a.w;
+              sr[2] += (double)b.x;
+              si[2] += (double)b.y;
+              sr[3] += (double)b.z;
+              si[3] += (double)b.w;
+            } else {
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-              if (!((zq >> k) & 1u)) continue;
-              sr[k] += (double)src[k].x;
-              si[k] += (double)src[k].y;
+              for (int k = 0; k < 4; k++) {
+                if (!((zq >> k) & 1u)) continue;
+                sr[k] += (double)src[k].x;
+                si[k] += (double)src[k].y;
+              }
             }
           }
         }
@@ -750,10 +754,10 @@ __global__ __launch_bounds__(128) void fold4_k(BArgs<R> A) {
 #pragma unroll
       for (int j = 0; j < 7; j++) {
         const int s2 = ((T2 - 3 + j) % nt2 + nt2) % nt2;
-        const int slot = A.tile_slot[((long)s0 * nt1 + s1) * nt2 + s2];
-        if (slot < 0) continue;
+        const int2 ts = A.tile_slot[((long)s0 * nt1 + s1) * nt2 + s2];
         const int p2 = c + 12 - 4 * j;
-        if (row_ok && p2 >= 0 && p2 < P) {
+        if (!(row_ok && p2 >= 0 && p2 < P)) continue;
+        for (int slot = ts.x; slot < ts.x + ts.y; slot++) {
           const Cplx<R>* src = A.slots + (size_t)slot * VOL + ((size_t)p0 * P + p1) * P + p2;
           if constexpr (sizeof(R) == 4) {  // one aligned 16-byte load (P and p2 even)
             const float4 v = *reinterpret_cast<const float4*>(src);

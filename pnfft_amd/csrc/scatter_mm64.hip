@@ -97,7 +97,7 @@ __global__ __launch_bounds__((ScatterShape<MT, MODE>::NT), (ScatterShape<MT, MOD
   __shared__ unsigned s_km[NB / 4];                       // per four nodes: planes reached, bit 31: rows past 15
   __shared__ unsigned char s_bad[3][NB];
 
-  const int4 range = A.ranges[blockIdx.x];
+  const int4 range = A.oranges[blockIdx.x];
   const int tile = range.x, beg = range.y, end = range.w;
   const int mid = P > 16 ? range.z : end;
   const int t2 = tile % A.ntile[2];
@@ -370,7 +370,7 @@ int launch(const BArgs<double>& A, hipStream_t s) {
 
 template <int MODE>
 int scatter_mm64(const BArgs<double>& A, hipStream_t s) {
-  if (A.no_mfma || !A.pre_psi || !A.pre_x || (MODE != B_F && !A.pre_dpsi) || !A.ranges || !A.slots || !A.tile_slot ||
+  if (A.no_mfma || !A.pre_psi || !A.pre_x || (MODE != B_F && !A.pre_dpsi) || !A.oranges || !A.slots || !A.tile_slot ||
       A.n_torder <= 0 || !A.perm || !A.stale_count || !A.stale_list || A.ts[0] != 8 || A.ts[1] != 8 || A.ts[2] != 8)
     return kUnsupported;
   switch (A.g.m) {
