@@ -318,9 +318,9 @@ constexpr int kClassTiles = 8 * kB;
 // (one tile per thread for small grids, where eight in a row would be a chain)
 inline int class_rounds(long ntiles) { return ntiles > 65536 ? kClassTiles / kB : 1; }
 
-// Slots (order entries) of a tile: one, or one per part_nodes nodes.
-__device__ inline unsigned tile_parts(int cnt, int part_nodes) {
-  return cnt > part_nodes ? (unsigned)((cnt + part_nodes - 1) / part_nodes) : (cnt > 0 ? 1u : 0u);
+// Slots (order entries) of a tile: one for up to c.whole nodes, else one per c.part nodes.
+__device__ inline unsigned tile_parts(int cnt, TileCut c) {
+  return cnt > c.whole ? (unsigned)((cnt + c.part - 1) / c.part) : (cnt > 0 ? 1u : 0u);
 }
 
 // Per tile: order entries by node-count class (leading zeros of the count: more
@@ -328,7 +328,7 @@ __device__ inline unsigned tile_parts(int cnt, int part_nodes) {
 // the tile: flag of 2..31 nodes, flag of one node, work items of the gather (and
 // of the scatter, where they differ).
 __global__ __launch_bounds__(kB) void tile_class_k(const int* __restrict__ tile_start, long ntiles, int dense_min,
-                                                   int part_nodes, bool two_lists, int rounds, unsigned* work,
+                                                   TileCut cut, bool two_lists, int rounds, unsigned* work,
                                                    unsigned* scan, unsigned char* dense, unsigned char* dense_s) {
   __shared__ unsigned lc[32];
   if (threadIdx.x < 32) lc[threadIdx.x] = 0;
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(kB) void tile_class_k(const int* __restrict__ tile_
       scan[2 * ntiles + t] = d ? ch : 0u;
       if (two_lists) scan[3 * ntiles + t] = ch;
     }
-    const unsigned parts = tile_parts(cnt, part_nodes);
+    const unsigned parts = tile_parts(cnt, cut);
     (void)wave_class_add(cnt > 0, cnt > 0 ? __clz(cnt) : 0, lc);
     if (parts > 1) atomicAdd(&lc[__clz(cnt)], parts - 1);
   }
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(kB) void tile_class_k(const int* __restrict__ tile_
 // range from mid on start in the upper half of axis 2, by bisection of the keys,
 // whose in-tile index counts the runs of four cells along axis 2 outermost.
 __global__ __launch_bounds__(kB) void tile_place_k(const int* __restrict__ tile_start, long ntiles, int dense_min,
-                                                   int part_nodes, bool two_lists, int rounds,
+                                                   TileCut cut, bool two_lists, int rounds,
                                                    const unsigned* __restrict__ keys, unsigned vol, unsigned* work,
                                                    const unsigned* __restrict__ scan, int* items, int* items_s,
                                                    int* order, int2* tile_slot, int4* ranges, int4* oranges) {
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(kB) void tile_place_k(const int* __restrict__ tile_
     if (i >= rounds) break;
     const long t = ((long)blockIdx.x * rounds + i) * kB + threadIdx.x;
     const int cnt = t < ntiles ? tile_start[t + 1] - tile_start[t] : 0;
-    const unsigned parts = tile_parts(cnt, part_nodes);
+    const unsigned parts = tile_parts(cnt, cut);
     lpos[i] = wave_class_add(cnt >= 32 && parts == 1, cnt > 0 ? __clz(cnt) : 0, lc);
     if (cnt >= 32 && parts > 1) lpos[i] = atomicAdd(&lc[__clz(cnt)], parts);
   }
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(kB) void tile_place_k(const int* __restrict__ tile_
     const long t = ((long)blockIdx.x * rounds + i) * kB + threadIdx.x;
     if (i >= rounds || t >= ntiles) continue;
     const int beg = tile_start[t], end = tile_start[t + 1], cnt = end - beg;
-    const unsigned parts = tile_parts(cnt, part_nodes);
+    const unsigned parts = tile_parts(cnt, cut);
     unsigned p = 0;
     if (cnt > 0) {
       p = cnt >= 32 ? gb[__clz(cnt)] + lpos[i] : cnt > 1 ? light0 + scan[t] : single0 + scan[ntiles + t];
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(kB) void tile_place_k(const int* __restrict__ tile_
       for (unsigned k = 0; k < parts; k++) {
         order[p + k] = (int)t;
         if (oranges) {
-          const int b = beg + (int)k * part_nodes, e = parts > 1 ? min(end, b + part_nodes) : end;
+          const int b = beg + (int)k * cut.part, e = parts > 1 ? min(end, b + cut.part) : end;
           oranges[p + k] = make_int4((int)t, b, min(max(mid, b), e), e);
         }
       }
@@ -626,7 +626,7 @@ __global__ __launch_bounds__(kB) void box_order_k(const int* __restrict__ order,
   if (p < n) box_ord[p] = box_tile[order[p]];
 }
 
-int build_tile_lists(const unsigned* keys, long M, const TileLayout& T, int dense_min, int part_nodes, bool boxes,
+int build_tile_lists(const unsigned* keys, long M, const TileLayout& T, int dense_min, const TileCut& cut, bool boxes,
                      TileLists& L, TileCounts* out, hipStream_t s) {
   const long nt = T.ntiles();
   const bool two = dense_min > 1;
@@ -634,10 +634,10 @@ int build_tile_lists(const unsigned* keys, long M, const TileLayout& T, int dens
                      (unsigned)T.tile_vol(), nt, L.tile_start, L.work, L.box_tile);
   const int rounds = class_rounds(nt);
   hipLaunchKernelGGL(tile_class_k, dim3(grid1d(nt, rounds * kB)), dim3(kB), 0, s, L.tile_start, nt, dense_min,
-                     part_nodes, two, rounds, L.work, L.scan, L.dense, L.dense_s);
+                     cut, two, rounds, L.work, L.scan, L.dense, L.dense_s);
   scan_exclusive(L.scan, nt, two ? 4 : 3, L.partial, s);
   hipLaunchKernelGGL(tile_place_k, dim3(grid1d(nt, rounds * kB)), dim3(kB), 0, s, L.tile_start, nt, dense_min,
-                     part_nodes, two, rounds, keys, (unsigned)T.tile_vol(), L.work, L.scan, L.items, L.items_s, L.order,
+                     cut, two, rounds, keys, (unsigned)T.tile_vol(), L.work, L.scan, L.items, L.items_s, L.order,
                      L.tile_slot, L.ranges, L.oranges);
   if (boxes && M > 0) {
     if (T.ts[0] > 8 || T.ts[1] > 8 || T.ts[2] > 8) return kUnsupported;

@@ -114,8 +114,8 @@ struct TileLayout {
 //    tile (the same list, and items_s unused, for dense_min = 1);
 //  * order: nonempty tiles, those of 32 nodes or more by decreasing node count
 //    (power-of-two classes), then those of 2..31 nodes and those of one node, both
-//    in tile order; a tile of more than part_nodes nodes has an entry per
-//    part_nodes nodes; tile_slot = (first entry, -1: empty tile; entries);
+//    in tile order; a tile of more than cut.whole nodes has an entry per
+//    cut.part nodes; tile_slot = (first entry, -1: empty tile; entries);
 //  * ranges, oranges (or null): position ranges (tile, beg, mid, end) of the items
 //    and of the order entries; the nodes [beg, mid) start in the lower half of the
 //    tile's cells along axis 2, [mid, end) in the upper half;
@@ -138,13 +138,16 @@ struct TileLists {
   unsigned *box_tile, *box_ord;
   long order_cap;     // entries order, oranges and box_ord hold
 };
+struct TileCut {
+  int part, whole;
+};
 struct TileCounts {
   int n_items, n_items_s, n_order;
   int n_heavy;   // order entries of tiles of 32 nodes or more
   int n_single;  // the last n_single entries: tiles of one node
 };
 // Returns kOk (synchronizes s), kUnsupported (boxes of tiles of more than 8 cells) or kHipError.
-int build_tile_lists(const unsigned* keys, long M, const TileLayout& T, int dense_min, int part_nodes, bool boxes,
+int build_tile_lists(const unsigned* keys, long M, const TileLayout& T, int dense_min, const TileCut& cut, bool boxes,
                      TileLists& L, TileCounts* out, hipStream_t s);
 
 // Sorting scratch (device): keys/values double-buffered, per-block digit counts, digit totals.

@@ -125,3 +125,37 @@ def test_scatter_matches_oracle(gpu, oracle, kind, m, c2r):
             assert dp.api.last_error() is None
             assert rel(dp.f_hat.cpu().numpy(), ref) < TOL, (flags, tables)
     dp.close()
+
+
+@pytest.mark.parametrize("precision,tol", [("double", TOL), ("float", 1e-5)])
+@pytest.mark.parametrize("m", [4, 6, 8])
+def test_tile_of_several_slots(gpu, oracle, precision, tol, m):
+    """More nodes in one tile than a block takes: it is scattered into several slots and gathered by several
+    blocks (m = 8: tiles of 4 cells, the vector kernels); adj repeats bit for bit.  The oracle sums the
+    same terms; FP32 at 1e-5 as for the other FP32 comparisons with it."""
+    print("case several slots", precision, m, flush=True)
+    rng = SplitMix64(4000 + m)
+    N, n = (16, 16, 16), (32, 32, 32)
+    x = (rng.uniform(3 * 7001).reshape(7001, 3) * 3.9 + 4.05) / 32 - 0.25  # 7001 nodes in one tile ...
+    x = np.concatenate([x, rng.uniform(3 * 500).reshape(500, 3) - 0.5])     # ... and some everywhere
+    if precision == "float":
+        x = x.astype(np.float32).astype(np.float64)
+    M = len(x)
+    fh, fv = rng.complex_normal(16 ** 3), rng.complex_normal(M)
+    dp = DevicePlan(N, n, m, PA.PNFFT_WINDOW_GAUSSIAN, M, precision=precision)
+    dp.set_x(x)
+    dp.set_f_hat(fh)
+    dp.trafo(PA.PNFFT_COMPUTE_F)
+    f = dp.f.cpu().numpy().copy()
+    dp.set_f(fv)
+    out = []
+    for _ in range(2):
+        dp.adj(PA.PNFFT_COMPUTE_F)
+        out.append(dp.f_hat.cpu().numpy().copy())
+    assert dp.api.last_error() is None
+    dp.close()
+    P = oracle.Plan(N, n, m, PA.PNFFT_WINDOW_GAUSSIAN)
+    assert rel(f, P.trafo(x, fh)[0]) < tol
+    assert rel(out[0], P.adj(x, f=fv)) < tol
+    if precision == "float" or m <= 6:  # (FP64 m = 8 scatters by atomics)
+        assert np.array_equal(out[0], out[1])
