@@ -281,6 +281,7 @@ struct NodesT {
   unsigned* d_keys = nullptr;
   TileLists tl{};
   TileCounts tc{};
+  int item_nodes = 0;
   bool has_ranges = false, boxes = false;
   int n_torder = 0;        // order entries (0: the layout has no column scatter)
   Cplx<R>* d_slots = nullptr;
@@ -657,8 +658,15 @@ static T* stage_in(void* user, T*& mirror, size_t count, bool upload, hipStream_
 // folding.  Adjoint at M = 2^20 on n = 64^3: 2048 uniform nodes per tile FP64 386 us
 // whole, 469 us in two; eight clusters 5429 us whole, 566 us cut.  M = 3 10^5 in
 // 64 tiles: 300 us whole, 239 us cut.
-static TileCut tile_cut(long M) {
+template <class R>
+static TileCut tile_cut(long M, int m) {
   TileCut c;
+  // work items: 512 nodes fill the blocks of the vector kernels; the FP64 matrix-core
+  // gather (m >= 4) takes 256, fewer (128 at least) where M / 256 items would not
+  // fill the chip (n = 64^3 in 64 tiles, m = 6: M = 3 10^5 154 us with 512, 148 us
+  // with 256; M = 3 10^4 40 and 33 us with 192)
+  c.item = 512;
+  if (sizeof(R) == 8 && m >= 4 && m <= 6) c.item = (int)std::min(256L, std::max(128L, (M / 160 + 63) / 64 * 64));
   c.part = (int)std::max(1024L, (M / 1024 + 63) / 64 * 64);
   c.whole = (int)std::max((long)c.part, M / 455);
   return c;
@@ -666,9 +674,9 @@ static TileCut tile_cut(long M) {
 
 // Lays the binning arrays for M nodes in tiles T out in bin_mem, (re)allocated when too small.
 template <class R>
-static bool ensure_bin_memory(NodesT<R>* D, const TileLayout& T) {
+static bool ensure_bin_memory(NodesT<R>* D, const TileLayout& T, const TileCut& cut) {
   const size_t M = (size_t)D->M, nt = (size_t)T.ntiles();
-  const size_t items = nt + M / kTileNodes + 2, order = nt + M / (size_t)tile_cut(D->M).part + 2;
+  const size_t items = nt + 2 * (M / cut.item) + 2, order = nt + M / (size_t)cut.part + 2;
   for (int pass = 0; pass < 2; pass++) {
     size_t at = 0;
     auto take = [&](auto*& p, size_t count) {
@@ -753,7 +761,14 @@ static void set_tiles(BArgs<R>& A, const NodesT<R>* D, bool for_scatter = false)
   A.tile_dense = two ? D->tl.dense_s : D->tl.dense;
   A.items = two ? D->tl.items_s : D->tl.items;
   A.n_items = two ? D->tc.n_items_s : D->tc.n_items;
-  A.ranges = D->has_ranges ? D->tl.ranges : nullptr;
+  A.item_nodes = D->item_nodes;
+  // The FP64 matrix-core gather needs the items' ranges.  At m = 2 the stencil fills
+  // too little of its 16-row products everywhere (M = 2^20, 2048 nodes per tile: 94
+  // us on the vector kernel, 119 on the matrix cores), at m = 3 where the vector
+  // kernel's threads are busy (170 and 190 us; 92 nodes per tile 467 and 319 us).
+  const bool light = D->tc.n_items > 0 && D->M / D->tc.n_items < 200 && D->M >= 65536;
+  A.ranges = D->has_ranges && (for_scatter || D->bin_geom.m > 3 || (D->bin_geom.m == 3 && light)) ? D->tl.ranges
+                                                                                                 : nullptr;
   // the scatter's list holds every nonempty tile; the gather's when dense_min is 1
   A.all_dense = (for_scatter || dense_min() == 1) ? 1 : 0;
   A.no_mfma = mfma_disabled() ? 1 : 0;
@@ -805,7 +820,8 @@ static void ensure_slots(PlanT<R>* P, NodesT<R>* D) {
 template <class R>
 static int bin(PlanT<R>* P, NodesT<R>* D, const R* dx, const GridGeom& g) {
   D->bins_valid = false;
-  if (!ensure_bin_memory(D, P->tiles)) {
+  const TileCut cut = tile_cut<R>(D->M, P->m);
+  if (!ensure_bin_memory(D, P->tiles, cut)) {
     set_error("device allocation for node binning failed");
     return kHipError;
   }
@@ -822,7 +838,7 @@ static int bin(PlanT<R>* P, NodesT<R>* D, const R* dx, const GridGeom& g) {
   D->has_ranges = sizeof(R) == 8 && P->m <= 6 && P->tiles.ts[2] == 8;
   TileLists tl = D->tl;
   if (!D->has_ranges) tl.ranges = nullptr;
-  if (build_tile_lists(D->d_keys, D->M, P->tiles, dense_min(), tile_cut(D->M), D->boxes, tl, &D->tc, P->stream) !=
+  if (build_tile_lists(D->d_keys, D->M, P->tiles, dense_min(), cut, D->boxes, tl, &D->tc, P->stream) !=
       kOk) {
     set_error("building the tile lists failed");
     return kHipError;
@@ -830,6 +846,7 @@ static int bin(PlanT<R>* P, NodesT<R>* D, const R* dx, const GridGeom& g) {
   D->n_torder = pad > 0 && D->M > 0 ? D->tc.n_order : 0;
   D->bin_geom = g;
   D->bin_tiles = P->tiles;
+  D->item_nodes = cut.item;
   D->bins_valid = true;
   return kOk;
 }
@@ -886,7 +903,7 @@ static T* grow(T*& p, size_t& cap, size_t need) {
 // the arguments stay without tables and the vector kernels evaluate the windows.
 template <class R>
 static void call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s) {
-  if (sizeof(R) != 8 || A.no_mfma || A.g.m > 6 || D->M == 0 || (A.pre_psi && (A.pre_dpsi || !need_grad))) return;
+  if (sizeof(R) != 8 || A.no_mfma || !A.ranges || A.g.m > 6 || D->M == 0 || (A.pre_psi && (A.pre_dpsi || !need_grad))) return;
   const bool kept = A.pre_psi != nullptr;  // psi tables of precompute_psi: written again with equal values
   const size_t M = (size_t)D->M, cm = 2 * (size_t)A.g.m + 1;
   R* psi = grow(D->d_pre_psi, D->pre_psi_cap, 3 * cm * M);

@@ -9,7 +9,7 @@
 // stencil kernels of kernel/assign.c:478-1066 (cutoff 2m+1, :910).
 //
 // Two paths:
-//  * tiled: one block per work item (tile, chunk of <= kTileNodes sorted
+//  * tiled: one block per work item (tile, chunk of about item_nodes sorted
 //    nodes).  The tile's padded subgrid ((TS + 2m) cells per axis, starting at
 //    the tile origin because tiles are keyed by the stencil start) is staged in
 //    LDS; the gather reads every stencil point from LDS, the scatter
@@ -92,8 +92,9 @@ __device__ inline TileItem tile_item(const BArgs<R>& A, int m) {
   it.o[2] = t2 * A.ts[2];
   for (int d = 0; d < 3; d++) it.P[d] = A.ts[d] + 2 * m;
   const int s = A.tile_start[t], e = A.tile_start[t + 1];
-  it.beg = s + chunk * kTileNodes;
-  it.end = min(e, it.beg + kTileNodes);
+  const int len = item_len(e - s, A.item_nodes);
+  it.beg = min(e, s + chunk * len);
+  it.end = min(e, it.beg + len);
   return it;
 }
 

@@ -1,4 +1,4 @@
-// gather_mm64.hip -- FP64 gather (trafo B) on the matrix cores, m = 2..6.
+// gather_mm64.hip -- FP64 gather (trafo B) on the matrix cores, m = 3..6.
 //
 // This file is compiled once per mode; the build passes PNFFT_B_MODE (BMode).
 //
@@ -26,7 +26,9 @@
 // no room for a second; staging alone is 0.49 ms).  Windows always come from
 // tables: evaluating them here costs registers for 13 doubles per axis and
 // leaves two waves per SIMD instead of three, with spills in the product loops
-// (gradient modes at m = 5: 1.27 ms with, 0.90 ms without the evaluation).
+// (gradient modes at m = 5: 1.27 ms with, 0.90 ms without the evaluation).  Waves
+// in flight decide the rest: m = 4, M = 2^20, 2048 nodes per tile, f takes 323 us
+// with three waves per SIMD and 227 us with four.
 #include "mm64.hpp"
 
 namespace pnfft_amd {
@@ -35,6 +37,10 @@ namespace {
 
 using namespace bdev;
 using namespace mm64;
+
+// Items of at most kFew nodes are gathered from the grid, one wave per node:
+// staging a subgrid reads P^3 cells where kFew stencils read kFew (2m+1)^3.
+constexpr int kFew = 3;
 
 template <int MT, int MODE, bool RG>
 struct GatherShape {
@@ -48,17 +54,21 @@ struct GatherShape {
   static constexpr size_t SUB = (size_t)P * P * PITCH * (RG ? 8 : 16);
   static constexpr int AREA = 16 * CM * (WG ? 2 : 1);  // doubles: one axis' windows of a wave's 16 nodes
   static constexpr size_t lds(int nw) { return SUB + (size_t)nw * AREA * 8; }
-  // waves per CU: three per SIMD for f (168 VGPRs suffice), two for the gradient
-  // modes, in as many blocks as the LDS holds
-  static constexpr int WAVES = WG ? 2 : 3;
+  // waves per SIMD: four for f up to m = 4 (128 VGPRs suffice) and three above,
+  // two for the gradient modes, in as many blocks as the LDS holds
+  static constexpr int WAVES = WG ? 2 : (P <= 16 ? 4 : 3);
   static constexpr bool fits(int blocks) {
-    return 4 * WAVES % blocks == 0 && blocks * lds(4 * WAVES / blocks) <= kLdsPerCu;
+    return 4 * WAVES % blocks == 0 && 4 * WAVES / blocks >= 4 && blocks * lds(4 * WAVES / blocks) <= kLdsPerCu;
   }
-  static constexpr int BLOCKS = fits(3) ? 3 : (fits(2) ? 2 : 1);
+  static constexpr int BLOCKS = fits(4) ? 4 : (fits(3) ? 3 : (fits(2) ? 2 : 1));
   static constexpr int NW = 4 * WAVES / BLOCKS;
+  // the next group's window loads are in flight during the products, except where
+  // their 4 CM registers would spill (gradient modes on complex grids at m = 5, 6)
+  static constexpr bool AHEAD = !WG || MT <= 4 || RG;
   static constexpr int NT = 64 * NW;
   static constexpr size_t LDS = lds(NW);
   static_assert(LDS <= kLdsPerCu, "subgrid and window rows fit the LDS");
+  static_assert(NW >= kFew, "a wave for each of few nodes");
 };
 
 // Position of cell c in LDS row b.  A wave's operand read takes one cell per
@@ -110,10 +120,6 @@ template <int N>
 struct IntC {
   static constexpr int value = N;
 };
-
-// Items of at most kFew nodes are gathered from the grid, one wave per node:
-// staging a subgrid reads P^3 cells where kFew stencils read kFew (2m+1)^3.
-constexpr int kFew = 3;
 
 template <int MT, int MODE, bool RG>
 __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, MODE, RG>::WAVES)) void gather_mm64_k(BArgs<double> A) {
@@ -394,8 +400,8 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
     }
     put(0);
 
-    // loads for the wave's next group, in flight during the matrix-core phase
-    if (it + 1 < nit) {
+    // loads for the wave's next group
+    if (S::AHEAD && it + 1 < nit) {
       load_group(it + 1, jn, L);
       jn = A.perm[pos_at(it + 2)];
     }
@@ -590,6 +596,10 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
         A.stale_list[atomicAdd(A.stale_count, 1u)] = pos;  // gathered by gather_stale64_k
       }
     }
+    if (!S::AHEAD && it + 1 < nit) {
+      load_group(it + 1, jn, L);
+      jn = A.perm[pos_at(it + 2)];
+    }
   }
 }
 
@@ -639,7 +649,6 @@ int gather_mm64(const BArgs<double>& A, hipStream_t s) {
       A.ts[0] != 8 || A.ts[1] != 8 || A.ts[2] != 8)
     return kUnsupported;
   switch (A.g.m) {
-    case 2: launch<2, MODE>(A, s); break;
     case 3: launch<3, MODE>(A, s); break;
     case 4: launch<4, MODE>(A, s); break;
     case 5: launch<5, MODE>(A, s); break;

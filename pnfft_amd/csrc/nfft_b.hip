@@ -338,7 +338,7 @@ __global__ __launch_bounds__(kB) void tile_class_k(const int* __restrict__ tile_
     const int cnt = t < ntiles ? tile_start[t + 1] - tile_start[t] : 0;
     if (t < ntiles) {
       const bool d = cnt >= dense_min && cnt > 0;
-      const unsigned ch = (unsigned)((cnt + kTileNodes - 1) / kTileNodes);
+      const unsigned ch = (unsigned)tile_items(cnt, cut.item);
       dense[t] = d ? 1 : 0;
       dense_s[t] = cnt > 0 ? 1 : 0;
       scan[t] = (cnt > 1 && cnt < 32) ? 1u : 0u;
@@ -420,13 +420,13 @@ __global__ __launch_bounds__(kB) void tile_place_k(const int* __restrict__ tile_
           oranges[p + k] = make_int4((int)t, b, min(max(mid, b), e), e);
         }
       }
-      const unsigned o = scan[2 * ntiles + t], ch = (unsigned)((cnt + kTileNodes - 1) / kTileNodes);
+      const unsigned o = scan[2 * ntiles + t], ch = (unsigned)tile_items(cnt, cut.item);
       for (unsigned k = 0; k < ch; k++) {
         if (cnt >= dense_min) {
           items[2 * (o + k)] = (int)t;
           items[2 * (o + k) + 1] = (int)k;
           if (ranges) {
-            const int b = beg + (int)k * kTileNodes, e = min(end, b + kTileNodes);
+            const int len = item_len(cnt, cut.item), b = min(end, beg + (int)k * len), e = min(end, b + len);
             ranges[o + k] = make_int4((int)t, b, min(max(mid, b), e), e);
           }
         }
@@ -439,7 +439,7 @@ __global__ __launch_bounds__(kB) void tile_place_k(const int* __restrict__ tile_
     }
     tile_slot[t] = cnt > 0 ? make_int2((int)p, (int)parts) : make_int2(-1, 0);
     if (t == ntiles - 1) {
-      const unsigned ch = (unsigned)((cnt + kTileNodes - 1) / kTileNodes);
+      const unsigned ch = (unsigned)tile_items(cnt, cut.item);
       work[64] = scan[2 * ntiles + t] + (cnt >= dense_min ? ch : 0u);
       work[65] = two_lists ? scan[3 * ntiles + t] + ch : work[64];
     }

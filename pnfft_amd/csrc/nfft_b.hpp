@@ -31,6 +31,7 @@ struct BArgs {
   const unsigned char* tile_dense;  // [ntiles] 1 if the tile's nodes go through the LDS path
   const int* items;        // work items: pairs (tile id, chunk index)
   int n_items;
+  int item_nodes;          // about this many nodes per work item (item_len)
   // position ranges (tile, beg, mid, end) of the work items and of the order entries (TileLists)
   const int4* ranges;
   const int4* oranges;
@@ -68,7 +69,6 @@ struct BArgs {
 constexpr int std_tile(int m, bool is_double) { return (m <= 4 || (m <= 6 && is_double)) ? 8 : 4; }
 
 constexpr int kTileThreads = 512;  // threads per block of the tiled kernels
-constexpr int kTileNodes = 512;    // nodes per work item
 
 // Column scatter: applies for m = 2..8 (FP64: m <= 6) when all three tile
 // sizes equal the layout's TS (std_tile); P = TS + 2m cells per
@@ -83,7 +83,7 @@ template <class R, int MODE>
 int cols_launch(const BArgs<R>& A, hipStream_t s);
 
 // FP64 gather on the matrix cores (gather_mm64.hip) for MODE (B_F, B_GRAD,
-// B_FGRAD, B_VJP): m = 2..6 on tiles of 8^3 cells with the work items of every
+// B_FGRAD, B_VJP): m = 3..6 on tiles of 8^3 cells with the work items of every
 // nonempty tile; kUnsupported (nothing launched) otherwise.
 template <int MODE>
 int gather_mm64(const BArgs<double>& A, hipStream_t s);
@@ -110,7 +110,7 @@ struct TileLayout {
 // unless said otherwise):
 //  * tile_start [ntiles + 1]: first sorted position of every tile;
 //  * dense, items: tiles of at least dense_min nodes, cut into work items (tile,
-//    chunk) of kTileNodes nodes in tile order; dense_s, items_s: every nonempty
+//    chunk) of about cut.item nodes (item_len) in tile order; dense_s, items_s: every nonempty
 //    tile (the same list, and items_s unused, for dense_min = 1);
 //  * order: nonempty tiles, those of 32 nodes or more by decreasing node count
 //    (power-of-two classes), then those of 2..31 nodes and those of one node, both
@@ -139,7 +139,8 @@ struct TileLists {
   long order_cap;     // entries order, oranges and box_ord hold
 };
 struct TileCut {
-  int part, whole;
+  int part, whole;  // order entries of a tile of more than `whole` nodes hold `part` nodes each
+  int item;         // about this many nodes per work item
 };
 struct TileCounts {
   int n_items, n_items_s, n_order;
