@@ -312,7 +312,7 @@ __global__ __launch_bounds__(kTileThreads) void scatter_tiled_k(BArgs<R> A) {
 
 // ---------------------------------------------------------------------------
 // Matrix-core gather (FP32 plans, P = TS + 2m <= 16: tiles of 8 cells for
-// m <= 4, of 4 cells for m = 5, 6; f, grad, f + grad).  For a plane a of the tile's padded subgrid and a group of 16
+// m <= 4, of 4 cells for m = 5, 6; f, grad, f + grad, VJP).  For a plane a of the tile's padded subgrid and a group of 16
 // nodes,
 //   T_a[b][j] = sum_c G[a][b][c] Z_j[c]      (Z_j = psi_z of node j, zero-padded)
 // is a 16 x 16 x 16 product: four v_mfma_f32_16x16x4f32 (K = 4 values of c
@@ -381,7 +381,7 @@ template <int MT, int MODE, int NW = 4>
 struct GatherMfmaShape {
   static constexpr int CM = 2 * MT + 1, TS = std_tile(MT, false), P = TS + 2 * MT;
   static constexpr bool WF = (MODE == B_F || MODE == B_FGRAD);
-  static constexpr bool WG = (MODE == B_GRAD || MODE == B_FGRAD);
+  static constexpr bool WG = (MODE == B_GRAD || MODE == B_FGRAD || MODE == B_VJP);
   // window rows of a wave's 16 nodes: x and z rows of 17 floats (read as
   // scalars), y rows of 20 floats (read as float4 chunks), at X 0, Y YOFF,
   // Z ZOFF; the derivative rows follow at ROWSZ / 2.  The odd and the 20-float
@@ -751,7 +751,7 @@ __global__ void zero_u32_k(unsigned* c) {
 template <int MT, int MODE>
 __global__ __launch_bounds__(256) void gather_stale_k(BArgs<float> A) {
   constexpr int CM = 2 * MT + 1;
-  constexpr bool WG = (MODE == B_GRAD || MODE == B_FGRAD);
+  constexpr bool WG = (MODE == B_GRAD || MODE == B_FGRAD || MODE == B_VJP);
   const unsigned count = *A.stale_count;
   for (unsigned k = blockIdx.x * 256 + threadIdx.x; k < count; k += gridDim.x * 256) {
     const long j = A.perm[A.stale_list[k]];
@@ -769,7 +769,7 @@ __global__ __launch_bounds__(256) void gather_stale_k(BArgs<float> A) {
 template <int MT, int MODE>
 __global__ __launch_bounds__(256) void gather_single_k(BArgs<float> A, int first) {
   constexpr int CM = 2 * MT + 1, NR = CM * CM;
-  constexpr bool WG = (MODE == B_GRAD || MODE == B_FGRAD);
+  constexpr bool WG = (MODE == B_GRAD || MODE == B_FGRAD || MODE == B_VJP);
   const int lane = threadIdx.x & 63;
   const int p = first + blockIdx.x * 4 + (threadIdx.x >> 6);
   if (p >= A.n_torder) return;  // whole wave; no barrier follows
@@ -858,12 +858,12 @@ __global__ __launch_bounds__(256) void gather_single_k(BArgs<float> A, int first
 
 inline unsigned grid1d(long n, int t) { return (unsigned)((n + t - 1) / t); }
 
-// the matrix-core gather applies to FP32 f / grad / f + grad with m <= 6 on the
+// the matrix-core gather applies to FP32 (f, grad, f + grad, VJP) with m <= 6 on the
 // standard tile layout (padded subgrids of at most 16 cells per axis), once the
 // nonempty tiles are listed
 template <class R, int MT, int MODE>
 bool mfma_gather(const BArgs<R>& A) {
-  if constexpr (sizeof(R) != 4 || MT > 6 || MODE > B_FGRAD) {
+  if constexpr (sizeof(R) != 4 || MT > 6) {
     return false;
   } else {
     constexpr int TS = GatherMfmaShape<MT, MODE, 4>::TS;
@@ -874,7 +874,7 @@ bool mfma_gather(const BArgs<R>& A) {
 
 template <class R, int MT, int MODE>
 void launch_gather_mfma(const BArgs<R>& A, hipStream_t s) {
-  if constexpr (sizeof(R) == 4 && MT <= 6 && MODE <= B_FGRAD) {
+  if constexpr (sizeof(R) == 4 && MT <= 6) {
     using S4 = GatherMfmaShape<MT, MODE, 4>;
     using S2 = GatherMfmaShape<MT, MODE, 2>;
     const int nh = min(max(A.n_heavy, 0), A.n_torder);
