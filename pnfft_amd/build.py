@@ -32,9 +32,13 @@ COLS_VARIANTS = [
     for r in ("f32", "f64")
     for mi, m in ((1, "f"), (2, "grad"), (3, "fgrad"))
 ]
-# gather_mm64.hip and scatter_mm64.hip (FP64) are compiled once per mode
-MM64_VARIANTS = [(m, [f"-DPNFFT_B_MODE={mi}"]) for mi, m in ((1, "f"), (2, "grad"), (3, "fgrad"), (4, "vjp"))]
-SM64_VARIANTS = MM64_VARIANTS[:3]
+# gather_mm.hip is compiled once per (precision, mode), scatter_mm64.hip (FP64) once per mode
+MM_VARIANTS = [
+    (f"{r}_{m}", [f"-DPNFFT_B_REAL={'float' if r == 'f32' else 'double'}", f"-DPNFFT_B_MODE={mi}"])
+    for r in ("f32", "f64")
+    for mi, m in ((1, "f"), (2, "grad"), (3, "fgrad"), (4, "vjp"))
+]
+SM64_VARIANTS = [(m, [f"-DPNFFT_B_MODE={mi}"]) for mi, m in ((1, "f"), (2, "grad"), (3, "fgrad"))]
 # pre_psi.hip, hessian.hip and window_tab.hip are compiled once per precision
 PRE_VARIANTS = [(r, [f"-DPNFFT_B_REAL={'float' if r == 'f32' else 'double'}"]) for r in ("f32", "f64")]
 ARCH = os.environ.get("PNFFT_AMD_ARCH", "gfx950")
@@ -70,7 +74,7 @@ def build(verbose=True, force=True):
     os.makedirs(BUILD, exist_ok=True)
     jobs = ([("b_kernels.hip", "_" + sfx, d) for sfx, d in B_VARIANTS] +
             [("scatter_cols.hip", "_" + sfx, d) for sfx, d in COLS_VARIANTS] +
-            [("gather_mm64.hip", "_" + sfx, d) for sfx, d in MM64_VARIANTS] +
+            [("gather_mm.hip", "_" + sfx, d) for sfx, d in MM_VARIANTS] +
             [("scatter_mm64.hip", "_" + sfx, d) for sfx, d in SM64_VARIANTS] +
             [("pre_psi.hip", "_" + sfx, d) for sfx, d in PRE_VARIANTS] +
             [("hessian.hip", "_" + sfx, d) for sfx, d in PRE_VARIANTS] +

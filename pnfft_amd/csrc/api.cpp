@@ -661,12 +661,12 @@ static T* stage_in(void* user, T*& mirror, size_t count, bool upload, hipStream_
 template <class R>
 static TileCut tile_cut(long M, int m) {
   TileCut c;
-  // work items: 512 nodes fill the blocks of the vector kernels; the FP64 matrix-core
-  // gather (m >= 4) takes 256, fewer (128 at least) where M / 256 items would not
+  // work items: 512 nodes fill the blocks of the vector kernels; the matrix-core gather
+  // with tables (FP64 m >= 4, FP32 m >= 7) takes 256, fewer (128 at least) where M / 256 items would not
   // fill the chip (n = 64^3 in 64 tiles, m = 6: M = 3 10^5 154 us with 512, 148 us
   // with 256; M = 3 10^4 40 and 33 us with 192)
   c.item = 512;
-  if (sizeof(R) == 8 && m >= 4 && m <= 6) c.item = (int)std::min(256L, std::max(128L, (M / 160 + 63) / 64 * 64));
+  if ((sizeof(R) == 8 && m >= 4 && m <= 6) || (sizeof(R) == 4 && m >= 7)) c.item = (int)std::min(256L, std::max(128L, (M / 160 + 63) / 64 * 64));
   c.part = (int)std::max(1024L, (M / 1024 + 63) / 64 * 64);
   c.whole = (int)std::max((long)c.part, M / 455);
   return c;
@@ -834,8 +834,8 @@ static int bin(PlanT<R>* P, NodesT<R>* D, const R* dx, const GridGeom& g) {
   // whose padded subgrids are a multiple of four cells wide (m = 2, 4)
   const int pad = cols_enabled() ? cols_pad(P->m, sizeof(R) == 8, P->tiles.ts) : 0;
   D->boxes = sizeof(R) == 4 && pad > 0 && P->tiles.ts[0] == 8 && pad <= 16 && pad % 4 == 0;
-  // ranges: FP64 matrix-core gather on tiles of 8 cells; its tile lists hold no fewer-node cut
-  D->has_ranges = sizeof(R) == 8 && P->m <= 6 && P->tiles.ts[2] == 8;
+  // ranges: the gather of gather_mm.hip on the standard tiles
+  D->has_ranges = (sizeof(R) == 8) == (P->m <= 6) && P->tiles.ts[2] == std_tile(P->m, sizeof(R) == 8);
   TileLists tl = D->tl;
   if (!D->has_ranges) tl.ranges = nullptr;
   if (build_tile_lists(D->d_keys, D->M, P->tiles, dense_min(), cut, D->boxes, tl, &D->tc, P->stream) !=
@@ -896,14 +896,15 @@ static T* grow(T*& p, size_t& cap, size_t need) {
   return p;
 }
 
-// Window tables for the FP64 matrix-core kernels, which take every window from
-// tables (their own evaluation would hold them to half the waves): where
+// Window tables for the matrix-core kernels that take every window from tables
+// (FP64 at m = 2..6, FP32 at m = 7, 8; their own evaluation would hold them to half
+// the waves): where
 // precompute_psi made none for this call (or none of the derivatives), the
 // tables are computed into the node set's buffers now.  Without memory for them
 // the arguments stay without tables and the vector kernels evaluate the windows.
 template <class R>
 static void call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s) {
-  if (sizeof(R) != 8 || A.no_mfma || !A.ranges || A.g.m > 6 || D->M == 0 || (A.pre_psi && (A.pre_dpsi || !need_grad))) return;
+  if ((sizeof(R) == 8) != (A.g.m <= 6) || A.no_mfma || !A.ranges || D->M == 0 || (A.pre_psi && (A.pre_dpsi || !need_grad))) return;
   const bool kept = A.pre_psi != nullptr;  // psi tables of precompute_psi: written again with equal values
   const size_t M = (size_t)D->M, cm = 2 * (size_t)A.g.m + 1;
   R* psi = grow(D->d_pre_psi, D->pre_psi_cap, 3 * cm * M);

@@ -1,19 +1,21 @@
-// gather_mm64.hip -- FP64 gather (trafo B) on the matrix cores, m = 3..6.
+// gather_mm.hip -- gather (trafo B) on the matrix cores with windows from tables:
+// FP64 at m = 3..6 (tiles of 8 cells), FP32 at m = 7, 8 (tiles of 4).
 //
-// This file is compiled once per mode; the build passes PNFFT_B_MODE (BMode).
+// This file is compiled once per (precision, mode); the build passes PNFFT_B_REAL
+// (float|double) and PNFFT_B_MODE (BMode).
 //
 // Reference: the node loops of kernel/ndft-parallel.c:2703-3009 and the
 // stencil kernels of kernel/assign.c:642-1066 (cutoff 2m+1, :910).
 //
-// For a plane a of a tile's padded subgrid (P = 8 + 2m cells per axis) and a
+// For a plane a of a tile's padded subgrid (P = TS + 2m cells per axis) and a
 // group of 16 sorted nodes,
 //   T_a[b][j] = sum_c G[a][b][c] Z_j[c]      (Z_j = psi_z of node j, zero outside its stencil)
-// is a product of a 16 x 4 NK and a 4 NK x 16 matrix: v_mfma_f64_16x16x4f64 per
+// is a product of a 16 x 4 NK and a 4 NK x 16 matrix: a 16x16x4 MFMA per
 // K-block of four c, per real and imaginary part (and with psi'_z for the
 // gradient).  A lane (j = lane & 15, k = lane >> 4) then holds T_a[b][j] for the
-// rows b = k + 4 r and forms f_j = sum_a X_j[a] sum_b Y_j[b] T_a[b][j] on the
-// vector units.  Subgrids of 18 and 20 rows (m = 5, 6) have R = 2 or 4 rows past
-// the sixteenth; those of 16 / R planes make one more 16-row product.
+// rows b = acc_row(k, r) and forms f_j = sum_a X_j[a] sum_b Y_j[b] T_a[b][j] on the
+// vector units.  Subgrids of 18 and 20 rows have XR = 2 or 4 rows past the
+// sixteenth; those of 16 / XR planes make one more 16-row product.
 //
 // What it is bound by: at m = 6 on uniform nodes (N = 128^3, M = 2^22, 128 nodes
 // per tile) a launch takes 2.49 ms, against 8.53 ms of the vector kernel, whose
@@ -29,42 +31,42 @@
 // (gradient modes at m = 5: 1.27 ms with, 0.90 ms without the evaluation).  Waves
 // in flight decide the rest: m = 4, M = 2^20, 2048 nodes per tile, f takes 323 us
 // with three waves per SIMD and 227 us with four.
-#include "mm64.hpp"
+#include "mm.hpp"
 
 namespace pnfft_amd {
 
 namespace {
 
 using namespace bdev;
-using namespace mm64;
+using namespace mm;
 
 // Items of at most kFew nodes are gathered from the grid, one wave per node:
 // staging a subgrid reads P^3 cells where kFew stencils read kFew (2m+1)^3.
 constexpr int kFew = 3;
 
-template <int MT, int MODE, bool RG>
+template <class R, int MT, int MODE, bool RG>
 struct GatherShape {
-  static constexpr int CM = 2 * MT + 1, TS = 8, P = TS + 2 * MT;
+  static constexpr int CM = 2 * MT + 1, TS = std_tile(MT, sizeof(R) == 8), P = TS + 2 * MT;
   static constexpr int NK = (P + 3) / 4;        // K-blocks of a subgrid row
   static constexpr int PITCH = 4 * NK;          // cells per row in LDS (columns past P are zero)
-  static constexpr int R = P > 16 ? P - 16 : 0;  // rows past the sixteenth
-  static constexpr int PB = R ? 16 / R : 1;     // planes whose extra rows fill one product
+  static constexpr int XR = P > 16 ? P - 16 : 0;  // rows past the sixteenth
+  static constexpr int PB = XR ? 16 / XR : 1;     // planes whose extra rows fill one product
   static constexpr bool WF = (MODE == B_F || MODE == B_FGRAD);
   static constexpr bool WG = (MODE == B_GRAD || MODE == B_FGRAD || MODE == B_VJP);
-  static constexpr size_t SUB = (size_t)P * P * PITCH * (RG ? 8 : 16);
-  static constexpr int AREA = 16 * CM * (WG ? 2 : 1);  // doubles: one axis' windows of a wave's 16 nodes
-  static constexpr size_t lds(int nw) { return SUB + (size_t)nw * AREA * 8; }
-  // waves per SIMD: four for f up to m = 4 (128 VGPRs suffice) and three above,
-  // two for the gradient modes, in as many blocks as the LDS holds
-  static constexpr int WAVES = WG ? 2 : (P <= 16 ? 4 : 3);
+  static constexpr size_t SUB = (size_t)P * P * PITCH * sizeof(R) * (RG ? 1 : 2);
+  static constexpr int AREA = 16 * CM * (WG ? 2 : 1);  // reals: one axis' windows of a wave's 16 nodes
+  static constexpr size_t lds(int nw) { return SUB + (size_t)nw * AREA * sizeof(R); }
+  // waves per SIMD, in as many blocks as the LDS holds: FP64 four for f up to m = 4
+  // (128 VGPRs suffice) and three above, two for the gradient modes; FP32 three
+  static constexpr int WAVES = sizeof(R) == 4 ? 3 : (WG ? 2 : (P <= 16 ? 4 : 3));
   static constexpr bool fits(int blocks) {
     return 4 * WAVES % blocks == 0 && 4 * WAVES / blocks >= 4 && blocks * lds(4 * WAVES / blocks) <= kLdsPerCu;
   }
   static constexpr int BLOCKS = fits(4) ? 4 : (fits(3) ? 3 : (fits(2) ? 2 : 1));
   static constexpr int NW = 4 * WAVES / BLOCKS;
   // the next group's window loads are in flight during the products, except where
-  // their 4 CM registers would spill (gradient modes on complex grids at m = 5, 6)
-  static constexpr bool AHEAD = !WG || MT <= 4 || RG;
+  // their 4 CM registers would spill (FP64 gradient modes on complex grids at m = 5, 6)
+  static constexpr bool AHEAD = !WG || MT <= 4 || RG || sizeof(R) == 4;
   static constexpr int NT = 64 * NW;
   static constexpr size_t LDS = lds(NW);
   static_assert(LDS <= kLdsPerCu, "subgrid and window rows fit the LDS");
@@ -74,22 +76,22 @@ struct GatherShape {
 // Position of cell c in LDS row b.  A wave's operand read takes one cell per
 // lane: 16 rows b and four consecutive c; the exclusive-or spreads rows whose
 // pitch is a multiple of the bank period over distinct banks.
-template <int NK, bool RG>
+template <class R, int NK, bool RG>
 __device__ __forceinline__ int cell_pos(int b, int c) {
-  if constexpr (RG)
+  if constexpr (RG || sizeof(R) == 4)
     return c ^ (NK % 2 == 0 ? 2 * ((b >> 1) & 7) : 2 * ((b >> 3) & 1));
   else
     return c ^ (NK % 2 == 0 ? (b & 7) : ((b >> 1) & 3));
 }
 
 // one lane's share of a node's window data: axis lk of node li of a group
-template <int CM, bool WG>
+template <class R, int CM, bool WG>
 struct AxisLoad {
-  int j;      // node id, -1: no node
-  double x;   // coordinate now ...
-  double px;  // ... and when the tables were made
-  double psi[CM];
-  double dpsi[WG ? CM : 1];
+  int j;  // node id, -1: no node
+  R x;    // coordinate now ...
+  R px;   // ... and when the tables were made
+  R psi[CM];
+  R dpsi[WG ? CM : 1];
 };
 
 // positions of one group of nodes
@@ -121,18 +123,21 @@ struct IntC {
   static constexpr int value = N;
 };
 
-template <int MT, int MODE, bool RG>
-__global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, MODE, RG>::WAVES)) void gather_mm64_k(BArgs<double> A) {
-  using S = GatherShape<MT, MODE, RG>;
-  constexpr int CM = S::CM, TS = S::TS, P = S::P, NK = S::NK, PITCH = S::PITCH, R = S::R, PB = S::PB;
+template <class R, int MT, int MODE, bool RG>
+__global__ __launch_bounds__((GatherShape<R, MT, MODE, RG>::NT),
+                             (GatherShape<R, MT, MODE, RG>::WAVES)) void gather_mm_k(BArgs<R> A) {
+  using S = GatherShape<R, MT, MODE, RG>;
+  using V2 = typename Vec<R>::V2;
+  using V4 = typename Vec<R>::V4;
+  constexpr int CM = S::CM, TS = S::TS, P = S::P, NK = S::NK, PITCH = S::PITCH, XR = S::XR, PB = S::PB;
   constexpr int NW = S::NW, NT = S::NT;
   constexpr bool WF = S::WF, WG = S::WG;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  double2* const sub = reinterpret_cast<double2*>(smem_raw);  // [P][P][PITCH] complex cells ...
-  double* const sub_r = reinterpret_cast<double*>(smem_raw);  // ... or real cells (c2r plans)
+  V2* const sub = reinterpret_cast<V2*>(smem_raw);  // [P][P][PITCH] complex cells ...
+  R* const sub_r = reinterpret_cast<R*>(smem_raw);  // ... or real cells (c2r plans)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lk = lane >> 4;
-  double* const rows = reinterpret_cast<double*>(smem_raw + S::SUB) + wave * S::AREA;  // this wave's window rows
+  R* const rows = reinterpret_cast<R*>(smem_raw + S::SUB) + wave * S::AREA;  // this wave's window rows
 
   const int4 range = A.ranges[blockIdx.x];
   const int tile = range.x, beg = range.y, end = range.w;
@@ -162,8 +167,8 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
   const int ax = lk < 3 ? lk : 0;
   const int nt = ax == 0 ? n0 : (ax == 1 ? n1 : n2);
   const int ot = ax == 0 ? o0 : (ax == 1 ? o1 : o2);
-  const double bt = ax == 0 ? A.g.b[0] : (ax == 1 ? A.g.b[1] : A.g.b[2]);
-  const double wst = ax == 0 ? A.g.ws[0] : (ax == 1 ? A.g.ws[1] : A.g.ws[2]);
+  const R bt = (R)(ax == 0 ? A.g.b[0] : (ax == 1 ? A.g.b[1] : A.g.b[2]));
+  const R wst = (R)(ax == 0 ? A.g.ws[0] : (ax == 1 ? A.g.ws[1] : A.g.ws[2]));
   const long M = A.M;
 
   // unconditional loads from clamped positions (discarded where no node exists)
@@ -171,24 +176,24 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
     const Group p = group_at(min(group_of(min(it, nit - 1), rounds, NW, wave, whole, sp), ngroups - 1), beg, mid, end, nlow);
     return min(p.first + li, p.end - 1);
   };
-  auto load_group = [&](int it, int j, AxisLoad<CM, WG>& L) __attribute__((always_inline)) {
+  auto load_group = [&](int it, int j, AxisLoad<R, CM, WG>& L) __attribute__((always_inline)) {
     const Group p = group_at(min(group_of(min(it, nit - 1), rounds, NW, wave, whole, sp), ngroups - 1), beg, mid, end, nlow);
     const bool ok = p.first + li < p.end;
     const long q = min(p.first + li, p.end - 1);
     L.j = ok ? j : -1;
     L.x = A.x[3 * (long)j + ax];
     L.px = A.pre_x[(long)ax * M + q];
-    const double* tp = A.pre_psi + (long)ax * CM * M + q;
+    const R* tp = A.pre_psi + (long)ax * CM * M + q;
 #pragma unroll
     for (int s = 0; s < CM; s++) L.psi[s] = tp[s * M];
     if (WG) {
-      const double* td = A.pre_dpsi + (long)ax * CM * M + q;
+      const R* td = A.pre_dpsi + (long)ax * CM * M + q;
 #pragma unroll
       for (int s = 0; s < CM; s++) L.dpsi[s] = td[s * M];
     }
   };
 
-  AxisLoad<CM, WG> L;
+  AxisLoad<R, CM, WG> L;
   const int j0 = A.perm[pos_at(0)];
   int jn = A.perm[pos_at(1)];
 
@@ -196,33 +201,33 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
     // stage the subgrid: LDS positions in order, the cells they hold from the grid
     if constexpr (RG) {  // pairs of real cells (an even offset never straddles the wrap)
       constexpr int NQ = P * P * PITCH / 2, K = (NQ + NT - 1) / NT;
-      const double2* src = reinterpret_cast<const double2*>(A.grid);
-      double2 v[K];
+      const V2* src = reinterpret_cast<const V2*>(A.grid);
+      V2 v[K];
 #pragma unroll
       for (int k = 0; k < K; k++) {
         const int q = tid + NT * k;
-        v[k] = make_double2(0., 0.);
+        v[k].x = v[k].y = R(0);
         if (q < NQ) {
           const int cy = (q / (PITCH / 2)) % P, cx = q / (PITCH / 2 * P);
-          const int c = cell_pos<NK, RG>(cy, 2 * (q % (PITCH / 2)));
+          const int c = cell_pos<R, NK, RG>(cy, 2 * (q % (PITCH / 2)));
           const size_t row = (size_t)((o0 + cx) & (n0 - 1)) * n1 + ((o1 + cy) & (n1 - 1));
           if (c < P) v[k] = src[(row * n2 + ((o2 + c) & (n2 - 1))) >> 1];
         }
       }
 #pragma unroll
       for (int k = 0; k < K; k++)
-        if (tid + NT * k < NQ) reinterpret_cast<double2*>(sub_r)[tid + NT * k] = v[k];
+        if (tid + NT * k < NQ) reinterpret_cast<V2*>(sub_r)[tid + NT * k] = v[k];
     } else {
       constexpr int NQ = P * P * PITCH, K = (NQ + NT - 1) / NT;
-      const double2* src = reinterpret_cast<const double2*>(A.grid);
-      double2 v[K];
+      const V2* src = reinterpret_cast<const V2*>(A.grid);
+      V2 v[K];
 #pragma unroll
       for (int k = 0; k < K; k++) {
         const int q = tid + NT * k;
-        v[k] = make_double2(0., 0.);
+        v[k].x = v[k].y = R(0);
         if (q < NQ) {
           const int cy = (q / PITCH) % P, cx = q / (PITCH * P);
-          const int c = cell_pos<NK, RG>(cy, q % PITCH);
+          const int c = cell_pos<R, NK, RG>(cy, q % PITCH);
           const size_t row = (size_t)((o0 + cx) & (n0 - 1)) * n1 + ((o1 + cy) & (n1 - 1));
           if (c < P) v[k] = src[row * n2 + ((o2 + c) & (n2 - 1))];
         }
@@ -239,7 +244,7 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
   const int bl = min(li, P - 1);
   int off[NK];
 #pragma unroll
-  for (int e = 0; e < NK; e++) off[e] = bl * PITCH + cell_pos<NK, RG>(bl, 4 * e + lk);
+  for (int e = 0; e < NK; e++) off[e] = bl * PITCH + cell_pos<R, NK, RG>(bl, 4 * e + lk);
 
   for (int it = 0; it < nit; it++) {
     const bool adds = it == rounds && sp > 1;  // uniform in the block
@@ -255,9 +260,9 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
     int l = 1 << 20, start = 0;  // l: offset of the stencil start in the tile; out of reach: no contribution
     bool bad = false;
     bool moved = false;  // coordinates changed since the tables were made
-    double frac = 0.;
+    R frac = R(0);
     if (lk < 3 && jg >= 0) {
-      const NodeAxis<double> na = node_axis<double>(L.x, nt, MT, A.g.shift);
+      const NodeAxis<R> na = node_axis<R>(L.x, nt, MT, A.g.shift);
       start = na.start;
       frac = na.frac;
       const int lo = local_off(na.start, ot, TS, nt);
@@ -270,7 +275,7 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
         const bool mine = lk == t && moved;
         wave_sync();
         if (mine)
-          eval_rows<CM, WG>(A.g.win, frac, (double)nt, bt, wst, rows + li * CM, rows + 16 * CM + li * CM);
+          eval_rows<R, CM, WG>(A.g.win, frac, (R)nt, bt, wst, rows + li * CM, rows + 16 * CM + li * CM);
         wave_sync();
         if (mine) {
 #pragma unroll
@@ -286,7 +291,7 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
     const bool ok = jg >= 0 && !((stale >> li) & 1u);
     if (!ok) l = 1 << 20;
 
-    double fr = 0., fi = 0., g0r = 0., g0i = 0., g1r = 0., g1i = 0., g2r = 0., g2i = 0.;
+    R fr = R(0), fi = R(0), g0r = R(0), g0i = R(0), g1r = R(0), g1i = R(0), g2r = R(0), g2i = R(0);
     if (few) {
       // this wave's node straight from the grid: windows of axis t of node li at
       // rows[(4 t + li) CM ..], lane r takes the stencil rows (a, b) = (r / CM, r % CM), r + 64, ...
@@ -301,19 +306,19 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
       const int s0 = __shfl(start, wave), s1 = __shfl(start, 16 + wave), s2 = __shfl(start, 32 + wave);
       const int j = __shfl(jg, wave);
       wave_sync();
-      const double *wx = rows + wave * CM, *wy = wx + 4 * CM, *wz = wx + 8 * CM;
+      const R *wx = rows + wave * CM, *wy = wx + 4 * CM, *wz = wx + 8 * CM;
       for (int r = lane; r < CM * CM; r += 64) {
         const int a = r / CM, b = r - (r / CM) * CM;
         const size_t row = ((size_t)((s0 + a) & (n0 - 1)) * n1 + ((s1 + b) & (n1 - 1))) * n2;
-        double hr = 0., hi = 0., hzr = 0., hzi = 0.;
+        R hr = R(0), hi = R(0), hzr = R(0), hzi = R(0);
 #pragma unroll
         for (int s = 0; s < CM; s++) {
           const size_t i = row + ((s2 + s) & (n2 - 1));
-          double gr, gi = 0.;
+          R gr, gi = R(0);
           if constexpr (RG) {
-            gr = reinterpret_cast<const double*>(A.grid)[i];
+            gr = reinterpret_cast<const R*>(A.grid)[i];
           } else {
-            const double2 v = reinterpret_cast<const double2*>(A.grid)[i];
+            const V2 v = reinterpret_cast<const V2*>(A.grid)[i];
             gr = v.x;
             gi = v.y;
           }
@@ -324,11 +329,11 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
             if (!RG) hzi += wz[16 * CM + s] * gi;
           }
         }
-        const double xy = wx[a] * wy[b];
+        const R xy = wx[a] * wy[b];
         fr += xy * hr;
         fi += xy * hi;
         if (WG) {
-          const double dxy = wx[16 * CM + a] * wy[b], xdy = wx[a] * wy[16 * CM + b];
+          const R dxy = wx[16 * CM + a] * wy[b], xdy = wx[a] * wy[16 * CM + b];
           g0r += dxy * hr;
           g0i += dxy * hi;
           g1r += xdy * hr;
@@ -337,19 +342,18 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
           g2i += xy * hzi;
         }
       }
-      auto red = [](double v) {
+      auto red = [](R v) {
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
         return v;
       };
-      Cplx<double> v[4] = {cmk<double>(red(fr), red(fi)), cmk<double>(0., 0.), cmk<double>(0., 0.),
-                           cmk<double>(0., 0.)};
+      Cplx<R> v[4] = {cmk<R>(red(fr), red(fi)), cmk<R>(R(0), R(0)), cmk<R>(R(0), R(0)), cmk<R>(R(0), R(0))};
       if (WG) {
-        v[1] = cmk<double>(red(g0r), red(g0i));
-        v[2] = cmk<double>(red(g1r), red(g1i));
-        v[3] = cmk<double>(red(g2r), red(g2i));
+        v[1] = cmk<R>(red(g0r), red(g0i));
+        v[2] = cmk<R>(red(g1r), red(g1i));
+        v[3] = cmk<R>(red(g2r), red(g2i));
       }
-      if (lane == 0) gather_store<double, MODE>(A, j, v);
+      if (lane == 0) gather_store<R, MODE>(A, j, v);
       return;
     }
 
@@ -378,25 +382,26 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
     auto at = [&](int d, int c, int lo) __attribute__((always_inline)) {
       const int i = c - lo;
       const bool in = (unsigned)i < (unsigned)CM;
-      const double v = rows[(d ? 16 * CM : 0) + li * CM + (in ? i : 0)];
-      return in ? v : 0.;
+      const R v = rows[(d ? 16 * CM : 0) + li * CM + (in ? i : 0)];
+      return in ? v : R(0);
     };
-    double y[4], dy[4], y16 = 0., dy16 = 0., z[NK], dz[NK];
+    R y[4], dy[4], y16[4], dy16[4], z[NK], dz[NK];
     put(1);
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      y[r] = at(0, lk + 4 * r, ly);
-      dy[r] = WG ? at(1, lk + 4 * r, ly) : 0.;
-    }
-    if constexpr (R > 0) {
-      y16 = at(0, 16 + lk % R, ly);
-      dy16 = WG ? at(1, 16 + lk % R, ly) : 0.;
+      const int b = acc_row<R>(lk, r);
+      y[r] = at(0, b, ly);
+      dy[r] = WG ? at(1, b, ly) : R(0);
+      if constexpr (XR > 0) {  // rows past the sixteenth: row b of their product is row 16 + b % XR
+        y16[r] = at(0, 16 + b % XR, ly);
+        dy16[r] = WG ? at(1, 16 + b % XR, ly) : R(0);
+      }
     }
     put(2);
 #pragma unroll
     for (int e = 0; e < NK; e++) {
       z[e] = at(0, 4 * e + lk, lz);
-      dz[e] = WG ? at(1, 4 * e + lk, lz) : 0.;
+      dz[e] = WG ? at(1, 4 * e + lk, lz) : R(0);
     }
     put(0);
 
@@ -411,7 +416,7 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
     auto sums = [&](auto k0c, auto nkc) __attribute__((always_inline)) {
       constexpr int K0 = decltype(k0c)::value, N = decltype(nkc)::value;
       struct Op {
-        double re[N], im[N];
+        R re[N], im[N];
       };
       auto ld = [&](int base, const int (&of)[NK], Op& o) __attribute__((always_inline)) {
 #pragma unroll
@@ -419,19 +424,19 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
           if constexpr (RG) {
             o.re[e] = sub_r[base + of[K0 + e]];
           } else {
-            const double2 v = sub[base + of[K0 + e]];
+            const V2 v = sub[base + of[K0 + e]];
             o.re[e] = v.x;
             o.im[e] = v.y;
           }
         }
       };
-      auto prod = [&](const Op& o, const double (&zz)[NK], d4& tr, d4& ti) __attribute__((always_inline)) {
-        tr = d4{0., 0., 0., 0.};
+      auto prod = [&](const Op& o, const R (&zz)[NK], V4& tr, V4& ti) __attribute__((always_inline)) {
+        tr = V4{R(0), R(0), R(0), R(0)};
         ti = tr;
 #pragma unroll
         for (int e = 0; e < N; e++) {
-          tr = __builtin_amdgcn_mfma_f64_16x16x4f64(o.re[e], zz[K0 + e], tr, 0, 0, 0);
-          if constexpr (!RG) ti = __builtin_amdgcn_mfma_f64_16x16x4f64(o.im[e], zz[K0 + e], ti, 0, 0, 0);
+          tr = mfma(o.re[e], zz[K0 + e], tr);
+          if constexpr (!RG) ti = mfma(o.im[e], zz[K0 + e], ti);
         }
       };
       Op o;
@@ -439,10 +444,10 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
       for (int a = amin + part; a <= amax; a += step) {
         Op on;
         ld(min(a + step, P - 1) * (P * PITCH), off, on);
-        const double xa = at(0, a, lx);
-        d4 tr, ti;
+        const R xa = at(0, a, lx);
+        V4 tr, ti;
         prod(o, z, tr, ti);
-        double sr = y[0] * tr[0], si = y[0] * ti[0];
+        R sr = y[0] * tr[0], si = y[0] * ti[0];
 #pragma unroll
         for (int r = 1; r < 4; r++) {
           sr += y[r] * tr[r];
@@ -453,7 +458,7 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
           if constexpr (!RG) fi += xa * si;
         }
         if constexpr (WG) {
-          const double da = at(1, a, lx);
+          const R da = at(1, a, lx);
           g0r += da * sr;
           if constexpr (!RG) g0i += da * si;
           sr = dy[0] * tr[0];
@@ -478,53 +483,46 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
         }
         o = on;
       }
-      if constexpr (R > 0) {
+      if constexpr (XR > 0) {
         // rows 16 .. P - 1 of the planes a0 .. a0 + PB - 1: row i of the product is
-        // row 16 + i % R of plane a0 + i / R (past amax the x windows are zero)
-        if (ym >> (16 - (CM - 1))) {
-          const int b16 = 16 + li % R;
+        // row 16 + i % XR of plane a0 + i / XR (past amax the x windows are zero)
+        if (ym >> (16 - (CM - 1) > 0 ? 16 - (CM - 1) : 0)) {
+          const int b16 = 16 + li % XR;
           int of[NK];
 #pragma unroll
-          for (int e = 0; e < NK; e++) of[e] = b16 * PITCH + cell_pos<NK, RG>(b16, 4 * e + lk);
+          for (int e = 0; e < NK; e++) of[e] = b16 * PITCH + cell_pos<R, NK, RG>(b16, 4 * e + lk);
           for (int a0 = amin + PB * part; a0 <= amax; a0 += PB * step) {
             Op q;
-            ld(min(a0 + li / R, P - 1) * (P * PITCH), of, q);
-            d4 tr, ti;
+            ld(min(a0 + li / XR, P - 1) * (P * PITCH), of, q);
+            V4 tr, ti;
             prod(q, z, tr, ti);
-            double sr = 0., si = 0., dr = 0., di = 0.;
-            double xa[4];
+            R xy[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-              xa[r] = at(0, a0 + (lk + 4 * r) / R, lx);
-              sr += xa[r] * tr[r];
-              if constexpr (!RG) si += xa[r] * ti[r];
-              if constexpr (WG) {
-                const double da = at(1, a0 + (lk + 4 * r) / R, lx);
-                dr += da * tr[r];
-                if constexpr (!RG) di += da * ti[r];
+              const int a = a0 + acc_row<R>(lk, r) / XR;
+              const R xa = at(0, a, lx);
+              xy[r] = xa * y16[r];
+              if (WF) {
+                fr += xy[r] * tr[r];
+                if constexpr (!RG) fi += xy[r] * ti[r];
               }
-            }
-            if (WF) {
-              fr += y16 * sr;
-              if constexpr (!RG) fi += y16 * si;
+              if constexpr (WG) {
+                const R dxy = at(1, a, lx) * y16[r], xdy = xa * dy16[r];
+                g0r += dxy * tr[r];
+                g1r += xdy * tr[r];
+                if constexpr (!RG) {
+                  g0i += dxy * ti[r];
+                  g1i += xdy * ti[r];
+                }
+              }
             }
             if constexpr (WG) {
-              g0r += y16 * dr;
-              g1r += dy16 * sr;
-              if constexpr (!RG) {
-                g0i += y16 * di;
-                g1i += dy16 * si;
-              }
               prod(q, dz, tr, ti);
-              sr = xa[0] * tr[0];
-              si = xa[0] * ti[0];
 #pragma unroll
-              for (int r = 1; r < 4; r++) {
-                sr += xa[r] * tr[r];
-                if constexpr (!RG) si += xa[r] * ti[r];
+              for (int r = 0; r < 4; r++) {
+                g2r += xy[r] * tr[r];
+                if constexpr (!RG) g2i += xy[r] * ti[r];
               }
-              g2r += y16 * sr;
-              if constexpr (!RG) g2i += y16 * si;
             }
           }
         }
@@ -535,12 +533,13 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
       // K-block, one from four or more starts after the first; both meet in a
       // group only where nodes moved since they were binned
       const bool lo = (zm & 0x0Fu) != 0, hi = (zm & 0xF0u) != 0;
-      if (lo && hi) sums(IntC<0>{}, IntC<NK>{});
+      if constexpr (TS < 8) sums(IntC<0>{}, IntC<NK>{});  // stencils of 4 (NK - 1) - 1 cells and more
+      else if (lo && hi) sums(IntC<0>{}, IntC<NK>{});
       else if (lo) sums(IntC<0>{}, IntC<NK - 1>{});
       else sums(IntC<1>{}, IntC<NK - 1>{});
     }
-    // sum over the four lane groups (rows b = lk + 4 r)
-    auto red = [](double v) {
+    // sum over the four lane groups
+    auto red = [](R v) {
       v += __shfl_xor(v, 16);
       v += __shfl_xor(v, 32);
       return v;
@@ -559,7 +558,7 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
     }
     if (adds) {
       // the sums of the group's waves, through their window rows (read by now)
-      const double part_sum[8] = {fr, fi, g0r, g0i, g1r, g1i, g2r, g2i};
+      const R part_sum[8] = {fr, fi, g0r, g0i, g1r, g1i, g2r, g2i};
       constexpr int V0 = WF ? 0 : 2, NV = (WG ? 8 : 2) - V0;
       static_assert(16 * NV <= S::AREA, "a wave's sums fit its window rows");
       wave_sync();
@@ -568,7 +567,7 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
         for (int k = 0; k < NV; k++) rows[k * 16 + li] = part_sum[V0 + k];
       __syncthreads();
       if (part > 0) break;
-      double sum[8];
+      R sum[8];
 #pragma unroll
       for (int k = 0; k < NV; k++) {
         sum[V0 + k] = part_sum[V0 + k];
@@ -589,11 +588,11 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
     }
     if (lk == 0 && jg >= 0) {
       if (ok) {
-        Cplx<double> v[4] = {cmk<double>(fr, fi), cmk<double>(g0r, g0i), cmk<double>(g1r, g1i),
-                             cmk<double>(g2r, g2i)};
-        gather_store<double, MODE>(A, jg, v);
+        Cplx<R> v[4] = {cmk<R>(fr, fi), cmk<R>(g0r, g0i), cmk<R>(g1r, g1i),
+                             cmk<R>(g2r, g2i)};
+        gather_store<R, MODE>(A, jg, v);
       } else {
-        A.stale_list[atomicAdd(A.stale_count, 1u)] = pos;  // gathered by gather_stale64_k
+        A.stale_list[atomicAdd(A.stale_count, 1u)] = pos;  // gathered by gather_stale_mm_k
       }
     }
     if (!S::AHEAD && it + 1 < nit) {
@@ -605,16 +604,16 @@ __global__ __launch_bounds__((GatherShape<MT, MODE, RG>::NT), (GatherShape<MT, M
 
 // nodes found outside the tile they are binned to (bins older than x): gathered
 // straight from the grid
-template <int MT, int MODE>
-__global__ __launch_bounds__(256) void gather_stale64_k(BArgs<double> A) {
+template <class R, int MT, int MODE>
+__global__ __launch_bounds__(256) void gather_stale_mm_k(BArgs<R> A) {
   constexpr int CM = 2 * MT + 1;
   constexpr bool WG = (MODE == B_GRAD || MODE == B_FGRAD || MODE == B_VJP);
   const unsigned count = *A.stale_count;
   for (unsigned k = blockIdx.x * 256 + threadIdx.x; k < count; k += gridDim.x * 256) {
     const long j = A.perm[A.stale_list[k]];
-    NodeWin<double, CM> w;
-    node_windows<double, MT, CM, WG>(A, -1, j, MT, w);
-    gather_node_global<double, CM, MODE, true>(A, j, w, CM);
+    NodeWin<R, CM> w;
+    node_windows<R, MT, CM, WG>(A, -1, j, MT, w);
+    gather_node_global<R, CM, MODE, true>(A, j, w, CM);
   }
 }
 
@@ -622,15 +621,15 @@ __global__ void zero_u32_k(unsigned* c) {
   if (threadIdx.x == 0) *c = 0u;
 }
 
-template <int MT, int MODE>
-void launch(const BArgs<double>& A, hipStream_t s) {
+template <class R, int MT, int MODE>
+void launch(const BArgs<R>& A, hipStream_t s) {
   hipLaunchKernelGGL(zero_u32_k, dim3(1), dim3(64), 0, s, A.stale_count);
   auto go = [&](auto rgc) {
     constexpr bool RG = decltype(rgc)::value;
-    using S = GatherShape<MT, MODE, RG>;
-    (void)hipFuncSetAttribute((const void*)gather_mm64_k<MT, MODE, RG>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    using S = GatherShape<R, MT, MODE, RG>;
+    (void)hipFuncSetAttribute((const void*)gather_mm_k<R, MT, MODE, RG>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)S::LDS);
-    hipLaunchKernelGGL((gather_mm64_k<MT, MODE, RG>), dim3((unsigned)A.n_items), dim3(S::NT), S::LDS, s, A);
+    hipLaunchKernelGGL((gather_mm_k<R, MT, MODE, RG>), dim3((unsigned)A.n_items), dim3(S::NT), S::LDS, s, A);
   };
   if (A.c2r)
     go(std::true_type{});
@@ -638,26 +637,35 @@ void launch(const BArgs<double>& A, hipStream_t s) {
     go(std::false_type{});
   if (A.mid) (void)hipEventRecord(A.mid, s);
   if (A.mid2) (void)hipEventRecord(A.mid2, s);
-  hipLaunchKernelGGL((gather_stale64_k<MT, MODE>), dim3(64), dim3(256), 0, s, A);
+  hipLaunchKernelGGL((gather_stale_mm_k<R, MT, MODE>), dim3(64), dim3(256), 0, s, A);
 }
 
 }  // namespace
 
-template <int MODE>
-int gather_mm64(const BArgs<double>& A, hipStream_t s) {
-  if (A.no_mfma || !A.pre_psi || !A.pre_x || (MODE != B_F && !A.pre_dpsi) || !A.ranges || A.n_items <= 0 || !A.all_dense || !A.perm || !A.stale_count || !A.stale_list ||
-      A.ts[0] != 8 || A.ts[1] != 8 || A.ts[2] != 8)
+template <class R, int MODE>
+int gather_mm(const BArgs<R>& A, hipStream_t s) {
+  const int ts = std_tile(A.g.m, sizeof(R) == 8);
+  if (A.no_mfma || !A.pre_psi || !A.pre_x || (MODE != B_F && !A.pre_dpsi) || !A.ranges || A.n_items <= 0 ||
+      !A.all_dense || !A.perm || !A.stale_count || !A.stale_list || A.ts[0] != ts || A.ts[1] != ts || A.ts[2] != ts)
     return kUnsupported;
-  switch (A.g.m) {
-    case 3: launch<3, MODE>(A, s); break;
-    case 4: launch<4, MODE>(A, s); break;
-    case 5: launch<5, MODE>(A, s); break;
-    case 6: launch<6, MODE>(A, s); break;
-    default: return kUnsupported;
+  if constexpr (sizeof(R) == 8) {
+    switch (A.g.m) {
+      case 3: launch<R, 3, MODE>(A, s); break;
+      case 4: launch<R, 4, MODE>(A, s); break;
+      case 5: launch<R, 5, MODE>(A, s); break;
+      case 6: launch<R, 6, MODE>(A, s); break;
+      default: return kUnsupported;
+    }
+  } else {
+    switch (A.g.m) {
+      case 7: launch<R, 7, MODE>(A, s); break;
+      case 8: launch<R, 8, MODE>(A, s); break;
+      default: return kUnsupported;
+    }
   }
   return hipGetLastError() == hipSuccess ? kOk : kHipError;
 }
 
-template int gather_mm64<PNFFT_B_MODE>(const BArgs<double>&, hipStream_t);
+template int gather_mm<PNFFT_B_REAL, PNFFT_B_MODE>(const BArgs<PNFFT_B_REAL>&, hipStream_t);
 
 }  // namespace pnfft_amd

@@ -412,7 +412,7 @@ __global__ __launch_bounds__(kB) void tile_place_k(const int* __restrict__ tile_
     unsigned p = 0;
     if (cnt > 0) {
       p = cnt >= 32 ? gb[__clz(cnt)] + lpos[i] : cnt > 1 ? light0 + scan[t] : single0 + scan[ntiles + t];
-      const int mid = oranges ? mid_of(beg, end) : end;
+      const int mid = vol == 512u ? mid_of(beg, end) : end;  // tiles of 8^3 cells
       for (unsigned k = 0; k < parts; k++) {
         order[p + k] = (int)t;
         if (oranges) {
@@ -663,17 +663,15 @@ template <class R>
 int gather(const BArgs<R>& A, int mode, hipStream_t s) {
   if (A.M == 0) return kOk;
   if (A.g.m < kMinPlanM || A.g.m > kMaxPlanM) return kUnsupported;
-  if constexpr (sizeof(R) == 8) {
-    int st = kUnsupported;
-    switch (mode) {
-      case B_F: st = gather_mm64<B_F>(A, s); break;
-      case B_GRAD: st = gather_mm64<B_GRAD>(A, s); break;
-      case B_FGRAD: st = gather_mm64<B_FGRAD>(A, s); break;
-      case B_VJP: st = gather_mm64<B_VJP>(A, s); break;
-      default: break;
-    }
-    if (st != kUnsupported) return st;  // kUnsupported: nothing was launched
+  int st = kUnsupported;
+  switch (mode) {
+    case B_F: st = gather_mm<R, B_F>(A, s); break;
+    case B_GRAD: st = gather_mm<R, B_GRAD>(A, s); break;
+    case B_FGRAD: st = gather_mm<R, B_FGRAD>(A, s); break;
+    case B_VJP: st = gather_mm<R, B_VJP>(A, s); break;
+    default: break;
   }
+  if (st != kUnsupported) return st;  // kUnsupported: nothing was launched
   switch (mode) {
     case B_F: return b_launch<R, 0, B_F>(A, s);
     case B_GRAD: return b_launch<R, 0, B_GRAD>(A, s);

@@ -82,11 +82,11 @@ int cols_pad(int m, bool is_double, const int* ts);
 template <class R, int MODE>
 int cols_launch(const BArgs<R>& A, hipStream_t s);
 
-// FP64 gather on the matrix cores (gather_mm64.hip) for MODE (B_F, B_GRAD,
-// B_FGRAD, B_VJP): m = 3..6 on tiles of 8^3 cells with the work items of every
-// nonempty tile; kUnsupported (nothing launched) otherwise.
-template <int MODE>
-int gather_mm64(const BArgs<double>& A, hipStream_t s);
+// Gather on the matrix cores with windows from tables (gather_mm.hip) for MODE
+// (B_F, B_GRAD, B_FGRAD, B_VJP): FP64 at m = 3..6, FP32 at m = 7, 8, on the standard
+// tiles with the work items' ranges; kUnsupported (nothing launched) otherwise.
+template <class R, int MODE>
+int gather_mm(const BArgs<R>& A, hipStream_t s);
 
 // FP64 scatter on the matrix cores (scatter_mm64.hip) for MODE (B_F, B_GRAD,
 // B_FGRAD): m = 2..6 on tiles of 8^3 cells, every window from tables; slots,
@@ -118,7 +118,8 @@ struct TileLayout {
 //    cut.part nodes; tile_slot = (first entry, -1: empty tile; entries);
 //  * ranges, oranges (or null): position ranges (tile, beg, mid, end) of the items
 //    and of the order entries; the nodes [beg, mid) start in the lower half of the
-//    tile's cells along axis 2, [mid, end) in the upper half;
+//    tile's cells along axis 2, [mid, end) in the upper half (tiles of 8^3 cells;
+//    else mid = end);
 //  * box_tile, box_ord: offset masks of the tile's nodes per axis, by tile and by
 //    order entry (with `boxes`).  The slots of the matrix-core column scatter (with
 //    the brick fold) hold only the box these masks span (from the smallest offset to

@@ -33,14 +33,14 @@
 // (256 VGPRs and one block: the same time).  The gradient modes replace kernels
 // that added every stencil cell by FP64 LDS atomics: charges and dipoles at m =
 // 4, M = 2^19 2.86 -> 0.27 ms per launch.
-#include "mm64.hpp"
+#include "mm.hpp"
 
 namespace pnfft_amd {
 
 namespace {
 
 using namespace bdev;
-using namespace mm64;
+using namespace mm;
 
 template <int MT, int MODE>
 struct ScatterShape {
@@ -241,7 +241,7 @@ __global__ __launch_bounds__((ScatterShape<MT, MODE>::NT), (ScatterShape<MT, MOD
           }
         }
       } else if (!half) {  // its coordinates changed since the tables were made
-        eval_rows<CM, WG>(A.g.win, frac, (double)nt, bt, wst, row + l, drow + l);
+        eval_rows<double, CM, WG>(A.g.win, frac, (double)nt, bt, wst, row + l, drow + l);
       }
       // zeros at the entries outside the stencil, split between the two threads
 #pragma unroll

@@ -1,4 +1,5 @@
-"""FP64 matrix-core gather and scatter against the oracle at the sizes where its tiling can go wrong (GPU).
+"""Matrix-core gather and scatter with windows from tables (FP64; FP32 at m = 7, 8) against the oracle
+at the sizes where their tiling can go wrong (GPU).
 
 A tile holds 8^3 cells and its padded subgrid 8 + 2m per axis (12 to 20: below, at and past the sixteen
 rows of a product, with 2 or 4 rows left over); nodes are taken in groups of 16, work items in chunks of
@@ -159,3 +160,48 @@ def test_tile_of_several_slots(gpu, oracle, precision, tol, m):
     assert rel(out[0], P.adj(x, f=fv)) < tol
     if precision == "float" or m <= 6:  # (FP64 m = 8 scatters by atomics)
         assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("c2r", [False, True])
+@pytest.mark.parametrize("kind", ["few", "tile", "corner", "lines"])
+@pytest.mark.parametrize("m,wname", [(7, "bspline"), (8, "gauss"), (7, "kb")])
+def test_fp32_wide_windows_match_oracle(gpu, oracle, kind, m, wname, c2r):
+    """FP32 at m = 7, 8 (tiles of 4 cells, subgrids of 18 and 20 rows): trafo, gradient, x-VJP and adj of
+    both, at the 1e-5 of the other FP32 comparisons with the oracle."""
+    import torch
+    print("case fp32 wide", kind, m, wname, c2r, flush=True)
+    rng = SplitMix64(5000 + 10 * m + len(kind))
+    flags = {"kb": 0, "gauss": PA.PNFFT_WINDOW_GAUSSIAN, "bspline": PA.PNFFT_WINDOW_BSPLINE}[wname]
+    N, n = (8, 16, 12), (16, 32, 32) if m == 7 else (32, 32, 32)
+    x = node_set(kind, rng, n).astype(np.float32).astype(np.float64)
+    M = len(x)
+    fh = rng.complex_normal(8 * 16 * (7 if c2r else 12)).reshape(8, 16, -1)
+    if c2r:
+        fh[0], fh[:, 0], fh[:, :, 0] = 0, 0, 0  # Nyquist planes
+    fv = rng.normal(M) if c2r else rng.complex_normal(M)
+    gv = rng.normal(3 * M) if c2r else rng.complex_normal(3 * M)
+    P = oracle.Plan(N, n, m, flags, c2r=c2r)
+    f_o, g_o = (P.trafo_c2r if c2r else P.trafo)(x, fh, compute_grad=True)
+    adj = P.adj_c2r if c2r else P.adj
+    a_o = np.asarray(adj(x, f=fv)).reshape(-1)
+    ag_o = np.asarray(adj(x, grad=gv)).reshape(-1)
+    dp = DevicePlan(N, n, m, flags, M, precision="float", c2r=c2r)
+    dp.set_x(x)
+    for tables in (False, True):
+        if tables:
+            dp.precompute(PA.PNFFT_PRE_PSI | PA.PNFFT_PRE_GRAD_PSI)
+        dp.set_f_hat(fh)
+        dp.trafo(PA.PNFFT_COMPUTE_F | PA.PNFFT_COMPUTE_GRAD_F)
+        assert rel(dp.f.cpu().numpy(), f_o) < 1e-5 and rel(dp.grad.cpu().numpy(), g_o) < 1e-5
+        dp.trafo(PA.PNFFT_COMPUTE_F)
+        assert rel(dp.f.cpu().numpy(), f_o) < 1e-5
+        gx = dp.grad_x_vjp(torch.as_tensor(fv, device="cuda:0")).cpu().numpy()
+        assert rel(gx, (np.conj(fv)[:, None] * np.asarray(g_o).reshape(M, 3)).real) < 1e-5
+        dp.set_f(fv)
+        dp.set_grad(gv)
+        dp.adj(PA.PNFFT_COMPUTE_F)
+        assert rel(dp.f_hat.cpu().numpy(), a_o) < 1e-5
+        dp.adj(PA.PNFFT_COMPUTE_F | PA.PNFFT_COMPUTE_GRAD_F)
+        assert rel(dp.f_hat.cpu().numpy(), a_o + ag_o) < 1e-5
+        assert dp.api.last_error() is None
+    dp.close()
