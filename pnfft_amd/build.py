@@ -27,18 +27,16 @@ B_VARIANTS = [
 ]
 # scatter_cols.hip is compiled once per (precision, mode)
 COLS_VARIANTS = [
-    (f"{r}_{m}", [f"-DPNFFT_B_REAL={'float' if r == 'f32' else 'double'}",
-                  f"-DPNFFT_B_IS_DOUBLE={int(r == 'f64')}", f"-DPNFFT_B_MODE={mi}"])
+    (f"{r}_{m}", [f"-DPNFFT_B_REAL={'float' if r == 'f32' else 'double'}", f"-DPNFFT_B_MODE={mi}"])
     for r in ("f32", "f64")
     for mi, m in ((1, "f"), (2, "grad"), (3, "fgrad"))
 ]
-# gather_mm.hip is compiled once per (precision, mode), scatter_mm64.hip (FP64) once per mode
+# gather_mm.hip is compiled once per (precision, mode), scatter_mm.hip as scatter_cols.hip
 MM_VARIANTS = [
     (f"{r}_{m}", [f"-DPNFFT_B_REAL={'float' if r == 'f32' else 'double'}", f"-DPNFFT_B_MODE={mi}"])
     for r in ("f32", "f64")
     for mi, m in ((1, "f"), (2, "grad"), (3, "fgrad"), (4, "vjp"))
 ]
-SM64_VARIANTS = [(m, [f"-DPNFFT_B_MODE={mi}"]) for mi, m in ((1, "f"), (2, "grad"), (3, "fgrad"))]
 # pre_psi.hip, hessian.hip and window_tab.hip are compiled once per precision
 PRE_VARIANTS = [(r, [f"-DPNFFT_B_REAL={'float' if r == 'f32' else 'double'}"]) for r in ("f32", "f64")]
 ARCH = os.environ.get("PNFFT_AMD_ARCH", "gfx950")
@@ -75,7 +73,7 @@ def build(verbose=True, force=True):
     jobs = ([("b_kernels.hip", "_" + sfx, d) for sfx, d in B_VARIANTS] +
             [("scatter_cols.hip", "_" + sfx, d) for sfx, d in COLS_VARIANTS] +
             [("gather_mm.hip", "_" + sfx, d) for sfx, d in MM_VARIANTS] +
-            [("scatter_mm64.hip", "_" + sfx, d) for sfx, d in SM64_VARIANTS] +
+            [("scatter_mm.hip", "_" + sfx, d) for sfx, d in COLS_VARIANTS] +
             [("pre_psi.hip", "_" + sfx, d) for sfx, d in PRE_VARIANTS] +
             [("hessian.hip", "_" + sfx, d) for sfx, d in PRE_VARIANTS] +
             [("window_tab.hip", "_" + sfx, d) for sfx, d in PRE_VARIANTS] + [(s, "", []) for s in SOURCES])

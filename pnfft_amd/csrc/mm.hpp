@@ -1,5 +1,5 @@
 // mm.hpp -- helpers shared by the matrix-core kernels that take every window from
-// tables (gather_mm.hip, scatter_mm64.hip): FP64 at m = 2..6, FP32 at m = 7, 8.
+// tables (gather_mm.hip, scatter_mm.hip): FP64 at m = 2..6, FP32 at m = 7, 8.
 #pragma once
 
 #include "b_device.hpp"

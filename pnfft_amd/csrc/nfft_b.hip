@@ -685,16 +685,14 @@ template <class R>
 int scatter(const BArgs<R>& A, int mode, hipStream_t s) {
   if (A.M == 0) return kOk;
   if (A.g.m < kMinPlanM || A.g.m > kMaxPlanM) return kUnsupported;
-  if constexpr (sizeof(R) == 8) {
-    int st = kUnsupported;
-    switch (mode) {
-      case B_F: st = scatter_mm64<B_F>(A, s); break;
-      case B_GRAD: st = scatter_mm64<B_GRAD>(A, s); break;
-      case B_FGRAD: st = scatter_mm64<B_FGRAD>(A, s); break;
-      default: break;
-    }
-    if (st != kUnsupported) return st;  // kUnsupported: nothing was launched
+  int mst = kUnsupported;
+  switch (mode) {
+    case B_F: mst = scatter_mm<R, B_F>(A, s); break;
+    case B_GRAD: mst = scatter_mm<R, B_GRAD>(A, s); break;
+    case B_FGRAD: mst = scatter_mm<R, B_FGRAD>(A, s); break;
+    default: break;
   }
+  if (mst != kUnsupported) return mst;  // kUnsupported: nothing was launched
   if (A.slots) {  // column path: writes every grid cell through the fold
     int st = kUnsupported;
     switch (mode) {

@@ -88,14 +88,16 @@ int cols_launch(const BArgs<R>& A, hipStream_t s);
 template <class R, int MODE>
 int gather_mm(const BArgs<R>& A, hipStream_t s);
 
-// FP64 scatter on the matrix cores (scatter_mm64.hip) for MODE (B_F, B_GRAD,
-// B_FGRAD): m = 2..6 on tiles of 8^3 cells, every window from tables; slots,
-// fold and stale nodes as cols_launch.  kUnsupported (nothing launched) otherwise.
-template <int MODE>
-int scatter_mm64(const BArgs<double>& A, hipStream_t s);
+// Scatter on the matrix cores with windows from tables (scatter_mm.hip) for MODE
+// (B_F, B_GRAD, B_FGRAD): FP64 at m = 2..6, FP32 at m = 7, 8, on the standard tiles;
+// slots, fold and stale nodes as cols_launch.  kUnsupported (nothing launched)
+// otherwise.
+template <class R, int MODE>
+int scatter_mm(const BArgs<R>& A, hipStream_t s);
 
-// Fold of the FP64 slots (tiles of 8^3 cells, m = 2..6) into the grid, which it overwrites.
-int fold_slots64(const BArgs<double>& A, hipStream_t s);
+// Fold of the slots of scatter_mm into the grid, which it overwrites.
+template <class R>
+int fold_slots(const BArgs<R>& A, hipStream_t s);
 
 // Tile layout used by the binning: a node belongs to the tile that holds its
 // stencil start (floor(n x) - m) mod n on every axis.
