@@ -33,6 +33,7 @@ namespace {
 
 constexpr int kThreads = 256;
 
+// Elements per thread of a pass over long pencils (rows_ept, cols_ept for shorter ones).
 template <class R> struct FftEpt;
 template <> struct FftEpt<float> { static constexpr int value = 32; };   // C*L = 8192
 template <> struct FftEpt<double> { static constexpr int value = 16; };  // C*L = 4096
@@ -115,6 +116,17 @@ struct PassShape {
   static constexpr size_t LDS = sizeof(Cplx<R>) * (size_t)L * (size_t)LD;
 };
 
+// Elements per thread of a rows pass: 8 for pencils of up to 256 (one radix-8
+// butterfly per thread and stage, four or two times the blocks, each with a fourth
+// or half of the LDS: more loads in flight on every size; FP32 48 x 48 rows of 64
+// 30 -> 11 us, 128^2 rows of 256 31 -> 16 us per pass, FP64 20 -> 16), else FftEpt.
+template <class R, int L>
+constexpr int rows_ept() {
+  return L <= 256 ? 8 : FftEpt<R>::value;
+}
+template <class R, int L>
+using RowsShape = PassShape<R, L, kThreads, rows_ept<R, L>()>;
+
 // Threads of a columns pass: 512 where the doubled tile still fits in 160 KB of
 // LDS (twice the pencils per block, so every row segment is twice as long:
 // 256 B at L = 512 in FP32), else 256.
@@ -130,6 +142,10 @@ constexpr int cols_threads() {
 // there than the second block.
 template <class R, int L, bool NARROW>
 constexpr int cols_ept() {
+  // up to 256 points: as few as keep row segments of 256 bytes (FP64 n = 256^3 after
+  // 128^3: axis 1 44 -> 38, axis 0 85 -> 77 us; FP32 n = 128^2 x 64: 13 -> 7 us each)
+  if (L <= 128 || (L == 256 && sizeof(R) == 8)) return 8;
+  if (L == 256) return 16;
   return (NARROW && sizeof(R) == 4 && L == 512) ? 16 : FftEpt<R>::value;
 }
 
@@ -290,7 +306,7 @@ __device__ inline int store_index(const PassArgs<R>& P, int p, int L) {
 // consecutive lanes; all stages run in LDS.
 template <class R, int L>
 __global__ __launch_bounds__(kThreads) void fft_rows(PassArgs<R> P) {
-  using S = PassShape<R, L>;
+  using S = RowsShape<R, L>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Cplx<R>* sh = reinterpret_cast<Cplx<R>*>(smem_raw);
   const int tid = threadIdx.x;
@@ -353,7 +369,7 @@ __device__ inline Cplx<R> half_coef(const Cplx<R>* u, int k, int Nh, int L) {
 // is conj(FFT(conj)).
 template <class R, int L>
 __global__ __launch_bounds__(kThreads) void fft_rows_c2r(PassArgs<R> P) {
-  using S = PassShape<R, L>;
+  using S = RowsShape<R, L>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Cplx<R>* sh = reinterpret_cast<Cplx<R>*>(smem_raw);
   const int tid = threadIdx.x;
@@ -390,7 +406,7 @@ __global__ __launch_bounds__(kThreads) void fft_rows_c2r(PassArgs<R> P) {
 // stored half k2 = -k in [-Nh, 0] is conj G[k].
 template <class R, int L>
 __global__ __launch_bounds__(kThreads) void fft_rows_r2c(PassArgs<R> P) {
-  using S = PassShape<R, L>;
+  using S = RowsShape<R, L>;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   Cplx<R>* sh = reinterpret_cast<Cplx<R>*>(smem_raw);
   const int tid = threadIdx.x;
@@ -772,7 +788,7 @@ static PassArgs<R> make_args(const FftAxis<R>& ax) {
 
 template <class R, int L>
 static int pass_attr() {
-  constexpr size_t lr = PassShape<R, L>::LDS;
+  constexpr size_t lr = RowsShape<R, L>::LDS;
   constexpr size_t lc = cols_lds<R, L, false>();
   constexpr size_t ln = cols_lds<R, L, true>();
   auto attr = [](const void* f, size_t lds) {
@@ -797,14 +813,14 @@ static void pass_launch(int kind, dim3 grid, const PassArgs<R>& P, hipStream_t s
       else
         hipLaunchKernelGGL((fft_rows512<R, false>), grid, dim3(256), 0, s, P);
     } else {
-      constexpr size_t lds = PassShape<R, L>::LDS;
+      constexpr size_t lds = RowsShape<R, L>::LDS;
       hipLaunchKernelGGL((fft_rows<R, L>), grid, dim3(kThreads), lds, s, P);
     }
   } else if (kind == kPassRowsC2r) {
-    constexpr size_t lds = PassShape<R, L>::LDS;
+    constexpr size_t lds = RowsShape<R, L>::LDS;
     hipLaunchKernelGGL((fft_rows_c2r<R, L>), grid, dim3(kThreads), lds, s, P);
   } else if (kind == kPassRowsR2c) {
-    constexpr size_t lds = PassShape<R, L>::LDS;
+    constexpr size_t lds = RowsShape<R, L>::LDS;
     hipLaunchKernelGGL((fft_rows_r2c<R, L>), grid, dim3(kThreads), lds, s, P);
   } else {
     constexpr int nt = cols_threads<R, L>();
@@ -854,10 +870,11 @@ template <class R>
 int FftAxis<R>::init(int L_, bool half_angles) {
   L = L_;
   if (!fft_length_supported(L, sizeof(R) == 8)) return kUnsupported;
-  C = L == 512 ? kRows512Pencils : FftEpt<R>::value * kThreads / L;
   Ccols = 0;
   (void)with_length<R>(L, [&](auto Lc) {
     constexpr int LL = decltype(Lc)::value;
+    C = LL == 512 ? kRows512Pencils : RowsShape<R, LL>::C;
+    Creal = RowsShape<R, LL>::C;
     Ccols = ColsShape<R, LL, false>::C;
     Ccols_narrow = ColsShape<R, LL, true>::C;
     return kOk;
@@ -953,7 +970,7 @@ int fft3d_forward(const Fft3d<R>& F, const Cplx<R>* fhat, const double* tab, Cpl
       P.in = buf2; P.out = grid;
       P.in_outer = H; P.out_outer = n2 / 2;
       P.n_inner = n0 * n1;
-      P.C = FftEpt<R>::value * kThreads / F.ax[2].L;
+      P.C = F.ax[2].Creal;
       P.tw2 = F.ax[2].tw2;
       P.N2h = N2 / 2;
       dim3 grid_dim((P.n_inner + P.C - 1) / P.C, 1);
@@ -1021,7 +1038,7 @@ int fft3d_backward(const Fft3d<R>& F, const Cplx<R>* grid, const double* tab, Cp
       P.in = grid; P.out = buf2;
       P.in_outer = n2 / 2; P.out_outer = H;
       P.n_inner = n0 * n1;
-      P.C = FftEpt<R>::value * kThreads / F.ax[2].L;
+      P.C = F.ax[2].Creal;
       P.tw2 = F.ax[2].tw2;
       P.N2h = N2 / 2;
       P.backward = 1;

@@ -18,6 +18,7 @@ struct FftAxis {
   int L = 0;
   int C = 0;          // pencils per block, rows pass
   int Ccols = 0;         // pencils per block, axis-0 columns pass
+  int Creal = 0;         // pencils per block of the c2r / r2c rows passes
   int Ccols_narrow = 0;  // pencils per block, axis-1 columns pass
   Cplx<R>* tw = nullptr;   // device twiddles e^{-2 pi i j / L}
   Cplx<R>* tw2 = nullptr;  // c2r axis 2: e^{-i pi j / L}, j < L (the real transform has length 2L)
