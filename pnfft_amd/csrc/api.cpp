@@ -983,16 +983,21 @@ static int hessian_stage(PlanT<R>* P, NodesT<R>* D, BArgs<R> A, Cplx<R>* dh, int
   return hessian_gather<R>(A, P->ip, dh, tab, st, P->stream);
 }
 
-// Complex factor tables of this call (ctab_fill) uploaded to the device:
-// slot (pass, comp) at d_ctab + (pass * kCtabComps + comp) * 2 (N0 + N1 + N2).
+// Complex factor tables of this call (ctab_fill) uploaded to the device: slot
+// (pass, comp) at d_ctab + (pass * kCtabComps + comp) * 2 (N0 + N1 + N2), for the
+// components in the bit mask `comps` (the others are not read: a call that needs
+// one fills a tenth of the sines and cosines of all).
 template <class R>
-static const double* ctab_upload(PlanT<R>* P, bool adjoint, bool omit_d, int npass) {
+static const double* ctab_upload(PlanT<R>* P, bool adjoint, bool omit_d, int npass, unsigned comps) {
   const size_t per = 2 * (size_t)(P->N[0] + P->N[1] + P->N[2]);
-  for (int ps = 0; ps < npass; ps++)
-    for (int c = 0; c < kCtabComps; c++)
-      ctab_fill(P, ps == 1, adjoint, c, omit_d, P->h_ctab + (size_t)(ps * kCtabComps + c) * per);
-  (void)hipMemcpyAsync(P->d_ctab, P->h_ctab, sizeof(double) * per * npass * kCtabComps, hipMemcpyHostToDevice,
-                       P->stream);
+  const int nc = 32 - __builtin_clz(comps | 1u);  // components 0 .. nc - 1 are uploaded
+  for (int ps = 0; ps < npass; ps++) {
+    double* h = P->h_ctab + (size_t)ps * kCtabComps * per;
+    for (int c = 0; c < nc; c++)
+      if ((comps >> c) & 1u) ctab_fill(P, ps == 1, adjoint, c, omit_d, h + c * per);
+    (void)hipMemcpyAsync(P->d_ctab + (size_t)ps * kCtabComps * per, h, sizeof(double) * per * nc,
+                         hipMemcpyHostToDevice, P->stream);
+  }
   return P->d_ctab;
 }
 
@@ -1017,7 +1022,8 @@ static bool trafo_passes(PlanT<R>* P, NodesT<R>* D, unsigned cf, R* dx, Cplx<R>*
   const int npass = il ? 2 : 1;
   const int comps = P->c2r ? 1 : 2;
   const long M = D ? D->M : 0;
-  ctab_upload(P, false, cf & fl::OMIT_DECONV, npass);
+  unsigned need = ik ? (want_f ? 1u : 0u) | (want_g ? 0xEu : 0u) | (want_h ? 0x3F0u : 0u) : 1u;
+  ctab_upload(P, false, cf & fl::OMIT_DECONV, npass, need);
   auto fwd = [&](int ps, int comp) {
     if (cf & fl::OMIT_FFT) return true;
     if (fft3d_forward<R>(P->fft, dfh, nullptr, P->d_buf1, P->d_buf2, P->d_grid, s, P->c2r, nullptr, nullptr,
@@ -1196,7 +1202,7 @@ static bool adj_passes(PlanT<R>* P, NodesT<R>* D, unsigned cf, R* dx, Cplx<R>* d
   const int npass = il ? 2 : 1;
   const int comps = P->c2r ? 1 : 2;
   const long M = D ? D->M : 0;
-  ctab_upload(P, true, false, npass);
+  ctab_upload(P, true, false, npass, ik ? (use_f ? 1u : 0u) | (use_g ? 0xEu : 0u) : 1u);
   for (int ps = 0; ps < npass; ps++) {
     GridGeom g = P->geom;
     g.shift = ps ? 0.5 : 0.0;
