@@ -382,19 +382,19 @@ struct GatherMfmaShape {
   static constexpr int CM = 2 * MT + 1, TS = std_tile(MT, false), P = TS + 2 * MT;
   static constexpr bool WF = (MODE == B_F || MODE == B_FGRAD);
   static constexpr bool WG = (MODE == B_GRAD || MODE == B_FGRAD || MODE == B_VJP);
-  // window rows of a wave's 16 nodes: x and z rows of 17 floats (read as
-  // scalars), y rows of 20 floats (read as float4 chunks), at X 0, Y YOFF,
-  // Z ZOFF; the derivative rows follow at ROWSZ / 2.  The odd and the 20-float
-  // pitches keep the rows' stores and reads in distinct banks without a swizzle.
-  // With gradients in four-wave blocks (SYZ) the z rows take the y rows' place
-  // once those are read (both are read once per group), so such a block fits
-  // three times per CU (two-wave blocks fit three times either way).
-  static constexpr bool SYZ = WG && NW == 4;
-  static constexpr int YOFF = 16 * 17, ZOFF = SYZ ? YOFF : YOFF + 16 * 20;
-  static constexpr int ROWSZ = (WG ? 2 : 1) * (SYZ ? YOFF + 16 * 20 : ZOFF + 16 * 17);
-  // waves per SIMD the kernel is compiled for (the gradient kernels of m = 5, 6
-  // need more than the 168 VGPRs of three)
-  static constexpr int WAVES = WG && (MT >= 5 || !SYZ) ? 2 : 3;
+  // window rows of a wave's 16 nodes, 16 floats each: the x rows, then the y rows,
+  // whose place the z rows take once the y rows are read (both are read once per
+  // group); the derivative rows follow at ROWSZ / 2.
+  static constexpr int YZ = 256, ROWSZ = (WG ? 2 : 1) * 512;
+  // Waves per SIMD the kernel is compiled for.  The row sums and staging of some blocks
+  // run beside the matrix-core phase of others, so each block that fits counts: f's
+  // 40 KB (m = 4, 6) fit four times per CU, the gradient modes' 48 KB three times (their
+  // registers allow two from m = 5 on).  With rows for y and z apart (46 KB, three
+  // blocks for f) f took 481 us and now 433 us at m = 4, N = 128^3, 2^21 uniform nodes;
+  // two-wave gradient blocks at m = 6 4.09 ms and now 3.53 ms of 2^25 crowded nodes.
+  // From 2^24 nodes of a Gaussian mixture on (m = 4) f is close to the products'
+  // own cycles (1.73 -> 1.67 ms).
+  static constexpr int WAVES = WG ? (NW == 2 || MT >= 5 ? 2 : 3) : (NW == 2 ? 3 : 4);
   static constexpr int NT = 64 * NW;        // threads per block
   static constexpr size_t LDS = sizeof(float) * (2 * P * 256 + NW * ROWSZ);
 };
@@ -518,8 +518,11 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
   int jn = perm_raw(g + NW < ngroups ? g + NW : g);
   bool jn_ok = g + NW < ngroups && perm_ok(g + NW);
 
-  // this lane's window rows (lane group lk < 3: axis lk of node li)
-  float* const r0 = rows + (lk == 0 ? 0 : (lk == 1 ? S::YOFF + li * 20 : S::ZOFF)) + (lk == 1 ? 0 : li * 17);
+  // this lane's window rows (lane group lk < 3: axis lk of node li),
+  // element v of an x or z row li at v ^ li (read as scalars), of a y row at v ^ sy
+  // (read as float4 chunks): reads of the 16 rows fall in distinct banks
+  const int sy = 4 * ((li >> 1) & 3), sw = lk == 1 ? sy : li;
+  float* const r0 = rows + (lk == 0 ? 0 : S::YZ) + li * 16;
   float* const r1 = r0 + S::ROWSZ / 2;  // the derivative rows (gradient modes)
 
   for (; g < ngroups; g += NW) {
@@ -537,44 +540,40 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
     // the row zero, so it adds nothing; it is listed for the stale kernel below)
     int l = 0;
     bool bad = false;
-    // window values of this lane's axis (the z lanes of SYZ write theirs after the y rows are read)
-    float zw[S::SYZ ? CM : 1], zdw[S::SYZ ? CM : 1];
-    const bool zlate = S::SYZ && lk == 2;
+    // window values of this lane's axis (the z lanes write theirs after the y rows are read)
+    float zw[CM], zdw[WG ? CM : 1];
+    const bool zlate = lk == 2;
     if (lk < 3 && jg >= 0) {
       const NodeAxis<float> na = node_axis<float>(L.x, nt, MT, A.g.shift);
       l = local_off(na.start, ot, TS, nt);
       bad = l < 0;
       if (tab && L.x == L.px) {
-        if constexpr (S::SYZ) {
 #pragma unroll
-          for (int s = 0; s < CM; s++) {
-            zw[s] = L.psi[s];
-            zdw[s] = L.dpsi[s];
-          }
+        for (int s = 0; s < CM; s++) {
+          zw[s] = L.psi[s];
+          if (WG) zdw[s] = L.dpsi[s];
         }
         if (!bad && !zlate) {
 #pragma unroll
           for (int s = 0; s < CM; s++) {
-            r0[l + s] = L.psi[s];
-            if (WG) r1[l + s] = L.dpsi[s];
+            r0[(l + s) ^ sw] = L.psi[s];
+            if (WG) r1[(l + s) ^ sw] = L.dpsi[s];
           }
         }
       } else {
         float w[CM], dw[CM];
         // inlined: an out-of-line call would keep w and dw in scratch memory
         [[clang::always_inline]] window_axis_s<float, CM, WG>(A.g.win, na.frac, (float)nt, bt, w, dw);
-        if constexpr (S::SYZ) {
 #pragma unroll
-          for (int s = 0; s < CM; s++) {
-            zw[s] = w[s] * wst;
-            zdw[s] = dw[s] * wst;
-          }
+        for (int s = 0; s < CM; s++) {
+          zw[s] = w[s] * wst;
+          if (WG) zdw[s] = dw[s] * wst;
         }
         if (!bad && !zlate) {
 #pragma unroll
           for (int s = 0; s < CM; s++) {
-            r0[l + s] = w[s] * wst;
-            if (WG) r1[l + s] = dw[s] * wst;
+            r0[(l + s) ^ sw] = w[s] * wst;
+            if (WG) r1[(l + s) ^ sw] = dw[s] * wst;
           }
         }
       }
@@ -598,39 +597,36 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
     const int jnn = perm_raw(g + 2 * NW < ngroups ? g + 2 * NW : g);
     const bool jnn_ok = g + 2 * NW < ngroups && perm_ok(g + 2 * NW);
 
-    const float* xr = rows + li * 17;
+    const float* xr = rows + li * 16;
     const float* dxr = xr + S::ROWSZ / 2;
     const int ch = 4 * (lk ^ sw4(li));
-    const float4 yb = *reinterpret_cast<const float4*>(rows + S::YOFF + li * 20 + 4 * lk);  // Y_j[4 lk + e]
+    const float4 yb = *reinterpret_cast<const float4*>(rows + S::YZ + li * 16 + ((4 * lk) ^ sy));  // Y_j[4 lk + e]
     float4 dyb = yb;
-    if (WG) dyb = *reinterpret_cast<const float4*>(rows + S::ROWSZ / 2 + S::YOFF + li * 20 + 4 * lk);
-    if constexpr (S::SYZ) {
-      // the y rows are read: clear their area (values and derivatives) and write the z rows there
-      wave_sync();
+    if (WG) dyb = *reinterpret_cast<const float4*>(rows + S::ROWSZ / 2 + S::YZ + li * 16 + ((4 * lk) ^ sy));
+    wave_sync();
+    {
+      // the y rows are read: the z rows take their place
       const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-      constexpr int NQ = 16 * 20 / 4;  // 16-byte chunks of one area
-#pragma unroll
-      for (int k = 0; k < (2 * NQ + 63) / 64; k++) {
-        const int qq = lane + 64 * k;
-        if (qq < 2 * NQ)
-          reinterpret_cast<float4*>(rows + S::YOFF + (qq >= NQ ? S::ROWSZ / 2 - NQ * 4 : 0))[qq] = z4;
-      }
+      reinterpret_cast<float4*>(rows + S::YZ)[lane] = z4;
+      if (WG) reinterpret_cast<float4*>(rows + S::ROWSZ / 2 + S::YZ)[lane] = z4;
       if (zlate && jg >= 0 && !bad) {
-        float* const rz = rows + S::ZOFF + li * 17;
 #pragma unroll
         for (int s = 0; s < CM; s++) {
-          rz[l + s] = zw[s];
-          rz[S::ROWSZ / 2 + l + s] = zdw[s];
+          r0[(l + s) ^ sw] = zw[s];
+          if (WG) r1[(l + s) ^ sw] = zdw[s];
         }
       }
-      wave_sync();
     }
-    // Z_j[4 e + lk] in component e: the K-slice of this lane group in the e-th product
-    auto zread = [&](const float* row) { return make_float4(row[lk], row[4 + lk], row[8 + lk], row[12 + lk]); };
-    const float4 zc = zread(rows + S::ZOFF + li * 17);
-    float4 dzc = zc;
-    if (WG) dzc = zread(rows + S::ROWSZ / 2 + S::ZOFF + li * 17);
+    wave_sync();
+    const float* const zr = rows + S::YZ + li * 16;
     float fr = 0.f, fi = 0.f, g0r = 0.f, g0i = 0.f, g1r = 0.f, g1i = 0.f, g2r = 0.f, g2i = 0.f;
+    // Z_j[4 e + lk] in component e: the K-slice of this lane group in the e-th product
+    auto zread = [&](const float* row) {
+      return make_float4(row[lk ^ li], row[(4 + lk) ^ li], row[(8 + lk) ^ li], row[(12 + lk) ^ li]);
+    };
+    const float4 zc = zread(zr);
+    float4 dzc = zc;
+    if (WG) dzc = zread(zr + S::ROWSZ / 2);
     // plane a + 1's operands are read while plane a is on the matrix cores;
     // products e = K0 .. K0 + NK - 1 (the K-blocks the group's stencils reach)
     auto plane_loop = [&](auto k0c, auto nkc) __attribute__((always_inline)) {
@@ -638,8 +634,8 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
       auto ld_plane = [&](int a, float4& gr, float4& gi, float& xa, float& dxa) {
         gr = *reinterpret_cast<const float4*>(s_gr + (a * 16 + li) * 16 + ch);
         gi = *reinterpret_cast<const float4*>(s_gi + (a * 16 + li) * 16 + ch);
-        xa = xr[a];
-        dxa = WG ? dxr[a] : 0.f;
+        xa = xr[a ^ li];
+        dxa = WG ? dxr[a ^ li] : 0.f;
       };
       float4 gr, gi;
       float xa, dxa;

@@ -1,4 +1,4 @@
-"""Matrix-core gather and scatter with windows from tables (FP64; FP32 at m = 7, 8) against the oracle
+"""Matrix-core gather and scatter (FP64; FP32 at m = 7, 8; FP32 gather at m <= 6) against the oracle
 at the sizes where their tiling can go wrong (GPU).
 
 A tile holds 8^3 cells and its padded subgrid 8 + 2m per axis (12 to 20: below, at and past the sixteen
@@ -203,5 +203,45 @@ def test_fp32_wide_windows_match_oracle(gpu, oracle, kind, m, wname, c2r):
         assert rel(dp.f_hat.cpu().numpy(), a_o) < 1e-5
         dp.adj(PA.PNFFT_COMPUTE_F | PA.PNFFT_COMPUTE_GRAD_F)
         assert rel(dp.f_hat.cpu().numpy(), a_o + ag_o) < 1e-5
+        assert dp.api.last_error() is None
+    dp.close()
+
+
+@pytest.mark.parametrize("c2r", [False, True])
+@pytest.mark.parametrize("kind", ["few", "tile", "corner", "lines"])
+@pytest.mark.parametrize("m,wname", [(3, "kb"), (4, "gauss"), (5, "kb"), (5, "bspline"), (6, "gauss"), (6, "bspline")])
+def test_fp32_gather_matches_oracle(gpu, oracle, kind, m, wname, c2r):
+    """FP32 gather at m <= 6: f, gradient, both and x-VJP on tiles of one node, of two groups and of more,
+    at the 1e-5 of the other FP32 comparisons with the oracle; the magnitude of the coefficients leaves
+    the relative error alone."""
+    import torch
+    print("case fp32 gather", kind, m, wname, c2r, flush=True)
+    rng = SplitMix64(6000 + 10 * m + len(kind))
+    flags = {"kb": 0, "gauss": PA.PNFFT_WINDOW_GAUSSIAN, "bspline": PA.PNFFT_WINDOW_BSPLINE}[wname]
+    N, n = (8, 16, 12), (16, 32, 32)
+    x = node_set(kind, rng, n).astype(np.float32).astype(np.float64)
+    x[x >= 0.5] = -0.5
+    M = len(x)
+    fh = rng.complex_normal(8 * 16 * (7 if c2r else 12)).reshape(8, 16, -1)
+    if c2r:
+        fh[0], fh[:, 0], fh[:, :, 0] = 0, 0, 0  # Nyquist planes
+    fv = rng.normal(M) if c2r else rng.complex_normal(M)
+    P = oracle.Plan(N, n, m, flags, c2r=c2r)
+    f_o, g_o = (P.trafo_c2r if c2r else P.trafo)(x, fh, compute_grad=True)
+    dp = DevicePlan(N, n, m, flags, M, precision="float", c2r=c2r)
+    dp.set_x(x)
+    for tables, scale in ((False, 1.0), (True, 1.0), (True, 2.0 ** -80), (True, 2.0 ** 80)):
+        if tables:
+            dp.precompute(PA.PNFFT_PRE_PSI | PA.PNFFT_PRE_GRAD_PSI)
+        dp.set_f_hat(fh * scale)
+        dp.trafo(PA.PNFFT_COMPUTE_F | PA.PNFFT_COMPUTE_GRAD_F)
+        f, g = dp.f.cpu().numpy() / scale, dp.grad.cpu().numpy() / scale
+        assert rel(f, f_o) < 1e-5 and rel(g, g_o) < 1e-5
+        dp.trafo(PA.PNFFT_COMPUTE_GRAD_F)
+        assert np.array_equal(dp.grad.cpu().numpy() / scale, g)
+        dp.trafo(PA.PNFFT_COMPUTE_F)
+        assert rel(dp.f.cpu().numpy() / scale, f_o) < 1e-5
+        gx = dp.grad_x_vjp(torch.as_tensor(fv, device="cuda:0")).cpu().numpy() / scale
+        assert rel(gx, (np.conj(fv)[:, None] * np.asarray(g_o).reshape(M, 3)).real) < 1e-5
         assert dp.api.last_error() is None
     dp.close()
