@@ -662,11 +662,12 @@ template <class R>
 static TileCut tile_cut(long M, int m) {
   TileCut c;
   // work items: 512 nodes fill the blocks of the vector kernels; the matrix-core gather
-  // with tables (FP64 m >= 4, FP32 m >= 7) takes 256, fewer (128 at least) where M / 256 items would not
-  // fill the chip (n = 64^3 in 64 tiles, m = 6: M = 3 10^5 154 us with 512, 148 us
+  // with tables (FP64 m >= 4, FP32 m >= 7) takes 256, fewer (128 at least) where M / 256
+  // items would not fill the chip (n = 64^3 in 64 tiles, m = 6: M = 3 10^5 154 us with 512, 148 us
   // with 256; M = 3 10^4 40 and 33 us with 192)
   c.item = 512;
-  if ((sizeof(R) == 8 && m >= 4 && m <= 6) || (sizeof(R) == 4 && m >= 7)) c.item = (int)std::min(256L, std::max(128L, (M / 160 + 63) / 64 * 64));
+  if ((sizeof(R) == 8 && m >= 4 && m <= 6) || (sizeof(R) == 4 && m >= 7))
+    c.item = (int)std::min(256L, std::max(128L, (M / 160 + 63) / 64 * 64));
   c.part = (int)std::max(1024L, (M / 1024 + 63) / 64 * 64);
   c.whole = (int)std::max((long)c.part, M / 455);
   return c;
@@ -904,7 +905,9 @@ static T* grow(T*& p, size_t& cap, size_t need) {
 // the arguments stay without tables and the vector kernels evaluate the windows.
 template <class R>
 static void call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s) {
-  if ((sizeof(R) == 8) != (A.g.m <= 6) || A.no_mfma || !A.ranges || D->M == 0 || (A.pre_psi && (A.pre_dpsi || !need_grad))) return;
+  if ((sizeof(R) == 8) != (A.g.m <= 6) || A.no_mfma || !A.ranges || D->M == 0 ||
+      (A.pre_psi && (A.pre_dpsi || !need_grad)))
+    return;
   const bool kept = A.pre_psi != nullptr;  // psi tables of precompute_psi: written again with equal values
   const size_t M = (size_t)D->M, cm = 2 * (size_t)A.g.m + 1;
   R* psi = grow(D->d_pre_psi, D->pre_psi_cap, 3 * cm * M);

@@ -291,7 +291,10 @@ __global__ __launch_bounds__((GatherShape<R, MT, MODE, RG>::NT),
     const bool ok = jg >= 0 && !((stale >> li) & 1u);
     if (!ok) l = 1 << 20;
 
-    R fr = R(0), fi = R(0), g0r = R(0), g0i = R(0), g1r = R(0), g1i = R(0), g2r = R(0), g2i = R(0);
+    // A node's sums over planes and lane groups are FP64 for FP32 plans too: with FP32
+    // sums f at m = 8 was up to 1.3% further from an FP64 plan's than the vector
+    // kernel's.
+    double fr = 0.0, fi = 0.0, g0r = 0.0, g0i = 0.0, g1r = 0.0, g1i = 0.0, g2r = 0.0, g2i = 0.0;
     if (few) {
       // this wave's node straight from the grid: windows of axis t of node li at
       // rows[(4 t + li) CM ..], lane r takes the stencil rows (a, b) = (r / CM, r % CM), r + 64, ...
@@ -330,19 +333,19 @@ __global__ __launch_bounds__((GatherShape<R, MT, MODE, RG>::NT),
           }
         }
         const R xy = wx[a] * wy[b];
-        fr += xy * hr;
-        fi += xy * hi;
+        fr = fma((double)xy, (double)hr, fr);
+        fi = fma((double)xy, (double)hi, fi);
         if (WG) {
           const R dxy = wx[16 * CM + a] * wy[b], xdy = wx[a] * wy[16 * CM + b];
-          g0r += dxy * hr;
-          g0i += dxy * hi;
-          g1r += xdy * hr;
-          g1i += xdy * hi;
-          g2r += xy * hzr;
-          g2i += xy * hzi;
+          g0r = fma((double)dxy, (double)hr, g0r);
+          g0i = fma((double)dxy, (double)hi, g0i);
+          g1r = fma((double)xdy, (double)hr, g1r);
+          g1i = fma((double)xdy, (double)hi, g1i);
+          g2r = fma((double)xy, (double)hzr, g2r);
+          g2i = fma((double)xy, (double)hzi, g2i);
         }
       }
-      auto red = [](R v) {
+      auto red = [](double v) {
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
         return v;
@@ -454,13 +457,13 @@ __global__ __launch_bounds__((GatherShape<R, MT, MODE, RG>::NT),
           if constexpr (!RG) si += y[r] * ti[r];
         }
         if (WF) {
-          fr += xa * sr;
-          if constexpr (!RG) fi += xa * si;
+          fr = fma((double)xa, (double)sr, fr);
+          if constexpr (!RG) fi = fma((double)xa, (double)si, fi);
         }
         if constexpr (WG) {
           const R da = at(1, a, lx);
-          g0r += da * sr;
-          if constexpr (!RG) g0i += da * si;
+          g0r = fma((double)da, (double)sr, g0r);
+          if constexpr (!RG) g0i = fma((double)da, (double)si, g0i);
           sr = dy[0] * tr[0];
           si = dy[0] * ti[0];
 #pragma unroll
@@ -468,8 +471,8 @@ __global__ __launch_bounds__((GatherShape<R, MT, MODE, RG>::NT),
             sr += dy[r] * tr[r];
             if constexpr (!RG) si += dy[r] * ti[r];
           }
-          g1r += xa * sr;
-          if constexpr (!RG) g1i += xa * si;
+          g1r = fma((double)xa, (double)sr, g1r);
+          if constexpr (!RG) g1i = fma((double)xa, (double)si, g1i);
           prod(o, dz, tr, ti);
           sr = y[0] * tr[0];
           si = y[0] * ti[0];
@@ -478,8 +481,8 @@ __global__ __launch_bounds__((GatherShape<R, MT, MODE, RG>::NT),
             sr += y[r] * tr[r];
             if constexpr (!RG) si += y[r] * ti[r];
           }
-          g2r += xa * sr;
-          if constexpr (!RG) g2i += xa * si;
+          g2r = fma((double)xa, (double)sr, g2r);
+          if constexpr (!RG) g2i = fma((double)xa, (double)si, g2i);
         }
         o = on;
       }
@@ -503,16 +506,16 @@ __global__ __launch_bounds__((GatherShape<R, MT, MODE, RG>::NT),
               const R xa = at(0, a, lx);
               xy[r] = xa * y16[r];
               if (WF) {
-                fr += xy[r] * tr[r];
-                if constexpr (!RG) fi += xy[r] * ti[r];
+                fr = fma((double)xy[r], (double)tr[r], fr);
+                if constexpr (!RG) fi = fma((double)xy[r], (double)ti[r], fi);
               }
               if constexpr (WG) {
                 const R dxy = at(1, a, lx) * y16[r], xdy = xa * dy16[r];
-                g0r += dxy * tr[r];
-                g1r += xdy * tr[r];
+                g0r = fma((double)dxy, (double)tr[r], g0r);
+                g1r = fma((double)xdy, (double)tr[r], g1r);
                 if constexpr (!RG) {
-                  g0i += dxy * ti[r];
-                  g1i += xdy * ti[r];
+                  g0i = fma((double)dxy, (double)ti[r], g0i);
+                  g1i = fma((double)xdy, (double)ti[r], g1i);
                 }
               }
             }
@@ -520,8 +523,8 @@ __global__ __launch_bounds__((GatherShape<R, MT, MODE, RG>::NT),
               prod(q, dz, tr, ti);
 #pragma unroll
               for (int r = 0; r < 4; r++) {
-                g2r += xy[r] * tr[r];
-                if constexpr (!RG) g2i += xy[r] * ti[r];
+                g2r = fma((double)xy[r], (double)tr[r], g2r);
+                if constexpr (!RG) g2i = fma((double)xy[r], (double)ti[r], g2i);
               }
             }
           }
@@ -539,7 +542,7 @@ __global__ __launch_bounds__((GatherShape<R, MT, MODE, RG>::NT),
       else sums(IntC<1>{}, IntC<NK - 1>{});
     }
     // sum over the four lane groups
-    auto red = [](R v) {
+    auto red = [](double v) {
       v += __shfl_xor(v, 16);
       v += __shfl_xor(v, 32);
       return v;
@@ -558,7 +561,7 @@ __global__ __launch_bounds__((GatherShape<R, MT, MODE, RG>::NT),
     }
     if (adds) {
       // the sums of the group's waves, through their window rows (read by now)
-      const R part_sum[8] = {fr, fi, g0r, g0i, g1r, g1i, g2r, g2i};
+      const R part_sum[8] = {(R)fr, (R)fi, (R)g0r, (R)g0i, (R)g1r, (R)g1i, (R)g2r, (R)g2i};
       constexpr int V0 = WF ? 0 : 2, NV = (WG ? 8 : 2) - V0;
       static_assert(16 * NV <= S::AREA, "a wave's sums fit its window rows");
       wave_sync();
@@ -588,8 +591,8 @@ __global__ __launch_bounds__((GatherShape<R, MT, MODE, RG>::NT),
     }
     if (lk == 0 && jg >= 0) {
       if (ok) {
-        Cplx<R> v[4] = {cmk<R>(fr, fi), cmk<R>(g0r, g0i), cmk<R>(g1r, g1i),
-                             cmk<R>(g2r, g2i)};
+        Cplx<R> v[4] = {cmk<R>((R)fr, (R)fi), cmk<R>((R)g0r, (R)g0i), cmk<R>((R)g1r, (R)g1i),
+                        cmk<R>((R)g2r, (R)g2i)};
         gather_store<R, MODE>(A, jg, v);
       } else {
         A.stale_list[atomicAdd(A.stale_count, 1u)] = pos;  // gathered by gather_stale_mm_k
