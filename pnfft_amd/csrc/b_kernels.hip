@@ -619,7 +619,14 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
     }
     wave_sync();
     const float* const zr = rows + S::YZ + li * 16;
-    float fr = 0.f, fi = 0.f, g0r = 0.f, g0i = 0.f, g1r = 0.f, g1i = 0.f, g2r = 0.f, g2i = 0.f;
+    float fr = 0.f, fi = 0.f;
+    // The x-VJP adds planes and lane groups in FP64 and leaves the x window out of the
+    // products: with FP32 sums it was up to 15% further from an FP64 plan's than the
+    // vector kernel, which this kernel took over from (m = 4, 2^21 nodes: 1562 us there,
+    // here 825 us with FP32 sums, 875 us now).
+    constexpr bool FOLD = MODE != B_VJP;
+    using Acc = std::conditional_t<FOLD, float, double>;
+    Acc g0r = 0, g0i = 0, g1r = 0, g1i = 0, g2r = 0, g2i = 0;
     // Z_j[4 e + lk] in component e: the K-slice of this lane group in the e-th product
     auto zread = [&](const float* row) {
       return make_float4(row[lk ^ li], row[(4 + lk) ^ li], row[(8 + lk) ^ li], row[(12 + lk) ^ li]);
@@ -656,6 +663,7 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
             if constexpr (!RG) vi = __builtin_amdgcn_mfma_f32_16x16x4f32(comp4(gi, e), bz, vi, 0, 0, 0);
           }
         } else {
+          if constexpr (!FOLD) vr = vi = mfma_f4{0.f, 0.f, 0.f, 0.f};
           mfma_f4 tr = {0.f, 0.f, 0.f, 0.f}, ti = tr;
 #pragma unroll
           for (int e = K0; e < K0 + NK; e++) {
@@ -664,7 +672,7 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
           }
 #pragma unroll
           for (int e = K0; e < K0 + NK; e++) {
-            const float bz = xa * comp4(dzc, e);
+            const float bz = FOLD ? xa * comp4(dzc, e) : comp4(dzc, e);
             vr = __builtin_amdgcn_mfma_f32_16x16x4f32(comp4(gr, e), bz, vr, 0, 0, 0);
             if constexpr (!RG) vi = __builtin_amdgcn_mfma_f32_16x16x4f32(comp4(gi, e), bz, vi, 0, 0, 0);
           }
@@ -676,10 +684,16 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
           }
           const float syr = dyb.x * tr[0] + dyb.y * tr[1] + dyb.z * tr[2] + dyb.w * tr[3];
           const float syi = dyb.x * ti[0] + dyb.y * ti[1] + dyb.z * ti[2] + dyb.w * ti[3];
-          g0r += dxa * sr;
-          g0i += dxa * si;
-          g1r += xa * syr;
-          g1i += xa * syi;
+          g0r = fma((Acc)dxa, (Acc)sr, g0r);
+          g0i = fma((Acc)dxa, (Acc)si, g0i);
+          g1r = fma((Acc)xa, (Acc)syr, g1r);
+          g1i = fma((Acc)xa, (Acc)syi, g1i);
+          if constexpr (!FOLD) {
+            const float szr = yb.x * vr[0] + yb.y * vr[1] + yb.z * vr[2] + yb.w * vr[3];
+            const float szi = yb.x * vi[0] + yb.y * vi[1] + yb.z * vi[2] + yb.w * vi[3];
+            g2r = fma((Acc)xa, (Acc)szr, g2r);
+            g2i = fma((Acc)xa, (Acc)szi, g2i);
+          }
         }
         gr = grn;
         gi = gin;
@@ -691,7 +705,7 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
       if (!WG) {
         fr = vsr;
         fi = vsi;
-      } else {
+      } else if (FOLD) {
         g2r = vsr;
         g2i = vsi;
       }
@@ -707,7 +721,7 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
       plane_loop(IntC<0>{}, IntC<4>{});
     }
     // sum over the four lane groups (rows b = 4 lk + e)
-    auto red = [](float v) {
+    auto red = [](auto v) {
       v += __shfl_xor(v, 16);
       v += __shfl_xor(v, 32);
       return v;
@@ -724,7 +738,8 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
     }
     if (lk == 0 && jg >= 0) {
       if (ok) {
-        Cplx<float> v[4] = {cmk<float>(fr, fi), cmk<float>(g0r, g0i), cmk<float>(g1r, g1i), cmk<float>(g2r, g2i)};
+        Cplx<float> v[4] = {cmk<float>(fr, fi), cmk<float>((float)g0r, (float)g0i),
+                            cmk<float>((float)g1r, (float)g1i), cmk<float>((float)g2r, (float)g2i)};
         gather_store<float, MODE>(A, jg, v);
       } else {
         A.stale_list[atomicAdd(A.stale_count, 1u)] = beg + 16 * g + li;  // gathered by gather_stale_k
