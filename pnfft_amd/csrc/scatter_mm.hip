@@ -99,6 +99,10 @@ __global__ __launch_bounds__((ScatterShape<R, MT, MODE>::NT),
   // took 757 us instead of 849 (m = 8, M = 2^20, N = 64^3 real; column kernel 3431) but
   // f_hat of clustered nodes was 2.7 times further from an FP64 plan's
   using V4 = d4;
+  // Operands of the products.  In the gradient modes they hold sums of a node's terms (f Z +
+  // g2 Z', g0 X' Y + g1 X Y'): formed in FP64 as well, so that no term is rounded to 2^-24 of a
+  // larger one.
+  using Q = std::conditional_t<S::WG, double, R>;
   constexpr int CM = S::CM, TS = S::TS, P = S::P, XR = S::XR, PB = S::PB, E = S::E, PITCH = S::PITCH;
   constexpr int NW = S::NW, NB = S::NB, NP = S::NP, NX = S::NX, NXB = S::NXB;
   constexpr int XD = XR ? XR : 1;  // divisor where there are no extra rows
@@ -329,16 +333,22 @@ __global__ __launch_bounds__((ScatterShape<R, MT, MODE>::NT),
       const int v = 4 * q + lk, o = v * PITCH;
       const unsigned km = (unsigned)__builtin_amdgcn_readfirstlane((int)s_km[q]);
       // the B operands of column cell cc (weights times Z): f Z + g2 Z' and, with gradients, Z
-      V2 f, g0, g1, g2;
-      f.x = f.y = g0.x = g0.y = g1.x = g1.y = g2.x = g2.y = R(0);
-      if (WF) f = s_w[0][v];
+      struct Weight {
+        Q x, y;
+      };
+      auto weight = [&](int k) __attribute__((always_inline)) {
+        const V2 w = s_w[k][v];
+        return Weight{(Q)w.x, (Q)w.y};
+      };
+      Weight f = {Q(0), Q(0)}, g0 = f, g1 = f, g2 = f;
+      if (WF) f = weight(0);
       if constexpr (WG) {
-        g0 = s_w[1][v];
-        g1 = s_w[2][v];
-        g2 = s_w[3][v];
+        g0 = weight(1);
+        g1 = weight(2);
+        g2 = weight(3);
       }
       struct ColOp {
-        R z, re, im;
+        Q z, re, im;
       };
       auto col = [&](int cc) __attribute__((always_inline)) {
         ColOp q;
@@ -346,7 +356,7 @@ __global__ __launch_bounds__((ScatterShape<R, MT, MODE>::NT),
         q.re = f.x * q.z;
         q.im = f.y * q.z;
         if constexpr (WG) {
-          const R dz = s_row[WG ? 5 : 2][o + cc];
+          const Q dz = s_row[WG ? 5 : 2][o + cc];
           q.re = fma(g2.x, dz, q.re);
           q.im = fma(g2.y, dz, q.im);
         }
@@ -354,11 +364,11 @@ __global__ __launch_bounds__((ScatterShape<R, MT, MODE>::NT),
       };
       // plane cell a and row b of the A operand against column operand q
       auto mm = [&](int a, int b, const ColOp& q, V4& cr, V4& ci) __attribute__((always_inline)) {
-        const R x = s_row[0][o + a], y = s_row[1][o + b], xy = x * y;
+        const Q x = s_row[0][o + a], y = s_row[1][o + b], xy = x * y;
         cr = mfma(xy, q.re, cr);
         if constexpr (!RG) ci = mfma(xy, q.im, ci);
         if constexpr (WG) {
-          const R u = s_row[WG ? 3 : 0][o + a] * y, t = x * s_row[WG ? 4 : 1][o + b];
+          const Q u = s_row[WG ? 3 : 0][o + a] * y, t = x * s_row[WG ? 4 : 1][o + b];
           cr = mfma(fma(g0.x, u, g1.x * t), q.z, cr);
           if constexpr (!RG) ci = mfma(fma(g0.y, u, g1.y * t), q.z, ci);
         }
@@ -382,17 +392,17 @@ __global__ __launch_bounds__((ScatterShape<R, MT, MODE>::NT),
             // columns past the sixteenth: the planes are on the column side, the rows alone on the other,
             //   Y (x) ((f X + g0 X') Z + g2 X Z') + Y' (x) g1 X Z
             const int cc = 16 + li % XD;
-            const R x = s_row[0][o + a], y = s_row[1][o + li], xz = x * s_row[2][o + cc];
-            R br = f.x * xz, bi = f.y * xz;
+            const Q x = s_row[0][o + a], y = s_row[1][o + li], xz = x * s_row[2][o + cc];
+            Q br = f.x * xz, bi = f.y * xz;
             if constexpr (WG) {
-              const R dxz = s_row[WG ? 3 : 0][o + a] * s_row[2][o + cc], xdz = x * s_row[WG ? 5 : 2][o + cc];
+              const Q dxz = s_row[WG ? 3 : 0][o + a] * (Q)s_row[2][o + cc], xdz = x * s_row[WG ? 5 : 2][o + cc];
               br = fma(g0.x, dxz, fma(g2.x, xdz, br));
               bi = fma(g0.y, dxz, fma(g2.y, xdz, bi));
             }
             xre[u] = mfma(y, br, xre[u]);
             if constexpr (!RG) xim[u] = mfma(y, bi, xim[u]);
             if constexpr (WG) {
-              const R dy = s_row[WG ? 4 : 1][o + li];
+              const Q dy = s_row[WG ? 4 : 1][o + li];
               xre[u] = mfma(dy, g1.x * xz, xre[u]);
               if constexpr (!RG) xim[u] = mfma(dy, g1.y * xz, xim[u]);
             }

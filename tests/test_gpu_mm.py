@@ -245,3 +245,46 @@ def test_fp32_gather_matches_oracle(gpu, oracle, kind, m, wname, c2r):
         assert rel(gx, (np.conj(fv)[:, None] * np.asarray(g_o).reshape(M, 3)).real) < 1e-5
         assert dp.api.last_error() is None
     dp.close()
+
+
+@pytest.mark.parametrize("c2r", [False, True])
+@pytest.mark.parametrize("large", ["f", "gx"])
+@pytest.mark.parametrize("m,wname", [(7, "kb"), (8, "gauss")])
+def test_fp32_wide_scatter_keeps_small_terms(gpu, oracle, m, wname, large, c2r):
+    """Pairs of nodes at one place whose large values cancel: what is left of the adjoint is the small ones'.
+    The terms of a node (f; d/dx; d/dy and d/dz) are added in FP64, so each keeps its own FP32 accuracy, the 1e-5
+    of the other FP32 comparisons; a sum of a large and a small one in FP32 loses 2^-24 of the large (here 2^18
+    times the small, n times its derivative: 2^-24 2^18 / 32 = 5e-4 of the result)."""
+    print("case small terms", m, wname, large, c2r, flush=True)
+    rng = SplitMix64(7000 + m)
+    flags = {"kb": 0, "gauss": PA.PNFFT_WINDOW_GAUSSIAN}[wname]
+    N, n = (16, 16, 16), (32, 32, 32)
+    x = (rng.uniform(3 * 301).reshape(301, 3) - 0.5).astype(np.float32).astype(np.float64)
+    x[x >= 0.5] = -0.5
+    x = np.repeat(x, 2, axis=0)
+    M = len(x)
+
+    def values(k):
+        v = rng.normal(k) if c2r else rng.complex_normal(k)
+        return v.astype(np.float32 if c2r else np.complex64).astype(v.dtype)
+
+    big = np.repeat(values(M // 2), 2) * np.tile([1.0, -1.0], M // 2)
+    f, g = np.zeros_like(big), values(3 * M).reshape(M, 3) * 2.0 ** -18
+    if large == "f":
+        f = big
+    else:
+        g[:, 0] = big
+    small = g.copy()
+    if large == "gx":
+        small[:, 0] = 0
+    P = oracle.Plan(N, n, m, flags, c2r=c2r)
+    ref = np.asarray((P.adj_c2r if c2r else P.adj)(x, grad=small.reshape(-1))).reshape(-1)
+    dp = DevicePlan(N, n, m, flags, M, precision="float", c2r=c2r)
+    dp.set_x(x)
+    dp.set_f(f)
+    dp.set_grad(g)
+    for cf in (PA.PNFFT_COMPUTE_GRAD_F,) * (large == "gx") + (PA.PNFFT_COMPUTE_F | PA.PNFFT_COMPUTE_GRAD_F,):
+        dp.adj(cf)
+        assert dp.api.last_error() is None
+        assert rel(dp.f_hat.cpu().numpy(), ref) < 1e-5, cf
+    dp.close()
