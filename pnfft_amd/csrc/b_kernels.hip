@@ -94,7 +94,11 @@ __device__ inline TileItem tile_item(const BArgs<R>& A, int m) {
   const int s = A.tile_start[t], e = A.tile_start[t + 1];
   const int len = item_len(e - s, A.item_nodes);
   it.beg = min(e, s + chunk * len);
-  it.end = min(e, it.beg + len);
+  // An item has a thread per node.  The second bound tells the compiler so: without it the
+  // node loops of the scatter are compiled for several rounds, the next round's loads ahead
+  // (FP64 gradients: 246 VGPRs at m = 2, one block per CU, for 126 and two; spills from m =
+  // 3 on; M = 3 10^6 on n = 64^3 1294 us per adjoint for 948).
+  it.end = min(min(e, it.beg + len), it.beg + kTileThreads);
   return it;
 }
 
