@@ -220,7 +220,8 @@ extern "C" {
 #define PNFFT_KT_SCATTER_DIRECT 6  /* adj B^T, direct kernel */
 #define PNFFT_KT_BINNING 7         /* node binning (keys, radix sort, work items) */
 #define PNFFT_KT_SCATTER_FOLD 8    /* adj B^T, sum of the tiles' subgrids into the grid */
-#define PNFFT_KT_COUNT 9
+#define PNFFT_KT_TABLES 9          /* window tables that a call fills for its B stage */
+#define PNFFT_KT_COUNT 10
 
 #define PNFFT_MANGLE_DOUBLE(name) pnfft_##name
 #define PNFFT_MANGLE_FLOAT(name) pnfftf_##name

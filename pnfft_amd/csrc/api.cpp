@@ -172,8 +172,8 @@ static bool is_device_ptr(const void* p) {
 // ---------------------------------------------------------------------------
 // plan and nodes
 // ---------------------------------------------------------------------------
-// Event slots: 0/1 binning, 2/3 FFT (8, 9 after its first and second pass),
-// 4/5 B (10 and 13 between its kernels).
+// Event slots: 0/1 binning, 6/7 window tables of the call, 2/3 FFT (8, 9 after its first
+// and second pass), 4/5 B (10 and 13 between its kernels).
 struct EventTimer {
   hipEvent_t ev[16] = {};
   bool ok = false;
@@ -860,10 +860,16 @@ static void kt_add(PlanT<R>* P, int k, int a, int b) {
 
 // Accumulates the reference's stage timers (seconds) and the per-kernel times.
 // fwd: trafo (FFT passes rows, cols1, cols0; gather) or adj (cols0, cols1, rows;
-// scatter).  The B stage is up to three kernels separated by events 10 and 13:
-// tiled, fold (column scatter only) and direct.
+// scatter).  The B stage is the window tables of the call, where it makes any, and up to
+// three kernels separated by events 10 and 13: tiled, fold (column scatter only) and direct.
 template <class R>
-static void finish_timers(PlanT<R>* P, double* timer, bool fwd, bool had_sort, bool had_f, bool had_b) {
+static void finish_timers(PlanT<R>* P, double* timer, bool fwd, bool had_sort, bool had_tab, bool had_f, bool had_b) {
+  if (had_tab) {  // evaluating the windows is part of the B stage
+    const double t = 1e-3 * P->evt.ms(6, 7);
+    timer[T_B] += t;
+    timer[T_LOOP_B] += t;
+    kt_add(P, PNFFT_KT_TABLES, 6, 7);
+  }
   if (had_sort) {
     timer[T_SORT] += 1e-3 * P->evt.ms(0, 1);
     kt_add(P, PNFFT_KT_BINNING, 0, 1);
@@ -903,24 +909,26 @@ static T* grow(T*& p, size_t& cap, size_t need) {
 // precompute_psi made none for this call (or none of the derivatives), the
 // tables are computed into the node set's buffers now.  Without memory for them
 // the arguments stay without tables and the vector kernels evaluate the windows.
+// Returns whether tables were filled.
 template <class R>
-static void call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s) {
+static bool call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s) {
   if ((sizeof(R) == 8) != (A.g.m <= 6) || A.no_mfma || !A.ranges || D->M == 0 ||
       (A.pre_psi && (A.pre_dpsi || !need_grad)))
-    return;
+    return false;
   const bool kept = A.pre_psi != nullptr;  // psi tables of precompute_psi: written again with equal values
   const size_t M = (size_t)D->M, cm = 2 * (size_t)A.g.m + 1;
   R* psi = grow(D->d_pre_psi, D->pre_psi_cap, 3 * cm * M);
   R* dpsi = need_grad ? grow(D->d_pre_dpsi, D->pre_dpsi_cap, 3 * cm * M) : nullptr;
   R* xo = grow(D->d_pre_x, D->pre_x_cap, 3 * M);
   if (!kept) D->pre_valid = false;
-  if (!psi || !xo || (need_grad && !dpsi)) return;
+  if (!psi || !xo || (need_grad && !dpsi)) return false;
   A.pre_psi = nullptr;
   A.pre_dpsi = nullptr;
-  if (precompute_tables<R>(A, psi, dpsi, xo, s) != kOk) return;
+  if (precompute_tables<R>(A, psi, dpsi, xo, s) != kOk) return false;
   A.pre_psi = psi;
   A.pre_dpsi = dpsi;
   A.pre_x = xo;
+  return true;
 }
 
 // B stage arguments for geometry g: bins the nodes unless the bins of
@@ -928,7 +936,7 @@ static void call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s
 // and, with valid bins, the window tables.  false on a binning failure.
 template <class R>
 static bool b_args(PlanT<R>* P, NodesT<R>* D, R* dx, const GridGeom& g, bool host_x, bool for_scatter,
-                   bool timed, BArgs<R>& A, bool* had_sort, bool need_grad = true) {
+                   bool timed, BArgs<R>& A, bool* had_sort, bool* had_tab, bool need_grad = true) {
   // plans whose windows come from tables bin and tabulate on every call
   const bool reuse = !P->tab_only && D->bins_valid && (D->precompute_flags & fl::PRE_PSI) && !host_x &&
                      same_geom(D->bin_geom, g);
@@ -948,7 +956,8 @@ static bool b_args(PlanT<R>* P, NodesT<R>* D, R* dx, const GridGeom& g, bool hos
   if (for_scatter) ensure_slots(P, D);
   set_tiles(A, D, for_scatter);
   if (reuse) set_tables(A, P, D);
-  if (!P->tab_only) call_tables(A, D, need_grad, P->stream);
+  if (timed) P->evt.rec(6, P->stream);
+  bool filled = !P->tab_only && call_tables(A, D, need_grad, P->stream);
   if (P->tab_only && D->M > 0) {
     const size_t M = (size_t)D->M, cm = 2 * (size_t)P->m + 1;
     R* psi = grow(D->d_pre_psi, D->pre_psi_cap, 3 * cm * M);
@@ -962,7 +971,10 @@ static bool b_args(PlanT<R>* P, NodesT<R>* D, R* dx, const GridGeom& g, bool hos
     A.pre_psi = psi;
     A.pre_dpsi = dpsi;
     A.pre_x = xo;
+    filled = true;
   }
+  if (timed) P->evt.rec(7, P->stream);
+  if (had_tab) *had_tab = filled;
   return true;
 }
 
@@ -1041,7 +1053,7 @@ static bool trafo_passes(PlanT<R>* P, NodesT<R>* D, unsigned cf, R* dx, Cplx<R>*
     g.shift = ps ? 0.5 : 0.0;
     const int acc = (accumulate || ps > 0) ? 1 : 0;
     BArgs<R> A{};
-    if (conv && !b_args(P, D, dx, g, host_x, false, false, A, nullptr, !ik && want_g)) return false;
+    if (conv && !b_args(P, D, dx, g, host_x, false, false, A, nullptr, nullptr, !ik && want_g)) return false;
     A.real_only = (P->pnfft_flags & fl::REAL_F) ? 1 : 0;
     if (!ik) {
       if (!fwd(ps, 0)) return false;
@@ -1126,7 +1138,7 @@ static void trafo_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
     return;
   }
 
-  bool had_sort = false, had_f = false, had_b = false;
+  bool had_sort = false, had_tab = false, had_f = false, had_b = false;
   const bool general = P->pnfft_flags & (fl::INTERLACED | fl::DIFF_IK);
   if (direct) {
     NdftArgs<R> A{};
@@ -1158,7 +1170,7 @@ static void trafo_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
     // B
     if (!(cf & fl::OMIT_CONV) && M > 0 && (want_f || want_g || want_h)) {
       BArgs<R> A{};
-      if (!b_args(P, D, dx, P->geom, host_x, false, true, A, &had_sort, want_g)) return;
+      if (!b_args(P, D, dx, P->geom, host_x, false, true, A, &had_sort, &had_tab, want_g)) return;
       A.f = df;
       A.grad = dg;
       A.accumulate = accumulate;
@@ -1185,7 +1197,7 @@ static void trafo_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
     set_error("trafo: HIP error %s", hipGetErrorString(hipGetLastError()));
     return;
   }
-  finish_timers(P, P->timer_trafo, true, had_sort, had_f, had_b);
+  finish_timers(P, P->timer_trafo, true, had_sort, had_tab, had_f, had_b);
   P->timer_trafo[T_ITER] += 1;
   P->timer_trafo[T_WHOLE] += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
@@ -1210,7 +1222,7 @@ static bool adj_passes(PlanT<R>* P, NodesT<R>* D, unsigned cf, R* dx, Cplx<R>* d
     GridGeom g = P->geom;
     g.shift = ps ? 0.5 : 0.0;
     BArgs<R> A{};
-    if (conv && (use_f || use_g) && !b_args(P, D, dx, g, host_x, true, false, A, nullptr, !ik && use_g)) return false;
+    if (conv && (use_f || use_g) && !b_args(P, D, dx, g, host_x, true, false, A, nullptr, nullptr, !ik && use_g)) return false;
     // grid <- B^T (values) for one mode; then f_hat += factors(comp) F^H grid
     auto stage = [&](int mode, Cplx<R>* f, Cplx<R>* gr, int comp) {
       if (!(cf & fl::OMIT_CONV)) {
@@ -1283,7 +1295,7 @@ static void adj_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
   // zero f_hat unless accumulating (:355-356)
   if (!accumulate) fill_zero<R>(dfh, P->fhat_elems, s);
 
-  bool had_sort = false, had_f = false, had_b = false;
+  bool had_sort = false, had_tab = false, had_f = false, had_b = false;
   if (cf & fl::COMPUTE_DIRECT) {
     NdftArgs<R> A{};
     for (int t = 0; t < 3; t++) A.N[t] = (int)P->N[t];
@@ -1304,7 +1316,7 @@ static void adj_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
       // scatter() writes every cell itself
       if (M > 0 && (use_f || use_g)) {
         BArgs<R> A{};
-        if (!b_args(P, D, dx, P->geom, host_x, true, true, A, &had_sort, use_g)) return;
+        if (!b_args(P, D, dx, P->geom, host_x, true, true, A, &had_sort, &had_tab, use_g)) return;
         A.f = df;
         A.grad = dg;
         A.mid = P->evt.mark(10);
@@ -1333,7 +1345,7 @@ static void adj_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
     set_error("adj: HIP error %s", hipGetErrorString(hipGetLastError()));
     return;
   }
-  finish_timers(P, P->timer_adj, false, had_sort, had_f, had_b);
+  finish_timers(P, P->timer_adj, false, had_sort, had_tab, had_f, had_b);
   P->timer_adj[T_ITER] += 1;
   P->timer_adj[T_WHOLE] += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }

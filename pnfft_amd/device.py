@@ -118,7 +118,7 @@ class DevicePlan:
         return out
 
     KT_NAMES = ("fft_rows", "fft_cols1", "fft_cols0", "gather_tiled", "gather_direct", "scatter_tiled",
-                "scatter_direct", "binning", "scatter_fold")
+                "scatter_direct", "binning", "scatter_fold", "tables")
 
     def kernel_times(self):
         """{kernel class: (device ms accumulated, launches)} since the plan was made or reset."""
