@@ -295,6 +295,8 @@ struct NodesT {
   size_t pre_psi_cap = 0, pre_dpsi_cap = 0, pre_x_cap = 0;
   bool pre_valid = false, pre_grad = false;
   GridGeom pre_geom{};
+  R* d_call_tab = nullptr;  // tables that a call filled for itself (call_table_memory)
+  size_t call_tab_cap = 0;
   SortWork sw;
   bool bins_valid = false;
   GridGeom bin_geom{};
@@ -606,6 +608,8 @@ static void nodes_release_device(NodesT<R>* D) {
   dfree(D->d_pre_x);
   D->pre_psi_cap = D->pre_dpsi_cap = D->pre_x_cap = 0;
   D->pre_valid = false;
+  dfree(D->d_call_tab);
+  D->call_tab_cap = 0;
   D->bins_valid = false;
 }
 
@@ -903,31 +907,53 @@ static T* grow(T*& p, size_t& cap, size_t need) {
   return p;
 }
 
+// Room for the tables that a call fills for itself: psi, psi' if `grad`, coordinates,
+// in one allocation of their own, so that those of precompute_psi stay.
+template <class R>
+static bool call_table_memory(NodesT<R>* D, int m, bool grad, R*& psi, R*& dpsi, R*& x) {
+  const size_t M = (size_t)D->M, rows = 3 * (2 * (size_t)m + 1);
+  R* p = grow(D->d_call_tab, D->call_tab_cap, ((grad ? 2 : 1) * rows + 3) * M);
+  if (!p) return false;
+  psi = p;
+  dpsi = grad ? p + rows * M : nullptr;
+  x = p + (grad ? 2 : 1) * rows * M;
+  return true;
+}
+
 // Window tables for the matrix-core kernels that take every window from tables
 // (FP64 at m = 2..6, FP32 at m = 7, 8; their own evaluation would hold them to half
-// the waves): where
-// precompute_psi made none for this call (or none of the derivatives), the
-// tables are computed into the node set's buffers now.  Without memory for them
-// the arguments stay without tables and the vector kernels evaluate the windows.
-// Returns whether tables were filled.
+// the waves).  Where precompute_psi made none for this plan, the call fills its own;
+// where it made those of psi alone and the call needs psi', they are made now and
+// kept with the others.  Without memory the arguments stay without tables and the
+// vector kernels evaluate the windows.  Returns whether tables were filled.
 template <class R>
 static bool call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s) {
   if ((sizeof(R) == 8) != (A.g.m <= 6) || A.no_mfma || !A.ranges || D->M == 0 ||
       (A.pre_psi && (A.pre_dpsi || !need_grad)))
     return false;
-  const bool kept = A.pre_psi != nullptr;  // psi tables of precompute_psi: written again with equal values
-  const size_t M = (size_t)D->M, cm = 2 * (size_t)A.g.m + 1;
-  R* psi = grow(D->d_pre_psi, D->pre_psi_cap, 3 * cm * M);
-  R* dpsi = need_grad ? grow(D->d_pre_dpsi, D->pre_dpsi_cap, 3 * cm * M) : nullptr;
-  R* xo = grow(D->d_pre_x, D->pre_x_cap, 3 * M);
-  if (!kept) D->pre_valid = false;
-  if (!psi || !xo || (need_grad && !dpsi)) return false;
-  A.pre_psi = nullptr;
-  A.pre_dpsi = nullptr;
-  if (precompute_tables<R>(A, psi, dpsi, xo, s) != kOk) return false;
+  R *psi, *dpsi, *x;
+  const bool kept = A.pre_psi != nullptr;
+  if (kept) {
+    psi = D->d_pre_psi;  // written again, for the present coordinates, with psi' and them
+    dpsi = grow(D->d_pre_dpsi, D->pre_dpsi_cap, 3 * (2 * (size_t)A.g.m + 1) * (size_t)D->M);
+    x = D->d_pre_x;
+    if (!dpsi) return false;
+  } else if (!call_table_memory(D, A.g.m, need_grad, psi, dpsi, x)) {
+    return false;
+  }
+  BArgs<R> T = A;
+  T.pre_psi = T.pre_dpsi = nullptr;
+  if (precompute_tables<R>(T, psi, dpsi, x, s) != kOk) {
+    if (kept) {  // half-written tables
+      D->pre_valid = false;
+      A.pre_psi = nullptr;
+    }
+    return false;
+  }
+  if (kept) D->pre_grad = true;
   A.pre_psi = psi;
   A.pre_dpsi = dpsi;
-  A.pre_x = xo;
+  A.pre_x = x;
   return true;
 }
 
@@ -959,18 +985,15 @@ static bool b_args(PlanT<R>* P, NodesT<R>* D, R* dx, const GridGeom& g, bool hos
   if (timed) P->evt.rec(6, P->stream);
   bool filled = !P->tab_only && call_tables(A, D, need_grad, P->stream);
   if (P->tab_only && D->M > 0) {
-    const size_t M = (size_t)D->M, cm = 2 * (size_t)P->m + 1;
-    R* psi = grow(D->d_pre_psi, D->pre_psi_cap, 3 * cm * M);
-    R* dpsi = need_grad ? grow(D->d_pre_dpsi, D->pre_dpsi_cap, 3 * cm * M) : nullptr;
-    R* xo = grow(D->d_pre_x, D->pre_x_cap, 3 * M);
-    D->pre_valid = false;  // the precomputed tables, if any, are overwritten
-    if (!psi || !xo || (need_grad && !dpsi) || ext_tables<R>(A, P->ip, psi, dpsi, xo, P->stream) != kOk) {
+    R *psi, *dpsi, *x;
+    if (!call_table_memory(D, P->m, need_grad, psi, dpsi, x) ||
+        ext_tables<R>(A, P->ip, psi, dpsi, x, P->stream) != kOk) {
       set_error("window tables for the plan's window failed (device memory or launch)");
       return false;
     }
     A.pre_psi = psi;
     A.pre_dpsi = dpsi;
-    A.pre_x = xo;
+    A.pre_x = x;
     filled = true;
   }
   if (timed) P->evt.rec(7, P->stream);

@@ -43,3 +43,46 @@ def test_tables_are_timed_with_the_b_stage(gpu, precision, m):
         for slot in (MATRIX_B, LOOP_B):
             assert dp.timers()[side][slot] >= total * (1 - 4 * 2.0 ** -23)
     dp.close()
+
+
+@pytest.mark.parametrize("precision,m", [("double", 5), ("float", 7)])
+def test_derivative_tables_are_kept(gpu, precision, m):
+    """After precompute_psi(PRE_PSI) the first gradient makes psi' once; set_x discards it."""
+    print("case derivative tables", precision, m, flush=True)
+    dp = plan(precision, m)
+    dp.precompute(PA.PNFFT_PRE_PSI)
+    dp.trafo(F)
+    assert fills(dp) == 0
+    dp.trafo(G)
+    for run in (dp.trafo, dp.adj):
+        run(G)
+        run(F | G)
+        run(F)
+    assert fills(dp) == 1
+    dp.set_x(dp.x.clone())
+    dp.trafo(G)
+    assert fills(dp) == 2 and dp.api.last_error() is None
+    dp.close()
+
+
+@pytest.mark.parametrize("precision,m", [("double", 5), ("float", 7)])
+@pytest.mark.parametrize("other", ["gauss", "bessel"])
+def test_another_plan_leaves_precomputed_tables(gpu, precision, m, other):
+    """Two plans of one n and m on one node set: the second, whose window differs (or always comes from
+    tables), fills tables for its own calls and leaves those of the first."""
+    print("case two plans", precision, m, other, flush=True)
+    flags = PA.PNFFT_WINDOW_GAUSSIAN if other == "gauss" else PA.PNFFT_WINDOW_BESSEL_I0
+    a, b = plan(precision, m), plan(precision, m, flags)
+    a.precompute(PA.PNFFT_PRE_PSI | PA.PNFFT_PRE_GRAD_PSI)
+    a.trafo(F | G)
+    f, g = a.f.cpu().numpy().copy(), a.grad.cpu().numpy().copy()
+    for cf in (F, F | G):
+        b.api.trafo(b.plan, a.nodes, cf)
+        assert b.api.last_error() is None
+    assert fills(b) == 2
+    for _ in range(2):
+        a.trafo(F | G)
+        assert (a.f.cpu().numpy() == f).all() and (a.grad.cpu().numpy() == g).all()
+    assert fills(a) == 0
+    a.close()
+    b.close()
