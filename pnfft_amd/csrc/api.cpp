@@ -959,10 +959,11 @@ static bool call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s
 
 // B stage arguments for geometry g: bins the nodes unless the bins of
 // pnfft_precompute_psi are valid for g (device-resident x), then the tile lists
-// and, with valid bins, the window tables.  false on a binning failure.
+// and, with valid bins, the window tables.  need_psi: the call gathers or scatters
+// (the Hessian gather has its own tables).  false on a binning failure.
 template <class R>
 static bool b_args(PlanT<R>* P, NodesT<R>* D, R* dx, const GridGeom& g, bool host_x, bool for_scatter,
-                   bool timed, BArgs<R>& A, bool* had_sort, bool* had_tab, bool need_grad = true) {
+                   bool timed, BArgs<R>& A, bool* had_sort, bool* had_tab, bool need_grad, bool need_psi = true) {
   // plans whose windows come from tables bin and tabulate on every call
   const bool reuse = !P->tab_only && D->bins_valid && (D->precompute_flags & fl::PRE_PSI) && !host_x &&
                      same_geom(D->bin_geom, g);
@@ -983,7 +984,7 @@ static bool b_args(PlanT<R>* P, NodesT<R>* D, R* dx, const GridGeom& g, bool hos
   set_tiles(A, D, for_scatter);
   if (reuse) set_tables(A, P, D);
   if (timed) P->evt.rec(6, P->stream);
-  bool filled = !P->tab_only && call_tables(A, D, need_grad, P->stream);
+  bool filled = !P->tab_only && need_psi && call_tables(A, D, need_grad, P->stream);
   if (P->tab_only && D->M > 0) {
     R *psi, *dpsi, *x;
     if (!call_table_memory(D, P->m, need_grad, psi, dpsi, x) ||
@@ -1076,7 +1077,8 @@ static bool trafo_passes(PlanT<R>* P, NodesT<R>* D, unsigned cf, R* dx, Cplx<R>*
     g.shift = ps ? 0.5 : 0.0;
     const int acc = (accumulate || ps > 0) ? 1 : 0;
     BArgs<R> A{};
-    if (conv && !b_args(P, D, dx, g, host_x, false, false, A, nullptr, nullptr, !ik && want_g)) return false;
+    if (conv && !b_args(P, D, dx, g, host_x, false, false, A, nullptr, nullptr, !ik && want_g, ik || want_f || want_g))
+      return false;
     A.real_only = (P->pnfft_flags & fl::REAL_F) ? 1 : 0;
     if (!ik) {
       if (!fwd(ps, 0)) return false;
@@ -1193,7 +1195,7 @@ static void trafo_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
     // B
     if (!(cf & fl::OMIT_CONV) && M > 0 && (want_f || want_g || want_h)) {
       BArgs<R> A{};
-      if (!b_args(P, D, dx, P->geom, host_x, false, true, A, &had_sort, &had_tab, want_g)) return;
+      if (!b_args(P, D, dx, P->geom, host_x, false, true, A, &had_sort, &had_tab, want_g, want_f || want_g)) return;
       A.f = df;
       A.grad = dg;
       A.accumulate = accumulate;

@@ -86,3 +86,18 @@ def test_another_plan_leaves_precomputed_tables(gpu, precision, m, other):
     assert fills(a) == 0
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("precision,m", [("double", 4), ("float", 8)])
+def test_hessian_fills_no_gather_tables(gpu, precision, m):
+    """A call for the Hessian alone evaluates psi, psi' and psi'' in its own kernel: no tables for a gather that
+    does not run."""
+    print("case hessian alone", precision, m, flush=True)
+    dp = plan(precision, m)
+    dp.alloc_hessian()
+    dp.trafo(H)
+    assert dp.api.last_error() is None and fills(dp) == 0
+    h = dp.hess.cpu().numpy().copy()
+    dp.trafo(F | H)
+    assert fills(dp) == 1 and (dp.hess.cpu().numpy() == h).all()
+    dp.close()
