@@ -172,8 +172,9 @@ static bool is_device_ptr(const void* p) {
 // ---------------------------------------------------------------------------
 // plan and nodes
 // ---------------------------------------------------------------------------
-// Event slots: 0/1 binning, 6/7 window tables of the call, 2/3 FFT (8, 9 after its first
-// and second pass), 4/5 B (10 and 13 between its kernels).
+// Event slots: 0/1 binning, 2/3 FFT (8, 9 after its first and second pass), 4/5 B (10 and
+// 13 between its kernels).  Window tables of the call are filled up to event 4, from the
+// end of the binning (1) or, without one, from event 6.
 struct EventTimer {
   hipEvent_t ev[16] = {};
   bool ok = false;
@@ -867,12 +868,12 @@ static void kt_add(PlanT<R>* P, int k, int a, int b) {
 // scatter).  The B stage is the window tables of the call, where it makes any, and up to
 // three kernels separated by events 10 and 13: tiled, fold (column scatter only) and direct.
 template <class R>
-static void finish_timers(PlanT<R>* P, double* timer, bool fwd, bool had_sort, bool had_tab, bool had_f, bool had_b) {
-  if (had_tab) {  // evaluating the windows is part of the B stage
-    const double t = 1e-3 * P->evt.ms(6, 7);
+static void finish_timers(PlanT<R>* P, double* timer, bool fwd, bool had_sort, int tab_ev, bool had_f, bool had_b) {
+  if (tab_ev) {  // evaluating the windows is part of the B stage
+    const double t = 1e-3 * P->evt.ms(tab_ev, 4);
     timer[T_B] += t;
     timer[T_LOOP_B] += t;
-    kt_add(P, PNFFT_KT_TABLES, 6, 7);
+    kt_add(P, PNFFT_KT_TABLES, tab_ev, 4);
   }
   if (had_sort) {
     timer[T_SORT] += 1e-3 * P->evt.ms(0, 1);
@@ -925,9 +926,10 @@ static bool call_table_memory(NodesT<R>* D, int m, bool grad, R*& psi, R*& dpsi,
 // the waves).  Where precompute_psi made none for this plan, the call fills its own;
 // where it made those of psi alone and the call needs psi', they are made now and
 // kept with the others.  Without memory the arguments stay without tables and the
-// vector kernels evaluate the windows.  Returns whether tables were filled.
+// vector kernels evaluate the windows.  timed: event 6 is recorded before the fill.
+// Returns whether tables were filled.
 template <class R>
-static bool call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s) {
+static bool call_tables(BArgs<R>& A, PlanT<R>* P, NodesT<R>* D, bool need_grad, bool timed) {
   if ((sizeof(R) == 8) != (A.g.m <= 6) || A.no_mfma || !A.ranges || D->M == 0 ||
       (A.pre_psi && (A.pre_dpsi || !need_grad)))
     return false;
@@ -943,7 +945,8 @@ static bool call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s
   }
   BArgs<R> T = A;
   T.pre_psi = T.pre_dpsi = nullptr;
-  if (precompute_tables<R>(T, psi, dpsi, x, s) != kOk) {
+  if (timed) P->evt.rec(6, P->stream);
+  if (precompute_tables<R>(T, psi, dpsi, x, P->stream) != kOk) {
     if (kept) {  // half-written tables
       D->pre_valid = false;
       A.pre_psi = nullptr;
@@ -960,10 +963,11 @@ static bool call_tables(BArgs<R>& A, NodesT<R>* D, bool need_grad, hipStream_t s
 // B stage arguments for geometry g: bins the nodes unless the bins of
 // pnfft_precompute_psi are valid for g (device-resident x), then the tile lists
 // and, with valid bins, the window tables.  need_psi: the call gathers or scatters
-// (the Hessian gather has its own tables).  false on a binning failure.
+// (the Hessian gather has its own tables).  *tab_ev: the event from which tables were
+// filled, 0 if none were (the caller records event 4 next).  false on a binning failure.
 template <class R>
 static bool b_args(PlanT<R>* P, NodesT<R>* D, R* dx, const GridGeom& g, bool host_x, bool for_scatter,
-                   bool timed, BArgs<R>& A, bool* had_sort, bool* had_tab, bool need_grad, bool need_psi = true) {
+                   bool timed, BArgs<R>& A, bool* had_sort, int* tab_ev, bool need_grad, bool need_psi = true) {
   // plans whose windows come from tables bin and tabulate on every call
   const bool reuse = !P->tab_only && D->bins_valid && (D->precompute_flags & fl::PRE_PSI) && !host_x &&
                      same_geom(D->bin_geom, g);
@@ -983,8 +987,7 @@ static bool b_args(PlanT<R>* P, NodesT<R>* D, R* dx, const GridGeom& g, bool hos
   if (for_scatter) ensure_slots(P, D);
   set_tiles(A, D, for_scatter);
   if (reuse) set_tables(A, P, D);
-  if (timed) P->evt.rec(6, P->stream);
-  bool filled = !P->tab_only && need_psi && call_tables(A, D, need_grad, P->stream);
+  bool filled = !P->tab_only && need_psi && call_tables(A, P, D, need_grad, timed && reuse);
   if (P->tab_only && D->M > 0) {
     R *psi, *dpsi, *x;
     if (!call_table_memory(D, P->m, need_grad, psi, dpsi, x) ||
@@ -997,8 +1000,7 @@ static bool b_args(PlanT<R>* P, NodesT<R>* D, R* dx, const GridGeom& g, bool hos
     A.pre_x = x;
     filled = true;
   }
-  if (timed) P->evt.rec(7, P->stream);
-  if (had_tab) *had_tab = filled;
+  if (tab_ev && filled) *tab_ev = reuse ? 6 : 1;
   return true;
 }
 
@@ -1163,7 +1165,8 @@ static void trafo_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
     return;
   }
 
-  bool had_sort = false, had_tab = false, had_f = false, had_b = false;
+  bool had_sort = false, had_f = false, had_b = false;
+  int tab_ev = 0;
   const bool general = P->pnfft_flags & (fl::INTERLACED | fl::DIFF_IK);
   if (direct) {
     NdftArgs<R> A{};
@@ -1195,7 +1198,7 @@ static void trafo_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
     // B
     if (!(cf & fl::OMIT_CONV) && M > 0 && (want_f || want_g || want_h)) {
       BArgs<R> A{};
-      if (!b_args(P, D, dx, P->geom, host_x, false, true, A, &had_sort, &had_tab, want_g, want_f || want_g)) return;
+      if (!b_args(P, D, dx, P->geom, host_x, false, true, A, &had_sort, &tab_ev, want_g, want_f || want_g)) return;
       A.f = df;
       A.grad = dg;
       A.accumulate = accumulate;
@@ -1222,7 +1225,7 @@ static void trafo_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
     set_error("trafo: HIP error %s", hipGetErrorString(hipGetLastError()));
     return;
   }
-  finish_timers(P, P->timer_trafo, true, had_sort, had_tab, had_f, had_b);
+  finish_timers(P, P->timer_trafo, true, had_sort, tab_ev, had_f, had_b);
   P->timer_trafo[T_ITER] += 1;
   P->timer_trafo[T_WHOLE] += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
@@ -1320,7 +1323,8 @@ static void adj_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
   // zero f_hat unless accumulating (:355-356)
   if (!accumulate) fill_zero<R>(dfh, P->fhat_elems, s);
 
-  bool had_sort = false, had_tab = false, had_f = false, had_b = false;
+  bool had_sort = false, had_f = false, had_b = false;
+  int tab_ev = 0;
   if (cf & fl::COMPUTE_DIRECT) {
     NdftArgs<R> A{};
     for (int t = 0; t < 3; t++) A.N[t] = (int)P->N[t];
@@ -1341,7 +1345,7 @@ static void adj_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
       // scatter() writes every cell itself
       if (M > 0 && (use_f || use_g)) {
         BArgs<R> A{};
-        if (!b_args(P, D, dx, P->geom, host_x, true, true, A, &had_sort, &had_tab, use_g)) return;
+        if (!b_args(P, D, dx, P->geom, host_x, true, true, A, &had_sort, &tab_ev, use_g)) return;
         A.f = df;
         A.grad = dg;
         A.mid = P->evt.mark(10);
@@ -1370,7 +1374,7 @@ static void adj_impl(PlanT<R>* P, NodesT<R>* D, unsigned cf) {
     set_error("adj: HIP error %s", hipGetErrorString(hipGetLastError()));
     return;
   }
-  finish_timers(P, P->timer_adj, false, had_sort, had_tab, had_f, had_b);
+  finish_timers(P, P->timer_adj, false, had_sort, tab_ev, had_f, had_b);
   P->timer_adj[T_ITER] += 1;
   P->timer_adj[T_WHOLE] += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
@@ -1417,7 +1421,7 @@ static void vjp_impl(PlanT<R>* P, NodesT<R>* D, const Cplx<R>* w, R* gx) {
   A.c2r = P->c2r;
   set_tiles(A, D);
   if (reuse) set_tables(A, P, D);
-  call_tables(A, D, true, s);
+  call_tables(A, P, D, true, false);
   if (gather<R>(A, B_VJP, s) != kOk) set_error("gather launch failed");
   if (host_gx) (void)hipMemcpyAsync(gx, dgx, sizeof(R) * 3 * M, hipMemcpyDeviceToHost, s);
   if (hipStreamSynchronize(s) != hipSuccess) set_error("vjp: HIP error %s", hipGetErrorString(hipGetLastError()));
