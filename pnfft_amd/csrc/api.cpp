@@ -658,11 +658,14 @@ static T* stage_in(void* user, T*& mirror, size_t count, bool upload, hipStream_
 // Where a tile's nodes are cut into several blocks and slots.  One block per tile
 // leaves a launch to its heaviest tile where nodes cluster or the grid is small
 // (the chip holds 512 blocks of the FP64 scatter, 768 to 1024 of the FP32 one), so
-// tiles of much more than 1/512 of the nodes are cut into parts of 1/1024, of 1024
-// nodes at least.  Lighter tiles stay whole: a further slot costs its writing and
-// folding.  Adjoint at M = 2^20 on n = 64^3: 2048 uniform nodes per tile FP64 386 us
-// whole, 469 us in two; eight clusters 5429 us whole, 566 us cut.  M = 3 10^5 in
-// 64 tiles: 300 us whole, 239 us cut.
+// tiles of much more than 1/512 of the nodes are cut into parts: of 1/1024 of the nodes
+// on large sets, of 1024 at M = 2 10^5 and down to 128 (two batches) below, M / 200, which
+// spreads a few tiles over the chip.  Lighter tiles stay whole: a further slot costs its
+// writing and folding.  Adjoint at M = 2^20 on n = 64^3: 2048 uniform nodes per tile FP64
+// 386 us whole, 469 us in two; eight clusters 5429 us whole, 566 us cut.  Eight clusters on
+// n = 32^3, FP64, m = 2..6, parts of 1024 / 512 / 256 / 128: M = 10^4 1 / 0.77 / 0.67 / 0.65 of the
+// time, 3 10^4 1 / 0.80 / 0.74 / 0.82, 10^5 1 / 0.88 / 1.01 / 1.42, 3 10^5 1 / 1.11 / 1.29 / 1.29 (the fold
+// of one tile's slots is one block's).
 template <class R>
 static TileCut tile_cut(long M, int m) {
   TileCut c;
@@ -673,7 +676,7 @@ static TileCut tile_cut(long M, int m) {
   c.item = 512;
   if ((sizeof(R) == 8 && m >= 4 && m <= 6) || (sizeof(R) == 4 && m >= 7))
     c.item = (int)std::min(256L, std::max(128L, (M / 160 + 63) / 64 * 64));
-  c.part = (int)std::max(1024L, (M / 1024 + 63) / 64 * 64);
+  c.part = (int)std::max(std::min(1024L, std::max(128L, (M / 200 + 63) / 64 * 64)), (M / 1024 + 63) / 64 * 64);
   c.whole = (int)std::max((long)c.part, M / 455);
   return c;
 }
