@@ -89,10 +89,12 @@ __device__ __forceinline__ Batch batch_at(int it, int beg, int mid, int end, int
   return b;
 }
 
-// RG: the real grid of a c2r plan (real node values: the imaginary products are left out)
-template <class R, int MT, int MODE, bool RG>
+// RG: the real grid of a c2r plan (real node values: the imaginary products are left out).
+// ONE: compiled for one block per CU (256 VGPRs) where two are the rule (light_tiles).
+template <class R, int MT, int MODE, bool RG, bool ONE>
 __global__ __launch_bounds__((ScatterShape<R, MT, MODE>::NT),
-                             ((sizeof(R) == 8 || !RG) && ScatterShape<R, MT, MODE>::WG ? 2 : 4)) void scatter_mm_k(BArgs<R> A) {
+                             (ONE || ((sizeof(R) == 8 || !RG) && ScatterShape<R, MT, MODE>::WG) ? 2 : 4)) void scatter_mm_k(
+    BArgs<R> A) {
   using S = ScatterShape<R, MT, MODE>;
   using V2 = typename Vec<R>::V2;
   // FP64 sums for FP32 plans as well, as the column and LDS-atomic kernels have: FP32 sums
@@ -433,14 +435,30 @@ __global__ void zero_u32_k(unsigned* c) {
   if (threadIdx.x == 0) *c = 0u;
 }
 
+// FP64 f on complex grids at m = 5, 6: most tiles hold at most one batch of nodes, so a
+// block is its prologue, one batch and its slot.  The two blocks per CU of the dense case
+// spill 35 of their 128 VGPRs there, and overlapping them gains nothing: m = 5, n = 256^3, M
+// = 10^5 2461 us, one block per CU with 173 VGPRs 2141 (vector column kernel 2264); n =
+// 128^3, M = 10^4 358 and 315 us.  From about 70 nodes per tile on two blocks are faster
+// (n = 128^3, M = 3 10^5 457 and 448 us, 10^6 673 and 760), and with few tiles as well (512 tiles
+// of 20 nodes 110 and 114 us).
+template <class R, int MT, int MODE>
+bool light_tiles(const BArgs<R>& A) {
+  return sizeof(R) == 8 && MODE == B_F && MT > 4 && !A.c2r && A.n_torder >= 1024 && A.M < 64L * A.n_torder;
+}
+
 template <class R, int MT, int MODE>
 int launch(const BArgs<R>& A, hipStream_t s) {
   using S = ScatterShape<R, MT, MODE>;
+  constexpr bool HAS_ONE = sizeof(R) == 8 && MODE == B_F && MT > 4;
   hipLaunchKernelGGL(zero_u32_k, dim3(1), dim3(64), 0, s, A.stale_count);
+  const dim3 grid((unsigned)A.n_torder), block(S::NT);
   if (A.c2r)
-    hipLaunchKernelGGL((scatter_mm_k<R, MT, MODE, true>), dim3((unsigned)A.n_torder), dim3(S::NT), 0, s, A);
+    hipLaunchKernelGGL((scatter_mm_k<R, MT, MODE, true, false>), grid, block, 0, s, A);
+  else if (light_tiles<R, MT, MODE>(A))
+    hipLaunchKernelGGL((scatter_mm_k<R, MT, MODE, false, HAS_ONE>), grid, block, 0, s, A);
   else
-    hipLaunchKernelGGL((scatter_mm_k<R, MT, MODE, false>), dim3((unsigned)A.n_torder), dim3(S::NT), 0, s, A);
+    hipLaunchKernelGGL((scatter_mm_k<R, MT, MODE, false, false>), grid, block, 0, s, A);
   if (A.mid) (void)hipEventRecord(A.mid, s);
   const int st = fold_slots<R>(A, s);
   if (st != kOk) return st;

@@ -140,6 +140,33 @@ def test_fp64_gather_m3_light_tiles(gpu, oracle, c2r):
 
 
 @pytest.mark.parametrize("c2r", [False, True])
+@pytest.mark.parametrize("m", [5, 6])
+def test_fp64_scatter_light_tiles(gpu, oracle, m, c2r):
+    """More than 1024 tiles of a few nodes each, one of 200 beside them: the adjoint of f in FP64 at m = 5, 6 has a
+    variant for one block per CU there."""
+    print("case light scatter", m, c2r, flush=True)
+    rng = SplitMix64(8500 + m)
+    N, n = (64, 64, 64), (128, 128, 128)
+    x = torus(np.concatenate([rng.uniform(3 * 4000).reshape(4000, 3) - 0.5, cluster(n, m, 8, 200, rng)]), "double")
+    M = len(x)
+    fv = values(M, c2r, rng)
+    dp = DevicePlan(N, n, m, 0, M, c2r=c2r)
+    dp.set_x(x)
+    counts = tile_counts(dp)
+    assert len(counts) >= 1024 and M < 64 * len(counts) and counts.max() >= 200
+    dp.set_f(fv)
+    P = oracle.Plan(N, n, m, 0, c2r=c2r)
+    ref = (P.adj_c2r if c2r else P.adj)(x, f=fv)
+    for tables in (False, True):
+        if tables:
+            dp.precompute(TABLES)
+        dp.adj(F)
+        assert dp.api.last_error() is None
+        assert rel(dp.f_hat.cpu().numpy(), ref) < 1e-12
+    dp.close()
+
+
+@pytest.mark.parametrize("c2r", [False, True])
 @pytest.mark.parametrize("precision,m", [("double", m) for m in (2, 3, 4, 5, 6)] + [("float", m) for m in range(2, 9)])
 def test_cut_tile(gpu, oracle, precision, m, c2r):
     """3001 nodes that start in one tile, all over its cells (both halves of axis 2 and nearly empty ends of its
