@@ -789,6 +789,7 @@ static void set_tiles(BArgs<R>& A, const NodesT<R>* D, bool for_scatter = false)
     A.n_torder = D->n_torder;
     A.n_heavy = D->tc.n_heavy;
     A.n_single = D->tc.n_single;
+    A.n_cut = D->tc.n_cut;
     if (for_scatter && D->d_slots) {
       A.slots = D->d_slots;
       A.tile_slot = D->tl.tile_slot;

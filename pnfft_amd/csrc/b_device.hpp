@@ -3,6 +3,8 @@
 // value loads, the separable gather sums and the per-node global scatter.
 #pragma once
 
+#include <type_traits>
+
 #include "b_common.hpp"
 #include "device_common.hpp"
 #include "nfft_b.hpp"
@@ -123,52 +125,60 @@ __device__ __forceinline__ Cplx<R> grid_cell(const Cplx<R>* row, int i) { return
 template <class R>
 __device__ __forceinline__ Cplx<R> grid_cell(const R* row, int i) { return cmk<R>(row[i], R(0)); }
 
+// The x-VJP of FP32 plans adds the rows in fours and those sums in FP64, as the
+// matrix-core gather does; every other mode adds a plane's rows in R.
 template <class R, int CM, int MODE, class RowFn, class IdxFn>
 __device__ inline void gather_sum(NodeWin<R, CM> w, RowFn row_of, IdxFn idx, Cplx<R>* out) {
   constexpr bool WG = (MODE == B_GRAD || MODE == B_FGRAD || MODE == B_VJP);
-  Cplx<R> f = cmk<R>(0, 0), g0 = cmk<R>(0, 0), g1 = cmk<R>(0, 0), g2 = cmk<R>(0, 0);
+  constexpr bool WIDE = MODE == B_VJP && sizeof(R) == 4;
+  constexpr int NB = WIDE ? 4 : CM;
+  using A = std::conditional_t<WIDE, double, R>;
+  Cplx<A> f = cmk<A>(0, 0), g0 = cmk<A>(0, 0), g1 = cmk<A>(0, 0), g2 = cmk<A>(0, 0);
 #pragma unroll 1
   for (int a = 0; a < CM; a++) {
-    Cplx<R> ha = cmk<R>(0, 0), hay = cmk<R>(0, 0), haz = cmk<R>(0, 0);
 #pragma unroll
-    for (int b = 0; b < CM; b++) {
-      const auto row = row_of(a, b);
-      Cplx<R> hb = cmk<R>(0, 0), hbz = cmk<R>(0, 0);
+    for (int b0 = 0; b0 < CM; b0 += NB) {
+      Cplx<R> ha = cmk<R>(0, 0), hay = cmk<R>(0, 0), haz = cmk<R>(0, 0);
 #pragma unroll
-      for (int s = 0; s < CM; s++) {
-        const Cplx<R> gv = grid_cell<R>(row, idx(s));
-        hb.x += w.pz[s] * gv.x;
-        hb.y += w.pz[s] * gv.y;
+      for (int b = b0; b < (b0 + NB < CM ? b0 + NB : CM); b++) {
+        const auto row = row_of(a, b);
+        Cplx<R> hb = cmk<R>(0, 0), hbz = cmk<R>(0, 0);
+#pragma unroll
+        for (int s = 0; s < CM; s++) {
+          const Cplx<R> gv = grid_cell<R>(row, idx(s));
+          hb.x += w.pz[s] * gv.x;
+          hb.y += w.pz[s] * gv.y;
+          if (WG) {
+            hbz.x += w.dz[s] * gv.x;
+            hbz.y += w.dz[s] * gv.y;
+          }
+        }
+        ha.x += w.py[b] * hb.x;
+        ha.y += w.py[b] * hb.y;
         if (WG) {
-          hbz.x += w.dz[s] * gv.x;
-          hbz.y += w.dz[s] * gv.y;
+          hay.x += w.dy[b] * hb.x;
+          hay.y += w.dy[b] * hb.y;
+          haz.x += w.py[b] * hbz.x;
+          haz.y += w.py[b] * hbz.y;
         }
       }
-      ha.x += w.py[b] * hb.x;
-      ha.y += w.py[b] * hb.y;
+      f.x += (A)w.px[0] * ha.x;
+      f.y += (A)w.px[0] * ha.y;
       if (WG) {
-        hay.x += w.dy[b] * hb.x;
-        hay.y += w.dy[b] * hb.y;
-        haz.x += w.py[b] * hbz.x;
-        haz.y += w.py[b] * hbz.y;
+        g0.x += (A)w.dx[0] * ha.x;
+        g0.y += (A)w.dx[0] * ha.y;
+        g1.x += (A)w.px[0] * hay.x;
+        g1.y += (A)w.px[0] * hay.y;
+        g2.x += (A)w.px[0] * haz.x;
+        g2.y += (A)w.px[0] * haz.y;
       }
-    }
-    f.x += w.px[0] * ha.x;
-    f.y += w.px[0] * ha.y;
-    if (WG) {
-      g0.x += w.dx[0] * ha.x;
-      g0.y += w.dx[0] * ha.y;
-      g1.x += w.px[0] * hay.x;
-      g1.y += w.px[0] * hay.y;
-      g2.x += w.px[0] * haz.x;
-      g2.y += w.px[0] * haz.y;
     }
     shift_x<R, CM, WG>(w);
   }
-  out[0] = f;
-  out[1] = g0;
-  out[2] = g1;
-  out[3] = g2;
+  out[0] = cmk<R>((R)f.x, (R)f.y);
+  out[1] = cmk<R>((R)g0.x, (R)g0.y);
+  out[2] = cmk<R>((R)g1.x, (R)g1.y);
+  out[3] = cmk<R>((R)g2.x, (R)g2.y);
 }
 
 // The same sum for a runtime width c <= CM (generic m); same operation order.

@@ -873,6 +873,21 @@ __global__ __launch_bounds__(256) void gather_single_k(BArgs<float> A, int first
 
 inline unsigned grid1d(long n, int t) { return (unsigned)((n + t - 1) / t); }
 
+// The x-VJP at m = 2, 3 on the vector kernel (gather_tiled_k), whose threads read the
+// (2m+1)^3 cells of their own node: less than a group's 16 x 16 x 4 products cost, once a
+// tile's nodes repay its staging and there are few tiles or uneven ones, whose parts leave
+// the last wave of matrix-core blocks unfilled.  Windows from tables, vector and matrix-core
+// kernel: n = 64^3, 10^6 uniform nodes m = 2 127 and 193 us, m = 3 202 and 232; eight clusters,
+// 10^5 nodes, n = 32^3 m = 2 41 and 100 us, n = 64^3 m = 3 63 and 120.  Light tiles (n = 256^3, 5 10^4
+// nodes: m = 2 285 and 249, m = 3 397 and 289), many even tiles of many nodes (n = 128^3, 3 10^6:
+// m = 3 716 and 612) and real grids at m = 3, which halve the products (n = 64^3, 10^6: 191 and
+// 168), stay on the matrix cores.
+template <int MT, int MODE>
+bool vector_vjp(const BArgs<float>& A) {
+  if (MODE != B_VJP || MT > 3 || (MT == 3 && A.c2r) || !A.items || A.n_items <= 0) return false;
+  return A.M >= 3L * (MT - 1) * A.n_torder && (A.n_cut > 0 || A.M <= (1L << 21)) && (MT == 2 || A.n_torder <= 4096);
+}
+
 // the matrix-core gather applies to FP32 (f, grad, f + grad, VJP) with m <= 6 on the
 // standard tile layout (padded subgrids of at most 16 cells per axis), once the
 // nonempty tiles are listed
@@ -883,7 +898,7 @@ bool mfma_gather(const BArgs<R>& A) {
   } else {
     constexpr int TS = GatherMfmaShape<MT, MODE, 4>::TS;
     return !A.no_mfma && A.torder && A.oranges && A.n_torder > 0 && A.stale_count && A.stale_list && A.ts[0] == TS &&
-           A.ts[1] == TS && A.ts[2] == TS;
+           A.ts[1] == TS && A.ts[2] == TS && !vector_vjp<MT, MODE>(A);
   }
 }
 

@@ -348,7 +348,10 @@ __global__ __launch_bounds__(kB) void tile_class_k(const int* __restrict__ tile_
     }
     const unsigned parts = tile_parts(cnt, cut);
     (void)wave_class_add(cnt > 0, cnt > 0 ? __clz(cnt) : 0, lc);
-    if (parts > 1) atomicAdd(&lc[__clz(cnt)], parts - 1);
+    if (parts > 1) {
+      atomicAdd(&lc[__clz(cnt)], parts - 1);
+      atomicAdd(&work[66], 1u);
+    }
   }
   __syncthreads();
   if (threadIdx.x < 32 && lc[threadIdx.x]) atomicAdd(&work[threadIdx.x], lc[threadIdx.x]);
@@ -656,6 +659,7 @@ int build_tile_lists(const unsigned* keys, long M, const TileLayout& T, int dens
   out->n_single = (int)w[31];
   out->n_items = (int)w[64];
   out->n_items_s = (int)w[65];
+  out->n_cut = (int)w[66];
   return kOk;
 }
 

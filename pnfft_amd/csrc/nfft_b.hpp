@@ -43,6 +43,7 @@ struct BArgs {
   int n_torder;
   int n_heavy;             // tiles torder[0, n_heavy) hold 32 nodes or more, the rest at most 31
   int n_single;            // the last n_single tiles of torder hold one node each
+  int n_cut;               // tiles with several order entries
   // column scatter (scatter_cols.hip): when slots is set, scatter() runs it instead of the LDS-atomic path
   Cplx<R>* slots;          // [n_torder][P^3] padded subgrid of every order entry
   const int2* tile_slot;   // [ntiles] (first slot of each tile, -1 if empty; slots)
@@ -127,7 +128,7 @@ struct TileLayout {
 //    the brick fold) hold only the box these masks span (from the smallest offset to
 //    the largest plus 2m per axis); a node whose stencil leaves that box (moved
 //    since binning) takes the stale path.
-constexpr int kTileWork = 66;  // counters: entries per class (32), placed (32), items, items_s
+constexpr int kTileWork = 67;  // counters: entries per class (32), placed (32), items, items_s, cut tiles
 struct TileLists {
   int* tile_start;
   unsigned* scan;     // [4 ntiles]
@@ -149,6 +150,7 @@ struct TileCounts {
   int n_items, n_items_s, n_order;
   int n_heavy;   // order entries of tiles of 32 nodes or more
   int n_single;  // the last n_single entries: tiles of one node
+  int n_cut;     // tiles with several order entries
 };
 // Returns kOk (synchronizes s), kUnsupported (boxes of tiles of more than 8 cells) or kHipError.
 int build_tile_lists(const unsigned* keys, long M, const TileLayout& T, int dense_min, const TileCut& cut, bool boxes,

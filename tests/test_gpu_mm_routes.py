@@ -218,6 +218,38 @@ def test_moved_nodes(gpu, oracle, precision, m, wname, c2r):
     dp.close()
 
 
+@pytest.mark.parametrize("c2r", [False, True])
+@pytest.mark.parametrize("kind", ["light", "dense", "cut"])
+@pytest.mark.parametrize("m", [2, 3])
+def test_fp32_vjp_small_m(gpu, oracle, m, kind, c2r):
+    """The x-VJP of FP32 plans at m = 2, 3 runs on the matrix cores or on the vector kernel by nodes per tile: about
+    one, eight and more, and a tile cut into parts."""
+    import torch
+    print("case vjp", m, kind, c2r, flush=True)
+    rng = SplitMix64(8600 + m)
+    N, n = (16, 16, 16), (32, 32, 32)
+    x = {"light": lambda: rng.uniform(3 * 60).reshape(60, 3) - 0.5,
+         "dense": lambda: rng.uniform(3 * 900).reshape(900, 3) - 0.5,
+         "cut": lambda: cluster(n, m, 8, 1500, rng)}[kind]()
+    x = torus(x, "float")
+    M = len(x)
+    fh, w = coefficients(N, c2r, rng), values(M, c2r, rng)
+    dp = DevicePlan(N, n, m, 0, M, precision="float", c2r=c2r)
+    dp.set_x(x)
+    counts = tile_counts(dp)
+    assert {"light": M < 3 * len(counts), "dense": M >= 6 * len(counts), "cut": counts.max() > 1024}[kind]
+    dp.set_f_hat(fh)
+    P = oracle.Plan(N, n, m, 0, c2r=c2r)
+    g_o = np.asarray((P.trafo_c2r if c2r else P.trafo)(x, fh, compute_grad=True)[1]).reshape(M, 3)
+    for tables in (False, True):
+        if tables:
+            dp.precompute(TABLES)
+        gx = dp.grad_x_vjp(torch.as_tensor(w, device="cuda:0")).cpu().numpy()
+        assert dp.api.last_error() is None
+        assert rel(gx, (np.conj(w)[:, None] * g_o).real) < 1e-5
+    dp.close()
+
+
 def fallback_cases():
     """The kernels in use under the environment's switches, on a cut tile beside tiles of a few nodes."""
     from oracle import oracle
