@@ -282,7 +282,6 @@ struct NodesT {
   unsigned* d_keys = nullptr;
   TileLists tl{};
   TileCounts tc{};
-  int item_nodes = 0;
   bool has_ranges = false, boxes = false;
   int n_torder = 0;        // order entries (0: the layout has no column scatter)
   Cplx<R>* d_slots = nullptr;
@@ -669,9 +668,8 @@ static T* stage_in(void* user, T*& mirror, size_t count, bool upload, hipStream_
 template <class R>
 static TileCut tile_cut(long M, int m) {
   TileCut c;
-  // work items: 512 nodes fill the blocks of the vector kernels; the matrix-core gather
-  // with tables (FP64 m >= 4, FP32 m >= 7) takes 256, fewer (128 at least) where M / 256
-  // items would not fill the chip (n = 64^3 in 64 tiles, m = 6: M = 3 10^5 154 us with 512, 148 us
+  // ranges of the matrix-core gather: 256 nodes (m = 3: 512), fewer (128 at least) where M / 256
+  // ranges would not fill the chip (n = 64^3 in 64 tiles, m = 6: M = 3 10^5 154 us with 512, 148 us
   // with 256; M = 3 10^4 40 and 33 us with 192)
   c.item = 512;
   if ((sizeof(R) == 8 && m >= 4 && m <= 6) || (sizeof(R) == 4 && m >= 7))
@@ -685,7 +683,8 @@ static TileCut tile_cut(long M, int m) {
 template <class R>
 static bool ensure_bin_memory(NodesT<R>* D, const TileLayout& T, const TileCut& cut) {
   const size_t M = (size_t)D->M, nt = (size_t)T.ntiles();
-  const size_t items = nt + 2 * (M / cut.item) + 2, order = nt + M / (size_t)cut.part + 2;
+  const size_t items = nt + M / kTileThreads + 2, ranges = nt + 2 * (M / cut.item) + 2;
+  const size_t order = nt + M / (size_t)cut.part + 2;
   for (int pass = 0; pass < 2; pass++) {
     size_t at = 0;
     auto take = [&](auto*& p, size_t count) {
@@ -704,8 +703,8 @@ static bool ensure_bin_memory(NodesT<R>* D, const TileLayout& T, const TileCut& 
     take(D->d_stale, M);
     take(D->d_stale_count, 1);
     take(D->tl.tile_start, nt + 1);
-    take(D->tl.scan, 4 * nt);
-    take(D->tl.partial, 4 * (nt / 4096 + 1));
+    take(D->tl.scan, 5 * nt);
+    take(D->tl.partial, 5 * (nt / 4096 + 1));
     take(D->tl.work, kTileWork);
     take(D->tl.dense, nt);
     take(D->tl.dense_s, nt);
@@ -713,7 +712,7 @@ static bool ensure_bin_memory(NodesT<R>* D, const TileLayout& T, const TileCut& 
     take(D->tl.items_s, 2 * items);
     take(D->tl.order, order);
     take(D->tl.tile_slot, nt);
-    take(D->tl.ranges, items);
+    take(D->tl.ranges, ranges);
     take(D->tl.oranges, order);
     take(D->tl.box_tile, nt);
     take(D->tl.box_ord, order);
@@ -770,12 +769,12 @@ static void set_tiles(BArgs<R>& A, const NodesT<R>* D, bool for_scatter = false)
   A.tile_dense = two ? D->tl.dense_s : D->tl.dense;
   A.items = two ? D->tl.items_s : D->tl.items;
   A.n_items = two ? D->tc.n_items_s : D->tc.n_items;
-  A.item_nodes = D->item_nodes;
-  // The FP64 matrix-core gather needs the items' ranges.  At m = 2 the stencil fills
+  // The matrix-core gather needs the ranges.  In FP64 at m = 2 the stencil fills
   // too little of its 16-row products everywhere (M = 2^20, 2048 nodes per tile: 94
   // us on the vector kernel, 119 on the matrix cores), at m = 3 where the vector
   // kernel's threads are busy (170 and 190 us; 92 nodes per tile 467 and 319 us).
   const bool light = D->tc.n_items > 0 && D->M / D->tc.n_items < 200 && D->M >= 65536;
+  A.n_ranges = D->tc.n_ranges;
   A.ranges = D->has_ranges && (for_scatter || D->bin_geom.m > 3 || (D->bin_geom.m == 3 && light)) ? D->tl.ranges
                                                                                                  : nullptr;
   // the scatter's list holds every nonempty tile; the gather's when dense_min is 1
@@ -856,7 +855,6 @@ static int bin(PlanT<R>* P, NodesT<R>* D, const R* dx, const GridGeom& g) {
   D->n_torder = pad > 0 && D->M > 0 ? D->tc.n_order : 0;
   D->bin_geom = g;
   D->bin_tiles = P->tiles;
-  D->item_nodes = cut.item;
   D->bins_valid = true;
   return kOk;
 }

@@ -29,17 +29,16 @@ __device__ inline NodeAxis<R> node_axis(R xv, int n, int m, double sh) {
   return a;
 }
 
-// Work items of a tile of cnt nodes and the nodes of one.  Items of 512 are the
-// vector kernels' (one node per thread, so no longer ones); shorter ones belong to
-// the FP64 matrix-core gather and hold about `item` nodes in whole groups of 16 (a
-// tile of up to 1.25 `item` is one; the last items may be short or empty).
-__host__ __device__ inline int tile_items(int cnt, int item) {
+// Ranges of a tile of cnt nodes for the matrix-core gather with tables (gather_mm.hip) and
+// the nodes of one: 512 each, or about `item` < 512 in whole groups of 16 (a tile of up to 1.25
+// `item` is one; the last ranges may be short or empty).
+__host__ __device__ inline int tile_ranges(int cnt, int item) {
   if (item >= 512) return (cnt + item - 1) / item;
   return cnt <= 0 ? 0 : (cnt + item * 3 / 4 < 2 * item ? 1 : (cnt + item * 3 / 4) / item);
 }
-__host__ __device__ inline int item_len(int cnt, int item) {
+__host__ __device__ inline int range_len(int cnt, int item) {
   if (item >= 512) return item;
-  const int k = tile_items(cnt, item);
+  const int k = tile_ranges(cnt, item);
   return k <= 1 ? cnt : ((cnt + k - 1) / k + 15) / 16 * 16;
 }
 

@@ -9,7 +9,7 @@
 // stencil kernels of kernel/assign.c:478-1066 (cutoff 2m+1, :910).
 //
 // Two paths:
-//  * tiled: one block per work item (tile, chunk of about item_nodes sorted
+//  * tiled: one block per work item (tile, chunk of <= kTileThreads sorted
 //    nodes).  The tile's padded subgrid ((TS + 2m) cells per axis, starting at
 //    the tile origin because tiles are keyed by the stencil start) is staged in
 //    LDS; the gather reads every stencil point from LDS, the scatter
@@ -92,13 +92,9 @@ __device__ inline TileItem tile_item(const BArgs<R>& A, int m) {
   it.o[2] = t2 * A.ts[2];
   for (int d = 0; d < 3; d++) it.P[d] = A.ts[d] + 2 * m;
   const int s = A.tile_start[t], e = A.tile_start[t + 1];
-  const int len = item_len(e - s, A.item_nodes);
-  it.beg = min(e, s + chunk * len);
-  // An item has a thread per node.  The second bound tells the compiler so: without it the
-  // node loops of the scatter are compiled for several rounds, the next round's loads ahead
-  // (FP64 gradients: 246 VGPRs at m = 2, one block per CU, for 126 and two; spills from m =
-  // 3 on; M = 3 10^6 on n = 64^3 1294 us per adjoint for 948).
-  it.end = min(min(e, it.beg + len), it.beg + kTileThreads);
+  it.beg = s + chunk * kTileThreads;
+  // a thread per node: the bound lets the compiler see that the node loop of the scatter runs once
+  it.end = min(e, it.beg + kTileThreads);
   return it;
 }
 

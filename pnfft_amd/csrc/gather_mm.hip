@@ -632,7 +632,7 @@ void launch(const BArgs<R>& A, hipStream_t s) {
     using S = GatherShape<R, MT, MODE, RG>;
     (void)hipFuncSetAttribute((const void*)gather_mm_k<R, MT, MODE, RG>, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)S::LDS);
-    hipLaunchKernelGGL((gather_mm_k<R, MT, MODE, RG>), dim3((unsigned)A.n_items), dim3(S::NT), S::LDS, s, A);
+    hipLaunchKernelGGL((gather_mm_k<R, MT, MODE, RG>), dim3((unsigned)A.n_ranges), dim3(S::NT), S::LDS, s, A);
   };
   if (A.c2r)
     go(std::true_type{});
@@ -648,7 +648,7 @@ void launch(const BArgs<R>& A, hipStream_t s) {
 template <class R, int MODE>
 int gather_mm(const BArgs<R>& A, hipStream_t s) {
   const int ts = std_tile(A.g.m, sizeof(R) == 8);
-  if (A.no_mfma || !A.pre_psi || !A.pre_x || (MODE != B_F && !A.pre_dpsi) || !A.ranges || A.n_items <= 0 ||
+  if (A.no_mfma || !A.pre_psi || !A.pre_x || (MODE != B_F && !A.pre_dpsi) || !A.ranges || A.n_ranges <= 0 ||
       !A.all_dense || !A.perm || !A.stale_count || !A.stale_list || A.ts[0] != ts || A.ts[1] != ts || A.ts[2] != ts)
     return kUnsupported;
   if constexpr (sizeof(R) == 8) {

@@ -323,10 +323,13 @@ __device__ inline unsigned tile_parts(int cnt, TileCut c) {
   return cnt > c.whole ? (unsigned)((cnt + c.part - 1) / c.part) : (cnt > 0 ? 1u : 0u);
 }
 
+// Work items of a tile.
+__device__ inline unsigned tile_chunks(int cnt) { return (unsigned)((cnt + kTileThreads - 1) / kTileThreads); }
+
 // Per tile: order entries by node-count class (leading zeros of the count: more
 // nodes, smaller class) added to work[class], and the values whose scans place
-// the tile: flag of 2..31 nodes, flag of one node, work items of the gather (and
-// of the scatter, where they differ).
+// the tile: flag of 2..31 nodes, flag of one node, work items of the gather, ranges
+// and work items of the scatter, where they differ.
 __global__ __launch_bounds__(kB) void tile_class_k(const int* __restrict__ tile_start, long ntiles, int dense_min,
                                                    TileCut cut, bool two_lists, int rounds, unsigned* work,
                                                    unsigned* scan, unsigned char* dense, unsigned char* dense_s) {
@@ -338,13 +341,14 @@ __global__ __launch_bounds__(kB) void tile_class_k(const int* __restrict__ tile_
     const int cnt = t < ntiles ? tile_start[t + 1] - tile_start[t] : 0;
     if (t < ntiles) {
       const bool d = cnt >= dense_min && cnt > 0;
-      const unsigned ch = (unsigned)tile_items(cnt, cut.item);
+      const unsigned ch = tile_chunks(cnt);
       dense[t] = d ? 1 : 0;
       dense_s[t] = cnt > 0 ? 1 : 0;
       scan[t] = (cnt > 1 && cnt < 32) ? 1u : 0u;
       scan[ntiles + t] = cnt == 1 ? 1u : 0u;
       scan[2 * ntiles + t] = d ? ch : 0u;
-      if (two_lists) scan[3 * ntiles + t] = ch;
+      scan[3 * ntiles + t] = (unsigned)tile_ranges(cnt, cut.item);
+      if (two_lists) scan[4 * ntiles + t] = ch;
     }
     const unsigned parts = tile_parts(cnt, cut);
     (void)wave_class_add(cnt > 0, cnt > 0 ? __clz(cnt) : 0, lc);
@@ -363,7 +367,7 @@ __global__ __launch_bounds__(kB) void tile_class_k(const int* __restrict__ tile_
 // tiles, whose padded subgrids overlap, are taken by neighbouring blocks, and the
 // tiles of one node come last, in tile order as well.  tile_slot[t] = (first
 // entry of tile t, -1: none; entries).  ranges, oranges (or null): the position
-// ranges of the gather's work items and of the order entries; the nodes of a
+// ranges of the matrix-core gather and of the order entries; the nodes of a
 // range from mid on start in the upper half of axis 2, by bisection of the keys,
 // whose in-tile index counts the runs of four cells along axis 2 outermost.
 __global__ __launch_bounds__(kB) void tile_place_k(const int* __restrict__ tile_start, long ntiles, int dense_min,
@@ -423,28 +427,33 @@ __global__ __launch_bounds__(kB) void tile_place_k(const int* __restrict__ tile_
           oranges[p + k] = make_int4((int)t, b, min(max(mid, b), e), e);
         }
       }
-      const unsigned o = scan[2 * ntiles + t], ch = (unsigned)tile_items(cnt, cut.item);
+      const unsigned o = scan[2 * ntiles + t], ch = tile_chunks(cnt);
       for (unsigned k = 0; k < ch; k++) {
         if (cnt >= dense_min) {
           items[2 * (o + k)] = (int)t;
           items[2 * (o + k) + 1] = (int)k;
-          if (ranges) {
-            const int len = item_len(cnt, cut.item), b = min(end, beg + (int)k * len), e = min(end, b + len);
-            ranges[o + k] = make_int4((int)t, b, min(max(mid, b), e), e);
-          }
         }
         if (two_lists) {
-          const unsigned os = scan[3 * ntiles + t];
+          const unsigned os = scan[4 * ntiles + t];
           items_s[2 * (os + k)] = (int)t;
           items_s[2 * (os + k) + 1] = (int)k;
+        }
+      }
+      if (ranges) {
+        const unsigned r = scan[3 * ntiles + t];
+        const int nr = tile_ranges(cnt, cut.item), len = range_len(cnt, cut.item);
+        for (int k = 0; k < nr; k++) {
+          const int b = min(end, beg + k * len), e = min(end, b + len);
+          ranges[r + k] = make_int4((int)t, b, min(max(mid, b), e), e);
         }
       }
     }
     tile_slot[t] = cnt > 0 ? make_int2((int)p, (int)parts) : make_int2(-1, 0);
     if (t == ntiles - 1) {
-      const unsigned ch = (unsigned)tile_items(cnt, cut.item);
+      const unsigned ch = tile_chunks(cnt);
       work[64] = scan[2 * ntiles + t] + (cnt >= dense_min ? ch : 0u);
-      work[65] = two_lists ? scan[3 * ntiles + t] + ch : work[64];
+      work[65] = two_lists ? scan[4 * ntiles + t] + ch : work[64];
+      work[67] = scan[3 * ntiles + t] + (unsigned)tile_ranges(cnt, cut.item);
     }
   }
 }
@@ -638,7 +647,7 @@ int build_tile_lists(const unsigned* keys, long M, const TileLayout& T, int dens
   const int rounds = class_rounds(nt);
   hipLaunchKernelGGL(tile_class_k, dim3(grid1d(nt, rounds * kB)), dim3(kB), 0, s, L.tile_start, nt, dense_min,
                      cut, two, rounds, L.work, L.scan, L.dense, L.dense_s);
-  scan_exclusive(L.scan, nt, two ? 4 : 3, L.partial, s);
+  scan_exclusive(L.scan, nt, two ? 5 : 4, L.partial, s);
   hipLaunchKernelGGL(tile_place_k, dim3(grid1d(nt, rounds * kB)), dim3(kB), 0, s, L.tile_start, nt, dense_min,
                      cut, two, rounds, keys, (unsigned)T.tile_vol(), L.work, L.scan, L.items, L.items_s, L.order,
                      L.tile_slot, L.ranges, L.oranges);
@@ -660,6 +669,7 @@ int build_tile_lists(const unsigned* keys, long M, const TileLayout& T, int dens
   out->n_items = (int)w[64];
   out->n_items_s = (int)w[65];
   out->n_cut = (int)w[66];
+  out->n_ranges = (int)w[67];
   return kOk;
 }
 

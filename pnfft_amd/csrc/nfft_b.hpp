@@ -31,9 +31,9 @@ struct BArgs {
   const unsigned char* tile_dense;  // [ntiles] 1 if the tile's nodes go through the LDS path
   const int* items;        // work items: pairs (tile id, chunk index)
   int n_items;
-  int item_nodes;          // about this many nodes per work item (item_len)
-  // position ranges (tile, beg, mid, end) of the work items and of the order entries (TileLists)
+  // position ranges (tile, beg, mid, end) of the matrix-core gather and of the order entries (TileLists)
   const int4* ranges;
+  int n_ranges;
   const int4* oranges;
   int ts[3];               // tile size per axis
   int ntile[3];            // tiles per axis
@@ -69,7 +69,7 @@ struct BArgs {
 // accumulators within the LDS).
 constexpr int std_tile(int m, bool is_double) { return (m <= 4 || (m <= 6 && is_double)) ? 8 : 4; }
 
-constexpr int kTileThreads = 512;  // threads per block of the tiled kernels
+constexpr int kTileThreads = 512;  // threads per block of the tiled kernels, nodes per work item
 
 // Column scatter: applies for m = 2..8 (FP64: m <= 6) when all three tile
 // sizes equal the layout's TS (std_tile); P = TS + 2m cells per
@@ -85,7 +85,7 @@ int cols_launch(const BArgs<R>& A, hipStream_t s);
 
 // Gather on the matrix cores with windows from tables (gather_mm.hip) for MODE
 // (B_F, B_GRAD, B_FGRAD, B_VJP): FP64 at m = 3..6, FP32 at m = 7, 8, on the standard
-// tiles with the work items' ranges; kUnsupported (nothing launched) otherwise.
+// tiles with their ranges; kUnsupported (nothing launched) otherwise.
 template <class R, int MODE>
 int gather_mm(const BArgs<R>& A, hipStream_t s);
 
@@ -113,14 +113,14 @@ struct TileLayout {
 // unless said otherwise):
 //  * tile_start [ntiles + 1]: first sorted position of every tile;
 //  * dense, items: tiles of at least dense_min nodes, cut into work items (tile,
-//    chunk) of about cut.item nodes (item_len) in tile order; dense_s, items_s: every nonempty
+//    chunk) of kTileThreads nodes in tile order; dense_s, items_s: every nonempty
 //    tile (the same list, and items_s unused, for dense_min = 1);
 //  * order: nonempty tiles, those of 32 nodes or more by decreasing node count
 //    (power-of-two classes), then those of 2..31 nodes and those of one node, both
 //    in tile order; a tile of more than cut.whole nodes has an entry per
 //    cut.part nodes; tile_slot = (first entry, -1: empty tile; entries);
-//  * ranges, oranges (or null): position ranges (tile, beg, mid, end) of the items
-//    and of the order entries; the nodes [beg, mid) start in the lower half of the
+//  * ranges (or null), oranges: position ranges (tile, beg, mid, end) of about cut.item
+//    nodes in tile order (range_len), and of the order entries; the nodes [beg, mid) start in the lower half of the
 //    tile's cells along axis 2, [mid, end) in the upper half (tiles of 8^3 cells;
 //    else mid = end);
 //  * box_tile, box_ord: offset masks of the tile's nodes per axis, by tile and by
@@ -128,11 +128,11 @@ struct TileLayout {
 //    the brick fold) hold only the box these masks span (from the smallest offset to
 //    the largest plus 2m per axis); a node whose stencil leaves that box (moved
 //    since binning) takes the stale path.
-constexpr int kTileWork = 67;  // counters: entries per class (32), placed (32), items, items_s, cut tiles
+constexpr int kTileWork = 68;  // counters: entries per class (32), placed (32), items, items_s, cut tiles, ranges
 struct TileLists {
   int* tile_start;
-  unsigned* scan;     // [4 ntiles]
-  unsigned* partial;  // [4 (ntiles / 4096 + 1)]
+  unsigned* scan;     // [5 ntiles]
+  unsigned* partial;  // [5 (ntiles / 4096 + 1)]
   unsigned* work;     // [kTileWork]
   unsigned char *dense, *dense_s;
   int *items, *items_s;
@@ -144,10 +144,10 @@ struct TileLists {
 };
 struct TileCut {
   int part, whole;  // order entries of a tile of more than `whole` nodes hold `part` nodes each
-  int item;         // about this many nodes per work item
+  int item;         // about this many nodes per range
 };
 struct TileCounts {
-  int n_items, n_items_s, n_order;
+  int n_items, n_items_s, n_ranges, n_order;
   int n_heavy;   // order entries of tiles of 32 nodes or more
   int n_single;  // the last n_single entries: tiles of one node
   int n_cut;     // tiles with several order entries
