@@ -769,11 +769,14 @@ static void set_tiles(BArgs<R>& A, const NodesT<R>* D, bool for_scatter = false)
   A.tile_dense = two ? D->tl.dense_s : D->tl.dense;
   A.items = two ? D->tl.items_s : D->tl.items;
   A.n_items = two ? D->tc.n_items_s : D->tc.n_items;
-  // The matrix-core gather needs the ranges.  In FP64 at m = 2 the stencil fills
-  // too little of its 16-row products everywhere (M = 2^20, 2048 nodes per tile: 94
-  // us on the vector kernel, 119 on the matrix cores), at m = 3 where the vector
-  // kernel's threads are busy (170 and 190 us; 92 nodes per tile 467 and 319 us).
-  const bool light = D->tc.n_items > 0 && D->M / D->tc.n_items < 200 && D->M >= 65536;
+  // The matrix-core gather needs the ranges.  In FP64 at m = 2 the stencil fills too little of
+  // its 16-row products everywhere (M = 2^20, 2048 nodes per tile: 94 us on the vector
+  // kernel, 119 on the matrix cores), at m = 3 where the vector kernel's threads are busy (170
+  // and 190 us; 92 nodes per tile 467 and 319 us): from 200 nodes per item on, and from 16 on where
+  // there are few nodes at all (5 10^4 nodes, n = 64^3, eight clusters 88 and 105 us; 12 per tile
+  // on n = 128^3 251 and 149 us).
+  const long per = D->tc.n_items > 0 ? D->M / D->tc.n_items : 0;
+  const bool light = D->tc.n_items > 0 && per < (D->M >= 65536 ? 200 : 16);
   A.n_ranges = D->tc.n_ranges;
   A.ranges = D->has_ranges && (for_scatter || D->bin_geom.m > 3 || (D->bin_geom.m == 3 && light)) ? D->tl.ranges
                                                                                                  : nullptr;

@@ -645,11 +645,31 @@ void launch(const BArgs<R>& A, hipStream_t s) {
 
 }  // namespace
 
+// FP64 gradient modes on complex grids whose node set the vector kernel takes faster, with
+// windows from the same tables.
+// m = 3: few tiles that are heavy, or so uneven that some are cut (n = 128^3, 3 10^5 nodes in
+// eight clusters 183 and 219 us here; 122 uniform nodes per tile 328 and 286).
+// m = 5, where registers and the 104 KB subgrid leave two waves per SIMD and nothing to overlap
+// the staging: tiles that are one vector block of 512 nodes but a long range or two short ones
+// here (n = 64^3, 293 per tile 184 and 216 us, n = 128^3, 488 per tile 1345 and 1462; 244 per tile
+// 1016 and 806, n = 64^3, 586 per tile 331 and 297), and sets of full ranges whose waves of 256
+// blocks (40 us each) cost more than those of the vector kernel (73 us; 10^5 nodes on n = 32^3
+// 128 and 151 us, 5 10^4 120 and 112).
+template <class R, int MODE>
+bool vector_gradient(const BArgs<R>& A) {
+  if (sizeof(R) != 8 || MODE == B_F || A.c2r || !A.items || A.n_items <= 0) return false;
+  if (A.g.m == 3) return A.n_torder <= 4096 && (A.n_cut > 0 || A.M >= 150L * A.n_items);
+  if (A.g.m != 5) return false;
+  const bool one = A.n_cut == 0 && A.M > 256L * A.n_torder && A.M <= 512L * A.n_torder;
+  return one || (A.M >= 65536 && 73L * ((A.n_items + 255) / 256) < 40L * ((A.n_ranges + 255) / 256));
+}
+
 template <class R, int MODE>
 int gather_mm(const BArgs<R>& A, hipStream_t s) {
   const int ts = std_tile(A.g.m, sizeof(R) == 8);
   if (A.no_mfma || !A.pre_psi || !A.pre_x || (MODE != B_F && !A.pre_dpsi) || !A.ranges || A.n_ranges <= 0 ||
-      !A.all_dense || !A.perm || !A.stale_count || !A.stale_list || A.ts[0] != ts || A.ts[1] != ts || A.ts[2] != ts)
+      !A.all_dense || !A.perm || !A.stale_count || !A.stale_list || A.ts[0] != ts || A.ts[1] != ts || A.ts[2] != ts ||
+      vector_gradient<R, MODE>(A))
     return kUnsupported;
   if constexpr (sizeof(R) == 8) {
     switch (A.g.m) {

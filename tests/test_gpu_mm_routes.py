@@ -97,16 +97,18 @@ def values(k, c2r, rng):
 
 
 @pytest.mark.parametrize("c2r", [False, True])
-def test_fp64_gather_m3_light_tiles(gpu, oracle, c2r):
+@pytest.mark.parametrize("heavy", [False, True])
+def test_fp64_gather_m3_light_tiles(gpu, oracle, c2r, heavy):
     """FP64 at m = 3 takes the matrix cores where tiles are light: 70000 nodes over the 4096 tiles of n = 128^3,
-    one tile of more than the 512 nodes of a work item, tiles of up to three nodes (a corner left nearly empty)."""
+    tiles of up to three nodes among them (a corner left nearly empty), with and without one of more than the 512
+    nodes of a work item."""
     import torch
-    print("case mm64 m3", c2r, flush=True)
+    print("case mm64 m3", c2r, heavy, flush=True)
     rng = SplitMix64(8100 + c2r)
     N, n, m = (64, 64, 64), (128, 128, 128), 3
     x = rng.uniform(3 * 80000).reshape(80000, 3) - 0.5
     inside = np.all((x > -0.4) & (x < -0.1), axis=1)
-    x = np.concatenate([x[~inside], x[inside][:40], cluster(n, m, 8, 700, rng)])
+    x = np.concatenate([x[~inside], x[inside][:40], cluster(n, m, 8, 700 if heavy else 250, rng)])
     x = torus(x, "double")
     M = len(x)
     fh = coefficients(N, c2r, rng)
@@ -114,10 +116,10 @@ def test_fp64_gather_m3_light_tiles(gpu, oracle, c2r):
     dp = DevicePlan(N, n, m, 0, M, c2r=c2r)
     dp.set_x(x)
     counts = tile_counts(dp)
-    assert M >= 65536 and M / np.sum((counts + 511) // 512) < 200 and counts.max() > 512
+    assert M >= 65536 and M / np.sum((counts + 511) // 512) < 150 and (counts.max() > 512) == heavy
     assert all(np.any(counts == k) for k in (1, 2, 3))
     # the nodes to compare: light and heavy regions
-    some = np.concatenate([np.arange(0, 2000, 5), np.arange(M - 740, M)])
+    some = np.concatenate([np.arange(0, 2000, 5), np.arange(M - (740 if heavy else 290), M)])
     f_o, g_o = (lambda P: (P.trafo_c2r if c2r else P.trafo)(x[some], fh, compute_grad=True))(
         oracle.Plan(N, n, m, 0, c2r=c2r))
     vjp = (np.conj(w[some])[:, None] * np.asarray(g_o).reshape(-1, 3)).real
@@ -215,6 +217,39 @@ def test_moved_nodes(gpu, oracle, precision, m, wname, c2r):
     torch.cuda.synchronize()
     check_all(oracle, dp, P, x2, coefficients(N, c2r, rng), values(M, c2r, rng), values(3 * M, c2r, rng),
               TOL[precision])
+    dp.close()
+
+
+@pytest.mark.parametrize("m,n,per", [(3, 64, 3), (3, 64, 18), (3, 128, 16), (3, 64, 160), (5, 64, 160), (5, 64, 300), (5, 64, 600),
+                                     (5, 32, 1562)])
+def test_fp64_gather_route_by_density(gpu, oracle, m, n, per):
+    """The FP64 gather at m = 3 and its gradients at m = 5 run on the matrix cores or on the vector kernel by nodes per
+    tile: uniform sets of `per` on both sides of the bounds."""
+    import torch
+    print("case density", m, n, per, flush=True)
+    rng = SplitMix64(8700 + m + per)
+    N, nn = (n // 2,) * 3, (n,) * 3
+    M = per * (n // 8) ** 3
+    x = torus(rng.uniform(3 * M).reshape(M, 3) - 0.5, "double")
+    fh, w = coefficients(N, False, rng), values(M, False, rng)
+    some = np.arange(0, M, max(1, M // 1000))
+    f_o, g_o = oracle.Plan(N, nn, m, 0).trafo(x[some], fh, compute_grad=True)
+    vjp = (np.conj(w[some])[:, None] * np.asarray(g_o).reshape(-1, 3)).real
+    dp = DevicePlan(N, nn, m, 0, M)
+    dp.set_x(x)
+    dp.set_f_hat(fh)
+    for tables in (False, True):
+        if tables:
+            dp.precompute(TABLES)
+        for flags in (F, G, F | G):
+            dp.trafo(flags)
+            assert dp.api.last_error() is None
+            if flags & F:
+                assert rel(dp.f.cpu().numpy()[some], f_o) < 1e-12
+            if flags & G:
+                assert rel(dp.grad.cpu().numpy()[some], g_o) < 1e-12
+        gx = dp.grad_x_vjp(torch.as_tensor(w, device="cuda:0")).cpu().numpy()
+        assert rel(gx[some], vjp) < 1e-12
     dp.close()
 
 
