@@ -295,8 +295,10 @@ struct NodesT {
   size_t pre_psi_cap = 0, pre_dpsi_cap = 0, pre_x_cap = 0;
   bool pre_valid = false, pre_grad = false;
   GridGeom pre_geom{};
-  R* d_call_tab = nullptr;  // tables that a call filled for itself (call_table_memory)
-  size_t call_tab_cap = 0;
+  // tables that a call filled for itself (call_table_memory)
+  R* d_call_tab = nullptr;
+  R* d_call_dtab = nullptr;
+  size_t call_tab_cap = 0, call_dtab_cap = 0;
   SortWork sw;
   bool bins_valid = false;
   GridGeom bin_geom{};
@@ -609,7 +611,8 @@ static void nodes_release_device(NodesT<R>* D) {
   D->pre_psi_cap = D->pre_dpsi_cap = D->pre_x_cap = 0;
   D->pre_valid = false;
   dfree(D->d_call_tab);
-  D->call_tab_cap = 0;
+  dfree(D->d_call_dtab);
+  D->call_tab_cap = D->call_dtab_cap = 0;
   D->bins_valid = false;
 }
 
@@ -913,17 +916,17 @@ static T* grow(T*& p, size_t& cap, size_t need) {
   return p;
 }
 
-// Room for the tables that a call fills for itself: psi, psi' if `grad`, coordinates,
-// in one allocation of their own, so that those of precompute_psi stay.
+// Room for the tables that a call fills for itself (psi and the coordinates; psi' if
+// `grad`), apart from those of precompute_psi, which stay.  psi' is an allocation of its
+// own: a node set whose first call needs none (adj of a particle step) would else free and
+// allocate again in the second (first step of 2^20 particles, FP64, 2.5 ms, 7.6 ms that way).
 template <class R>
 static bool call_table_memory(NodesT<R>* D, int m, bool grad, R*& psi, R*& dpsi, R*& x) {
   const size_t M = (size_t)D->M, rows = 3 * (2 * (size_t)m + 1);
-  R* p = grow(D->d_call_tab, D->call_tab_cap, ((grad ? 2 : 1) * rows + 3) * M);
-  if (!p) return false;
-  psi = p;
-  dpsi = grad ? p + rows * M : nullptr;
-  x = p + (grad ? 2 : 1) * rows * M;
-  return true;
+  psi = grow(D->d_call_tab, D->call_tab_cap, (rows + 3) * M);
+  dpsi = grad && psi ? grow(D->d_call_dtab, D->call_dtab_cap, rows * M) : nullptr;
+  x = psi ? psi + rows * M : nullptr;
+  return psi && (dpsi || !grad);
 }
 
 // Window tables for the matrix-core kernels that take every window from tables
