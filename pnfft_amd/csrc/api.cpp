@@ -296,9 +296,10 @@ struct NodesT {
   bool pre_valid = false, pre_grad = false;
   GridGeom pre_geom{};
   // tables that a call filled for itself (call_table_memory)
-  R* d_call_tab = nullptr;
-  R* d_call_dtab = nullptr;
-  size_t call_tab_cap = 0, call_dtab_cap = 0;
+  R* d_call_psi = nullptr;
+  R* d_call_dpsi = nullptr;
+  R* d_call_x = nullptr;
+  size_t call_psi_cap = 0, call_dpsi_cap = 0, call_x_cap = 0;
   SortWork sw;
   bool bins_valid = false;
   GridGeom bin_geom{};
@@ -610,9 +611,10 @@ static void nodes_release_device(NodesT<R>* D) {
   dfree(D->d_pre_x);
   D->pre_psi_cap = D->pre_dpsi_cap = D->pre_x_cap = 0;
   D->pre_valid = false;
-  dfree(D->d_call_tab);
-  dfree(D->d_call_dtab);
-  D->call_tab_cap = D->call_dtab_cap = 0;
+  dfree(D->d_call_psi);
+  dfree(D->d_call_dpsi);
+  dfree(D->d_call_x);
+  D->call_psi_cap = D->call_dpsi_cap = D->call_x_cap = 0;
   D->bins_valid = false;
 }
 
@@ -917,16 +919,17 @@ static T* grow(T*& p, size_t& cap, size_t need) {
 }
 
 // Room for the tables that a call fills for itself (psi and the coordinates; psi' if
-// `grad`), apart from those of precompute_psi, which stay.  psi' is an allocation of its
-// own: a node set whose first call needs none (adj of a particle step) would else free and
-// allocate again in the second (first step of 2^20 particles, FP64, 2.5 ms, 7.6 ms that way).
+// `grad`), apart from those of precompute_psi, which stay.  Each is an allocation of its
+// own: a node set whose first call needs no psi' (adj of a particle step) would else free
+// and allocate again in the second (first step of 2^20 particles, FP64, 2.3 ms, 7.6 ms with
+// one allocation).
 template <class R>
 static bool call_table_memory(NodesT<R>* D, int m, bool grad, R*& psi, R*& dpsi, R*& x) {
   const size_t M = (size_t)D->M, rows = 3 * (2 * (size_t)m + 1);
-  psi = grow(D->d_call_tab, D->call_tab_cap, (rows + 3) * M);
-  dpsi = grad && psi ? grow(D->d_call_dtab, D->call_dtab_cap, rows * M) : nullptr;
-  x = psi ? psi + rows * M : nullptr;
-  return psi && (dpsi || !grad);
+  psi = grow(D->d_call_psi, D->call_psi_cap, rows * M);
+  dpsi = grad && psi ? grow(D->d_call_dpsi, D->call_dpsi_cap, rows * M) : nullptr;
+  x = psi && (dpsi || !grad) ? grow(D->d_call_x, D->call_x_cap, 3 * M) : nullptr;
+  return x != nullptr;
 }
 
 // Window tables for the matrix-core kernels that take every window from tables
