@@ -410,6 +410,22 @@ __device__ inline void scatter_node_global(const BArgs<R>& A, long j, NodeWin<R,
   }
 }
 
+// OR of v over each row of 16 lanes (DPP row shifts); lane 15 of a row holds it
+__device__ __forceinline__ unsigned row_or16(unsigned v) {
+  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  return v;
+}
+
+// clears the count of nodes listed for a stale kernel
+namespace {
+__global__ void zero_u32_k(unsigned* c) {
+  if (threadIdx.x == 0) *c = 0u;
+}
+}  // namespace
+
 __device__ inline int wrapi(int v, int n) { return v >= n ? v - n : v; }
 
 // local offset of the node's stencil start inside the tile, or -1 if outside

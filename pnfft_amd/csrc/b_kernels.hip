@@ -359,15 +359,6 @@ __device__ __forceinline__ float comp4(const float4& v, int e) {
   return e == 0 ? v.x : (e == 1 ? v.y : (e == 2 ? v.z : v.w));
 }
 
-// OR of v over each row of 16 lanes (DPP row shifts); lane 15 of a row holds it
-__device__ __forceinline__ unsigned row_or16(unsigned v) {
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
-  return v;
-}
-
 // LDS writes of one lane become visible to the other lanes of its wave
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -392,8 +383,8 @@ struct GatherMfmaShape {
   // registers allow two from m = 5 on).  With rows for y and z apart (46 KB, three
   // blocks for f) f took 481 us and now 433 us at m = 4, N = 128^3, 2^21 uniform nodes;
   // two-wave gradient blocks at m = 6 4.09 ms and now 3.53 ms of 2^25 crowded nodes.
-  // From 2^24 nodes of a Gaussian mixture on (m = 4) f is close to the products'
-  // own cycles (1.73 -> 1.67 ms).
+  // 2^24 nodes of a Gaussian mixture (m = 4): f 1.73 -> 1.67 ms, with the matrix cores
+  // busy for 0.48 of it.
   static constexpr int WAVES = WG ? (NW == 2 || MT >= 5 ? 2 : 3) : (NW == 2 ? 3 : 4);
   static constexpr int NT = 64 * NW;        // threads per block
   static constexpr size_t LDS = sizeof(float) * (2 * P * 256 + NW * ROWSZ);
@@ -751,10 +742,6 @@ __global__ __launch_bounds__(64 * NW, (GatherMfmaShape<MT, MODE, NW>::WAVES)) vo
     jn_ok = jnn_ok;
     wave_sync();
   }
-}
-
-__global__ void zero_u32_k(unsigned* c) {
-  if (threadIdx.x == 0) *c = 0u;
 }
 
 // nodes the matrix-core gather listed as outside their tile: gathered straight

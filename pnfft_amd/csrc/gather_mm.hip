@@ -620,10 +620,6 @@ __global__ __launch_bounds__(256) void gather_stale_mm_k(BArgs<R> A) {
   }
 }
 
-__global__ void zero_u32_k(unsigned* c) {
-  if (threadIdx.x == 0) *c = 0u;
-}
-
 template <class R, int MT, int MODE>
 void launch(const BArgs<R>& A, hipStream_t s) {
   hipLaunchKernelGGL(zero_u32_k, dim3(1), dim3(64), 0, s, A.stale_count);

@@ -45,15 +45,6 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// OR of v over each row of 16 lanes (DPP row shifts); lane 15 of a row holds it
-__device__ __forceinline__ unsigned row_or16(unsigned v) {
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
-  return v;
-}
-
 // Windows of one axis evaluated straight into LDS rows (psi and, if WD, psi'),
 // for nodes whose coordinates are no longer those of the tables: the formulas
 // and operation order of window_axis_s with rolled loops, the B-spline recursion

@@ -242,15 +242,6 @@ struct MfmaShape {
 // rows (v even, v + 1).
 __device__ __forceinline__ constexpr int row_at(int v) { return 16 * v + (v >> 1); }
 
-// OR of v over each row of 16 lanes (DPP row shifts); lane 15 of a row holds it
-__device__ __forceinline__ unsigned row_or16(unsigned v) {
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
-  v |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
-  return v;
-}
-
 // OR of v over the 64 lanes of a wave, as a wave-uniform value
 __device__ __forceinline__ unsigned wave_or(unsigned v) {
   v = row_or16(v);
@@ -809,10 +800,6 @@ __global__ __launch_bounds__(256) void scatter_stale_k(BArgs<R> A) {
   }
 }
 
-__global__ void zero_count_k(unsigned* c) {
-  if (threadIdx.x == 0) *c = 0u;
-}
-
 inline unsigned grid1d(long n, int t) { return (unsigned)((n + t - 1) / t); }
 
 // the fold kernel of the layout (tiles of TS cells, padded subgrids of P)
@@ -846,7 +833,7 @@ void launch_m(const BArgs<R>& A0, hipStream_t s) {
   A.box_slots = 0;
   if constexpr (sizeof(R) == 4 && S::TS == 8 && S::P <= 16 && S::P % 4 == 0)
     A.box_slots = (A.box_tile && A.box_ord && !A.no_mfma && A.ts[2] == 8 && A.ntile[2] % 2 == 0) ? 1 : 0;
-  hipLaunchKernelGGL(zero_count_k, dim3(1), dim3(64), 0, s, A.stale_count);
+  hipLaunchKernelGGL(zero_u32_k, dim3(1), dim3(64), 0, s, A.stale_count);
   bool done = false;
   if constexpr (sizeof(R) == 4 && S::P <= 16) {
     if (!A.no_mfma) {

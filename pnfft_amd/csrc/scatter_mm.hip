@@ -35,7 +35,12 @@
 // so two blocks share a CU and the rows of one overlap the products of the other
 // (256 VGPRs and one block: the same time).  The gradient modes replace kernels
 // that added every stencil cell by FP64 LDS atomics: charges and dipoles at m =
-// 4, M = 2^19 2.86 -> 0.27 ms per launch.
+// 4, M = 2^19 2.86 -> 0.27 ms per launch.  At m = 2 (25 of the 144 cells of a plane) f is still
+// faster than on the column kernel (adjoint, n = 128^3, 6 10^5 uniform nodes 653 -> 252 us)
+// and f with gradients than with atomics (552 -> 330).  Gradients alone are 0.5 to 1.0 of the
+// atomics' time on most sets (n = 256^3, 10^6 nodes 1682 -> 1103 us) and up to 1.5 where a few
+// dense tiles keep the atomics in LDS (n = 32^3, 3 10^5 nodes 188 -> 282); they stay here, where
+// the sums repeat bit for bit.
 #include "mm.hpp"
 
 namespace pnfft_amd {
@@ -112,7 +117,7 @@ __global__ __launch_bounds__((ScatterShape<R, MT, MODE>::NT),
   constexpr int H0 = (CM + 1) / 2;  // window entries 0 .. H0 - 1 and H0 .. CM - 1 are two threads' share
   __shared__ R s_row[3 * (WG ? 2 : 1)][NB * PITCH];  // X, Y, Z (and X', Y', Z') rows
   __shared__ V2 s_w[WG ? 4 : 1][NB];                 // f, g0, g1, g2
-  __shared__ unsigned s_km[NB / 4];                       // per four nodes: planes reached, bit 31: rows past 15
+  __shared__ unsigned s_km[NB / 4];                       // per four nodes: planes reached
   __shared__ unsigned char s_bad[3][NB];
 
   const int4 range = A.oranges[blockIdx.x];
@@ -429,10 +434,6 @@ __global__ __launch_bounds__(256) void scatter_stale_mm_k(BArgs<R> A) {
     node_windows<R, MT, S::CM, S::WG>(A, -1, j, MT, w);
     scatter_node_global<R, S::CM, MODE, true>(A, j, w, S::CM);
   }
-}
-
-__global__ void zero_u32_k(unsigned* c) {
-  if (threadIdx.x == 0) *c = 0u;
 }
 
 // FP64 f on complex grids at m = 5, 6: most tiles hold at most one batch of nodes, so a
