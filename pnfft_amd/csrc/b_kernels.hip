@@ -856,19 +856,28 @@ __global__ __launch_bounds__(256) void gather_single_k(BArgs<float> A, int first
 
 inline unsigned grid1d(long n, int t) { return (unsigned)((n + t - 1) / t); }
 
-// The x-VJP at m = 2, 3 on the vector kernel (gather_tiled_k), whose threads read the
+// The x-VJP at m = 2, 3, 4 on the vector kernel (gather_tiled_k), whose threads read the
 // (2m+1)^3 cells of their own node: less than a group's 16 x 16 x 4 products cost, once a
 // tile's nodes repay its staging and there are few tiles or uneven ones, whose parts leave
 // the last wave of matrix-core blocks unfilled.  Windows from tables, vector and matrix-core
 // kernel: n = 64^3, 10^6 uniform nodes m = 2 127 and 193 us, m = 3 202 and 232; eight clusters,
-// 10^5 nodes, n = 32^3 m = 2 41 and 100 us, n = 64^3 m = 3 63 and 120.  Light tiles (n = 256^3, 5 10^4
-// nodes: m = 2 285 and 249, m = 3 397 and 289), many even tiles of many nodes (n = 128^3, 3 10^6:
-// m = 3 716 and 612) and real grids at m = 3, which halve the products (n = 64^3, 10^6: 191 and
-// 168), stay on the matrix cores.
+// 10^5 nodes, n = 32^3 m = 2 41 and 100 us, n = 64^3 m = 3 63 and 120.  On the matrix cores stay
+// light tiles (n = 256^3, 5 10^4 nodes: m = 2 285 and 249, m = 3 397 and 289), where there are
+// many even tiles of many nodes at m = 3 (n = 128^3, 3 10^6: 716 and 612; in the 512 tiles of
+// n = 64^3 518 and 606), and real grids, which halve the products, at m = 2 with many nodes
+// (n = 128^3, 3 10^6: 421 and 355).  On real grids at m = 3 and complex ones at m = 4 the vector
+// kernel has uneven sets only: some tiles cut, at most 3 / 4 of the grid's (m = 3, n = 64^3, 10^6:
+// uniform 191 and 168, eight clusters 180 and 219; n = 32^3, 2 10^6 uniform, all of the 64 tiles
+// cut, 346 and 279; m = 4, n = 64^3, 2 10^5: uniform 103 and 92, eight clusters 94 and 129;
+// n = 256^3, 3 10^6 in eight clusters 1100 and 789).
 template <int MT, int MODE>
 bool vector_vjp(const BArgs<float>& A) {
-  if (MODE != B_VJP || MT > 3 || (MT == 3 && A.c2r) || !A.items || A.n_items <= 0) return false;
-  return A.M >= 3L * (MT - 1) * A.n_torder && (A.n_cut > 0 || A.M <= (1L << 21)) && (MT == 2 || A.n_torder <= 4096);
+  if (MODE != B_VJP || MT > 4 || !A.items || A.n_items <= 0) return false;
+  if ((MT == 3 && A.c2r) || (MT == 4 && !A.c2r))
+    return A.n_cut > 0 && 4 * A.n_cut <= 3 * A.ntile[0] * A.ntile[1] * A.ntile[2] && A.n_torder <= 4096;
+  if (MT == 4 || A.M < 3L * (MT - 1) * A.n_torder) return false;
+  const bool few = A.n_cut > 0 || A.M <= (1L << 21);
+  return MT == 2 ? few || !A.c2r : (few || A.n_torder <= 1024) && A.n_torder <= 4096;
 }
 
 // the matrix-core gather applies to FP32 (f, grad, f + grad, VJP) with m <= 6 on the

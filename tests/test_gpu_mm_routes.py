@@ -255,9 +255,9 @@ def test_fp64_gather_route_by_density(gpu, oracle, m, n, per):
 
 @pytest.mark.parametrize("c2r", [False, True])
 @pytest.mark.parametrize("kind", ["light", "dense", "cut"])
-@pytest.mark.parametrize("m", [2, 3])
+@pytest.mark.parametrize("m", [2, 3, 4])
 def test_fp32_vjp_small_m(gpu, oracle, m, kind, c2r):
-    """The x-VJP of FP32 plans at m = 2, 3 runs on the matrix cores or on the vector kernel by nodes per tile: about
+    """The x-VJP of FP32 plans at m = 2, 3, 4 runs on the matrix cores or on the vector kernel by nodes per tile: about
     one, eight and more, and a tile cut into parts."""
     import torch
     print("case vjp", m, kind, c2r, flush=True)
